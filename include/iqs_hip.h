@@ -222,8 +222,8 @@ int iqsh_adjoint_1q(iqsh_handle psi, iqsh_handle lam, unsigned pos, const double
 int iqsh_apply_1q_all(iqsh_handle h, const double m[8]);
 /* Backward step through such a layer for both states: *grad := sum_q 2 Im <lam| G_q |psi>
  * (G on position q, each term as iqsh_adjoint_1q would take it), then psi := Uinv^(x)n psi,
- * lam := Uinv^(x)n lam, in 1 + ceil((n - 8) / 4) passes (G equal to X exactly, and Uinv of
- * the RX form, take shorter kernels).  n >= 10. */
+ * lam := Uinv^(x)n lam, in 1 + ceil((n - 12) / 8) passes (G equal to X exactly with Uinv of
+ * the RX form takes shorter kernels).  n >= 10. */
 int iqsh_adjoint_1q_all(iqsh_handle psi, iqsh_handle lam, const double Uinv[8], const double *G, double *grad);
 
 /* One QAOA layer, psi := mixer^(x)n exp(-i gamma C) psi with C the cut of the edge list (as

@@ -130,3 +130,35 @@ def test_qaoa_layer_fused_equals_unfused(dt, weighted, n):
     assert abs(db1 - db2) < tol * max(1, abs(db2)) and abs(dg1 - dg2) < tol * max(1, abs(dg2))
     assert np.abs(p1.download() - p2.download()).max() < TOL[dt]
     assert np.abs(l1.download() - l2.download()).max() < TOL[dt]
+
+
+@pytest.mark.parametrize("dt", ["c128", "c64"])
+@pytest.mark.parametrize("weighted", [False, True])
+@pytest.mark.parametrize("n", [10, 11, 13, 14, 16, 17, 18, 19, 21, 22, 23, 25])
+def test_layer_tiles(dt, weighted, n):
+    """Every tile size and number of passes, and the cache policies (32 MiB of states from 21
+    qubits on): the fused layer and its adjoint against the phase and the gates one by one,
+    on a graph of up to 64 edges with repeated ones.  Tolerances: 3 n + 2 roundings per
+    amplitude of size <= 1 (2^-53, 2^-24), and for the sums the existing relative ones."""
+    from iqs_amd import gates as Gt
+    r = np.random.default_rng(n)
+    pairs = [tuple(int(v) for v in r.choice(n, 2, replace=False)) for _ in range(min(64, 3 * n))]
+    pairs[-1] = pairs[0]
+    edges = [(u, v, float(r.uniform(0.1, 2.0)) if weighted else 1.0) for u, v in pairs]
+    gamma, beta = 0.37, 0.91
+    psi, lam = _state(n, dt, 51), _state(n, dt, 52)
+    X = np.array([[0, 1], [1, 0]])
+    a, b = _gpu(psi, dt), _gpu(psi, dt)
+    a.qaoa_layer(edges, gamma, Gt.rx(2 * beta))
+    b.qaoa_phase(edges, gamma)
+    for q in range(n):
+        b.apply_1q(q, Gt.rx(2 * beta))
+    assert a.maxabsdiff(b) < TOL[dt]
+    la, lb = _gpu(lam, dt), _gpu(lam, dt)
+    b.copy_from(a)
+    dg, db = a.qaoa_layer_adjoint(la, edges, gamma, Gt.rx(-2 * beta), X)
+    db1 = sum(b.adjoint_1q(lb, q, Gt.rx(-2 * beta), X) for q in range(n))
+    dg1 = b.qaoa_phase_adjoint(lb, edges, gamma)
+    tol = 1e-11 if dt == "c128" else 2e-5
+    assert abs(db - db1) < tol * max(1, abs(db1)) and abs(dg - dg1) < tol * max(1, abs(dg1))
+    assert a.maxabsdiff(b) < TOL[dt] and la.maxabsdiff(lb) < TOL[dt]
