@@ -9,6 +9,7 @@
 #include <cstdio>
 #include <cstring>
 #include <mutex>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/iqs_hip.h"
@@ -201,41 +202,57 @@ template <typename T>
 constexpr unsigned line_bits() { return sizeof(T) == 8 ? 3u : 4u; }
 constexpr int kSB = 256, kSP = 4;   // plain kernels for small states
 
+// Calls f with std::true_type (non-temporal accesses) or std::false_type (ordinary ones), by
+// the register's size (iqsi::cache_set).
+template <typename F>
+void by_cache_policy(iqsh_handle h, F f)
+{
+  if (iqsi::cache_set(h->size() * h->esz())) f(std::false_type{});
+  else f(std::true_type{});
+}
+
 template <typename T, int K, bool MOVE>
 int launch_pair_m(iqsh_handle h, const Ins<K>& ins, uint64_t mask0, uint64_t mask1, const double* m)
 {
   using V = typename Vec<T>::t;
   const uint64_t items = h->size() >> K;
   constexpr int TB = PairTile<T>::B, TP = PairTile<T>::P;
-  const dim3 grid = grid2(items / (TB * TP));
-  if (items >= kTiledMin && K >= 2 && ins.p[0] < line_bits<T>())
+  if (items < kTiledMin) {
+    k_pair<T, K, MOVE, false, kSB, kSP><<<grid2(grid_for(items, kSB * kSP)), kSB, 0, g_stream>>>((V*)h->d, items, ins, mask0,
+                                                                                                 mask1, mat2<T>(m));
+    CHECK_LAUNCH();
+    return IQSH_OK;
+  }
+  if (K >= 2 && ins.p[0] < line_bits<T>()) {
     // Lowest position inside a cache line (a control above it): cached accesses let L2
     // complete the lines that the two halves of each pair share.
-    k_pair<T, K, MOVE, true, TB, TP, kSub, kSubLog, false><<<grid, TB, 0, g_stream>>>((V*)h->d, items, ins, mask0,
-                                                                                           mask1, mat2<T>(m));
-  else if (items >= kTiledMin && sizeof(T) == 8 && ins.p[K - 1] <= 10)
-    // Complex128 with every touched position <= 10: sub-ranges 2^10 items apart (30q sweep,
-    // dense 1q targets 6-10: 6.44 TB/s at 2^11, 6.57 at 2^10).
-    k_pair<T, K, MOVE, true, TB, TP, kSub, 10><<<grid, TB, 0, g_stream>>>((V*)h->d, items, ins, mask0, mask1,
-                                                                            mat2<T>(m));
-  else if (items >= kTiledMin && K >= 2 && sizeof(T) == 8 && ins.p[0] < 6)
-    // Complex128 with the lowest position 3-5 (inside a wavefront, from the line width up):
-    // 128 x 1 (30q: controlled (3,20) 5.42 -> 6.16 TB/s, swap (4,25) 5.82 -> 6.57).
-    k_pair<T, K, MOVE, true, 128, 1><<<grid2(items / 128), 128, 0, g_stream>>>((V*)h->d, items, ins, mask0, mask1,
-                                                                               mat2<T>(m));
-  else if (items >= kTiledMin && K >= 2) {
-    constexpr int GB = MOVE ? PairTile<T>::MB : PairTile<T>::CB, GP = MOVE ? PairTile<T>::MP : PairTile<T>::CP;
-    k_pair<T, K, MOVE, true, GB, GP><<<grid2(items / (GB * GP)), GB, 0, g_stream>>>((V*)h->d, items, ins, mask0, mask1,
-                                                                                    mat2<T>(m));
+    k_pair<T, K, MOVE, true, TB, TP, kSub, kSubLog, false><<<grid2(items / (TB * TP)), TB, 0, g_stream>>>(
+        (V*)h->d, items, ins, mask0, mask1, mat2<T>(m));
+    CHECK_LAUNCH();
+    return IQSH_OK;
   }
-  else if (items >= kTiledMin) {
-    // one inserted bit here (two or more took the branch above)
-    constexpr int GB = PairTile<T>::SB, GP = PairTile<T>::SP;
-    k_pair<T, K, MOVE, true, GB, GP><<<grid2(items / (GB * GP)), GB, 0, g_stream>>>((V*)h->d, items, ins, mask0, mask1,
-                                                                                    mat2<T>(m));
-  } else
-    k_pair<T, K, MOVE, false, kSB, kSP><<<grid2(grid_for(items, kSB * kSP)), kSB, 0, g_stream>>>((V*)h->d, items, ins, mask0,
-                                                                                          mask1, mat2<T>(m));
+  by_cache_policy(h, [&](auto policy) {
+    constexpr bool NT = decltype(policy)::value;
+    auto go = [&](auto kernel, int b, int p) {
+      kernel<<<grid2(items / ((uint64_t)b * p)), b, 0, g_stream>>>((V*)h->d, items, ins, mask0, mask1, mat2<T>(m));
+    };
+    if (sizeof(T) == 8 && ins.p[K - 1] <= 10) {
+      // Complex128 with every touched position <= 10: sub-ranges 2^10 items apart (30q sweep,
+      // dense 1q targets 6-10: 6.44 TB/s at 2^11, 6.57 at 2^10).
+      go(k_pair<T, K, MOVE, true, TB, TP, kSub, 10, NT>, TB, TP);
+    } else if (K >= 2 && sizeof(T) == 8 && ins.p[0] < 6) {
+      // Complex128 with the lowest position 3-5 (inside a wavefront, from the line width up):
+      // 128 x 1 (30q: controlled (3,20) 5.42 -> 6.16 TB/s, swap (4,25) 5.82 -> 6.57).
+      go(k_pair<T, K, MOVE, true, 128, 1, kSub, kSubLog, NT>, 128, 1);
+    } else if (K >= 2) {
+      constexpr int GB = MOVE ? PairTile<T>::MB : PairTile<T>::CB, GP = MOVE ? PairTile<T>::MP : PairTile<T>::CP;
+      go(k_pair<T, K, MOVE, true, GB, GP, kSub, kSubLog, NT>, GB, GP);
+    } else {
+      // one inserted bit here (two or more took the branch above)
+      constexpr int GB = PairTile<T>::SB, GP = PairTile<T>::SP;
+      go(k_pair<T, K, MOVE, true, GB, GP, kSub, kSubLog, NT>, GB, GP);
+    }
+  });
   CHECK_LAUNCH();
   return IQSH_OK;
 }
@@ -252,8 +269,10 @@ int launch_lane(iqsh_handle h, unsigned t, const Ins<KC>& cins, uint64_t ctrl, c
   using V = typename Vec<T>::t;
   const uint64_t items = h->size() >> KC;
   constexpr int LB = LaneTile<T>::B, LP = LaneTile<T>::P;
-  k_pair_lane<T, KC, COND, MOVE, LB, LP><<<grid2(items / (LB * LP)), LB, 0, g_stream>>>((V*)h->d, t, cins, ctrl,
-                                                                                                  mat2<T>(m));
+  by_cache_policy(h, [&](auto policy) {
+    k_pair_lane<T, KC, COND, MOVE, LB, LP, decltype(policy)::value><<<grid2(items / (LB * LP)), LB, 0, g_stream>>>(
+        (V*)h->d, t, cins, ctrl, mat2<T>(m));
+  });
   CHECK_LAUNCH();
   return IQSH_OK;
 }
@@ -275,10 +294,11 @@ int launch_pair_cond(iqsh_handle h, unsigned t, uint64_t ctrl, const double* m, 
   // complex128: the pair kernel's 128 x 2 shape (30q: 6.0 -> 6.5 TB/s of full-pass traffic).
   constexpr int TB = PairTile<T>::B, TP = PairTile<T>::P;
   const uint64_t grid = items / (TB * TP);
-  if (move)
-    k_pair_cond<T, true, TB, TP><<<grid2(grid), TB, 0, g_stream>>>((V*)h->d, ins, ctrl, mat2<T>(m));
-  else
-    k_pair_cond<T, false, TB, TP><<<grid2(grid), TB, 0, g_stream>>>((V*)h->d, ins, ctrl, mat2<T>(m));
+  by_cache_policy(h, [&](auto policy) {
+    constexpr bool NT = decltype(policy)::value;
+    if (move) k_pair_cond<T, true, TB, TP, NT><<<grid2(grid), TB, 0, g_stream>>>((V*)h->d, ins, ctrl, mat2<T>(m));
+    else k_pair_cond<T, false, TB, TP, NT><<<grid2(grid), TB, 0, g_stream>>>((V*)h->d, ins, ctrl, mat2<T>(m));
+  });
   CHECK_LAUNCH();
   return IQSH_OK;
 }
@@ -308,9 +328,10 @@ int launch_scale(iqsh_handle h, const Ins<K>& ins, uint64_t mask, const double* 
     return launch_diag2<T>(h, pb, pa, d[0], d[1], d[2], d[3]);
   }
   if (items >= kTiledMin)
-    k_scale<T, K, true, DiagTile<T>::B, DiagTile<T>::P><<<grid2(items / (DiagTile<T>::B * DiagTile<T>::P)),
-                                                          DiagTile<T>::B, 0, g_stream>>>((V*)h->d, items, ins, mask,
-                                                                                         cx<T>(f));
+    by_cache_policy(h, [&](auto policy) {
+      k_scale<T, K, true, DiagTile<T>::B, DiagTile<T>::P, decltype(policy)::value>
+          <<<grid2(items / (DiagTile<T>::B * DiagTile<T>::P)), DiagTile<T>::B, 0, g_stream>>>((V*)h->d, items, ins, mask, cx<T>(f));
+    });
   else
     k_scale<T, K, false, kSB, kSP><<<grid2(grid_for(items, kSB * kSP)), kSB, 0, g_stream>>>((V*)h->d, items, ins, mask, cx<T>(f));
   CHECK_LAUNCH();
@@ -323,8 +344,10 @@ int launch_diag2(iqsh_handle h, unsigned p1, unsigned p2, Cx<T> d0, Cx<T> d1, Cx
   using V = typename Vec<T>::t;
   const uint64_t N = h->size();
   if (N >= kTiledMin)
-    k_diag2<T, true, DiagTile<T>::B, DiagTile<T>::P><<<grid2(N / (DiagTile<T>::B * DiagTile<T>::P)), DiagTile<T>::B, 0,
-                                                       g_stream>>>((V*)h->d, N, p1, p2, d0, d1, d2, d3);
+    by_cache_policy(h, [&](auto policy) {
+      k_diag2<T, true, DiagTile<T>::B, DiagTile<T>::P, decltype(policy)::value>
+          <<<grid2(N / (DiagTile<T>::B * DiagTile<T>::P)), DiagTile<T>::B, 0, g_stream>>>((V*)h->d, N, p1, p2, d0, d1, d2, d3);
+    });
   else
     k_diag2<T, false, kSB, kSP><<<grid2(grid_for(N, kSB * kSP)), kSB, 0, g_stream>>>((V*)h->d, N, p1, p2, d0, d1, d2, d3);
   CHECK_LAUNCH();
@@ -1300,20 +1323,16 @@ int launch_quad_lane(iqsh_handle h, unsigned pa, unsigned pb, const Mat4<T>& M, 
   const unsigned hi = std::max(pa, pb);
   const uint64_t items = hi >= 6 ? h->size() >> 1 : h->size();
   using Q = QuadLaneTile<T>;
-  if (hi >= 6) {
-    const uint64_t grid = items / (Q::B * Q::P);
-    if (move)
-      k_quad_lane<T, true, Q::B, Q::P><<<grid2(grid), Q::B, 0, g_stream>>>((V*)h->d, pa, pb, M);
-    else
-      k_quad_lane<T, false, Q::B, Q::P><<<grid2(grid), Q::B, 0, g_stream>>>((V*)h->d, pa, pb, M);
-    CHECK_LAUNCH();
-    return IQSH_OK;
-  }
-  const uint64_t grid = items / (Q::BL * Q::PL);
-  if (move)
-    k_quad_lane<T, true, Q::BL, Q::PL><<<grid2(grid), Q::BL, 0, g_stream>>>((V*)h->d, pa, pb, M);
-  else
-    k_quad_lane<T, false, Q::BL, Q::PL><<<grid2(grid), Q::BL, 0, g_stream>>>((V*)h->d, pa, pb, M);
+  by_cache_policy(h, [&](auto policy) {
+    constexpr bool NT = decltype(policy)::value;
+    auto go = [&](auto kernel, int b, int p) {
+      kernel<<<grid2(items / ((uint64_t)b * p)), b, 0, g_stream>>>((V*)h->d, pa, pb, M);
+    };
+    if (hi >= 6 && move) go(k_quad_lane<T, true, Q::B, Q::P, NT>, Q::B, Q::P);
+    else if (hi >= 6) go(k_quad_lane<T, false, Q::B, Q::P, NT>, Q::B, Q::P);
+    else if (move) go(k_quad_lane<T, true, Q::BL, Q::PL, NT>, Q::BL, Q::PL);
+    else go(k_quad_lane<T, false, Q::BL, Q::PL, NT>, Q::BL, Q::PL);
+  });
   CHECK_LAUNCH();
   return IQSH_OK;
 }
@@ -1399,14 +1418,18 @@ int do_2q(iqsh_handle h, unsigned ph, unsigned pl, const double* m)
   const unsigned ins[2] = {ph, pl};
   const uint64_t items = h->size() >> 2;
   constexpr int TB = PairTile<T>::QB, TP = PairTile<T>::QP;
-  if (items >= kTiledMin && std::max(ph, pl) <= 10)
-    // Both positions <= 10: 1024 x 1 blocks (30q complex128: 6.07-6.23 TB/s against 6.02-6.08
-    // with the small blocks, which are faster above).
-    k_quad<T, true, kTB, 1><<<grid2(items / kTB), kTB, 0, g_stream>>>((V*)h->d, items, sorted_ins<2>(ins),
-                                                                           uint64_t(1) << pl, uint64_t(1) << ph, M);
-  else if (items >= kTiledMin)
-    k_quad<T, true, TB, TP><<<grid2(items / (TB * TP)), TB, 0, g_stream>>>((V*)h->d, items, sorted_ins<2>(ins),
-                                                                            uint64_t(1) << pl, uint64_t(1) << ph, M);
+  if (items >= kTiledMin)
+    by_cache_policy(h, [&](auto policy) {
+      constexpr bool NT = decltype(policy)::value;
+      // Both positions <= 10: 1024 x 1 blocks (30q complex128: 6.07-6.23 TB/s against 6.02-6.08
+      // with the small blocks, which are faster above).
+      if (std::max(ph, pl) <= 10)
+        k_quad<T, true, kTB, 1, NT><<<grid2(items / kTB), kTB, 0, g_stream>>>((V*)h->d, items, sorted_ins<2>(ins),
+                                                                              uint64_t(1) << pl, uint64_t(1) << ph, M);
+      else
+        k_quad<T, true, TB, TP, NT><<<grid2(items / (TB * TP)), TB, 0, g_stream>>>((V*)h->d, items, sorted_ins<2>(ins),
+                                                                                   uint64_t(1) << pl, uint64_t(1) << ph, M);
+    });
   else
     k_quad<T, false, kSB, 2><<<grid2(grid_for(items, kSB * 2)), kSB, 0, g_stream>>>((V*)h->d, items, sorted_ins<2>(ins),
                                                                             uint64_t(1) << pl, uint64_t(1) << ph, M);

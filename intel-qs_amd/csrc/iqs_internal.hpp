@@ -30,6 +30,15 @@ int fail(int code, const char* fmt, ...) __attribute__((format(printf, 2, 3)));
 hipStream_t stream();
 // Compute units of the current device.
 int device_cus();
+// Whether amplitudes of `bytes` in all, gone over again by call after call, stay in the 256 MiB
+// last-level cache if the kernels use ordinary accesses (non-temporal ones stream past it).
+// Measured with one kernel after another on the same register: dense 1q complex128 21
+// qubits (32 MiB) 11.0 -> 7.5 us, 22 qubits 22 -> 19.5, 24 qubits (256 MiB) 85 -> 72.5; QAOA
+// layer 24 qubits 298 -> 241.  Above 256 MiB non-temporal accesses stream faster (25 qubits 167
+// against 177 us, layer at 26 qubits 1188 against 1236); below 32 MiB stores that stay in the
+// L2s cost more when the kernel ends and writes them back (20 qubits 4.6 against 5.3 us, layer 21
+// against 30).
+inline bool cache_set(uint64_t bytes) { return bytes >= (uint64_t(32) << 20) && bytes <= (uint64_t(256) << 20); }
 // Edge-parity tables and phase table of a MaxCut cost for register h (at most 64 edges):
 // the phase exp(-i gamma cut) per amplitude.
 int build_cut_spec(iqsh_handle h, unsigned ne, const unsigned* u, const unsigned* v, const double* w, double gamma,

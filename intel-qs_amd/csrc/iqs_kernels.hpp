@@ -201,7 +201,7 @@ __global__ __launch_bounds__(B) void k_pair(typename Vec<T>::t* __restrict__ st,
 //           controls below 6, whose skipped amplitudes share cache lines with updated ones).
 // MOVE exchanges partners exactly (X-type matrices).  Requires (N >> KC) a multiple of
 // B*P and >= kTiledMin (grid a multiple of 8).
-template <typename T, int KC, bool COND, bool MOVE, int B, int P>
+template <typename T, int KC, bool COND, bool MOVE, int B, int P, bool NT>
 __global__ __launch_bounds__(B) void k_pair_lane(typename Vec<T>::t* __restrict__ st, unsigned pos, Ins<KC> cins,
                                                  uint64_t ctrl, Mat2<T> m)
 {
@@ -213,7 +213,7 @@ __global__ __launch_bounds__(B) void k_pair_lane(typename Vec<T>::t* __restrict_
   for (int j = 0; j < P; ++j) {
     const uint64_t r = r0 + (uint64_t)j * B;
     idx[j] = KC > 0 ? (item_base(r, cins) | ctrl) : r;
-    v[j] = ldg(&st[idx[j]]);
+    v[j] = ldx<NT>(&st[idx[j]]);
   }
   const int msk = 1 << pos;
   const bool upper = (threadIdx.x >> pos) & 1;
@@ -226,14 +226,14 @@ __global__ __launch_bounds__(B) void k_pair_lane(typename Vec<T>::t* __restrict_
     if (MOVE) o = p;
     else o = upper ? cmad2(m.m10, p, m.m11, v[j]) : cmad2(m.m00, v[j], m.m01, p);
     if (COND && (idx[j] & ctrl) != ctrl) o = v[j];
-    stg(o, &st[idx[j]]);
+    stx<NT>(o, &st[idx[j]]);
   }
 }
 
 // Conditional pair update over the target only (controls below 3 share 128-byte lines
 // with uncontrolled amplitudes): every pair is read and written back, the update applied
 // where (i0 & ctrl) == ctrl.  Tiled mapping as k_pair.
-template <typename T, bool MOVE, int B, int P>
+template <typename T, bool MOVE, int B, int P, bool NT>
 __global__ __launch_bounds__(B) void k_pair_cond(typename Vec<T>::t* __restrict__ st, Ins<1> ins, uint64_t ctrl,
                                                  Mat2<T> m)
 {
@@ -245,8 +245,8 @@ __global__ __launch_bounds__(B) void k_pair_cond(typename Vec<T>::t* __restrict_
 #pragma unroll
   for (int j = 0; j < P; ++j) {
     base[j] = item_base(tiled_item<B, P, kSub>(bb, j * B + threadIdx.x), ins);
-    a[j] = ldg(&st[base[j]]);
-    b[j] = ldg(&st[base[j] | hb]);
+    a[j] = ldx<NT>(&st[base[j]]);
+    b[j] = ldx<NT>(&st[base[j] | hb]);
   }
 #pragma unroll
   for (int j = 0; j < P; ++j) {
@@ -260,8 +260,8 @@ __global__ __launch_bounds__(B) void k_pair_cond(typename Vec<T>::t* __restrict_
         y = cmad2(m.m10, a[j], m.m11, b[j]);
       }
     }
-    stg(x, &st[base[j]]);
-    stg(y, &st[base[j] | hb]);
+    stx<NT>(x, &st[base[j]]);
+    stx<NT>(y, &st[base[j] | hb]);
   }
 }
 
@@ -269,7 +269,7 @@ __global__ __launch_bounds__(B) void k_pair_cond(typename Vec<T>::t* __restrict_
 // Scale kernel: st[b|mask] *= f for every item (K=0: the whole state).  Serves diagonal
 // gates whose other entries are exactly 1 (Z, S, T, CZ, CPhase, ...) by touching only the
 // amplitudes that change.
-template <typename T, int K, bool TILED, int B, int P>
+template <typename T, int K, bool TILED, int B, int P, bool NT = true>
 __global__ __launch_bounds__(B) void k_scale(typename Vec<T>::t* __restrict__ st, uint64_t nitems, Ins<K> ins,
                                              uint64_t mask, Cx<T> f)
 {
@@ -281,10 +281,10 @@ __global__ __launch_bounds__(B) void k_scale(typename Vec<T>::t* __restrict__ st
 #pragma unroll
     for (int j = 0; j < P; ++j) {
       idx[j] = item_base(tiled_item<B, P, kSub>(bb, j * B + threadIdx.x), ins) | mask;
-      a[j] = ldg(&st[idx[j]]);
+      a[j] = ldx<NT>(&st[idx[j]]);
     }
 #pragma unroll
-    for (int j = 0; j < P; ++j) stg(cmul(f, a[j]), &st[idx[j]]);
+    for (int j = 0; j < P; ++j) stx<NT>(cmul(f, a[j]), &st[idx[j]]);
   } else {
     for (int j = 0; j < P; ++j) {
       const uint64_t k = block_id() * (B * P) + (uint64_t)j * B + threadIdx.x;
@@ -296,7 +296,7 @@ __global__ __launch_bounds__(B) void k_scale(typename Vec<T>::t* __restrict__ st
 }
 
 // Elementwise 2-qubit diagonal: st[i] *= d[2*b(p1) + b(p2)].
-template <typename T, bool TILED, int B, int P>
+template <typename T, bool TILED, int B, int P, bool NT = true>
 __global__ __launch_bounds__(B) void k_diag2(typename Vec<T>::t* __restrict__ st, uint64_t N, unsigned p1, unsigned p2,
                                              Cx<T> d0, Cx<T> d1, Cx<T> d2, Cx<T> d3)
 {
@@ -307,7 +307,7 @@ __global__ __launch_bounds__(B) void k_diag2(typename Vec<T>::t* __restrict__ st
 #pragma unroll
   for (int j = 0; j < P; ++j) {
     idx[j] = TILED ? tiled_item<B, P, kSub>(bb, j * B + threadIdx.x) : bb * (uint64_t)(B * P) + (uint64_t)j * B + threadIdx.x;
-    if (TILED || idx[j] < N) a[j] = ldg(&st[idx[j]]);
+    if (TILED || idx[j] < N) a[j] = ldx<NT>(&st[idx[j]]);
   }
 #pragma unroll
   for (int j = 0; j < P; ++j) {
@@ -315,13 +315,13 @@ __global__ __launch_bounds__(B) void k_diag2(typename Vec<T>::t* __restrict__ st
     if (TILED || i < N) {
       const bool b1 = (i >> p1) & 1, b2 = (i >> p2) & 1;
       const Cx<T> d = b1 ? (b2 ? d3 : d2) : (b2 ? d1 : d0);
-      stg(cmul(d, a[j]), &st[i]);
+      stx<NT>(cmul(d, a[j]), &st[i]);
     }
   }
 }
 
 // Dense 4x4 on (ph, pl): indices b, b|dl, b|dh, b|dh|dl; new[t] = sum_c m[t][c] old[c].
-template <typename T, bool TILED, int B, int P, int SUB = kSub, unsigned SL = kSubLog>
+template <typename T, bool TILED, int B, int P, bool NT = true, int SUB = kSub, unsigned SL = kSubLog>
 __global__ __launch_bounds__(B) void k_quad(typename Vec<T>::t* __restrict__ st, uint64_t nitems, Ins<2> ins,
                                             uint64_t dl, uint64_t dh, Mat4<T> m)
 {
@@ -336,10 +336,10 @@ __global__ __launch_bounds__(B) void k_quad(typename Vec<T>::t* __restrict__ st,
     ok[j] = TILED || k < nitems;
     base[j] = item_base(k, ins);
     if (ok[j]) {
-      x[j][0] = ldg(&st[base[j]]);
-      x[j][1] = ldg(&st[base[j] | dl]);
-      x[j][2] = ldg(&st[base[j] | dh]);
-      x[j][3] = ldg(&st[base[j] | dh | dl]);
+      x[j][0] = ldx<NT>(&st[base[j]]);
+      x[j][1] = ldx<NT>(&st[base[j] | dl]);
+      x[j][2] = ldx<NT>(&st[base[j] | dh]);
+      x[j][3] = ldx<NT>(&st[base[j] | dh | dl]);
     }
   }
 #pragma unroll
@@ -352,7 +352,7 @@ __global__ __launch_bounds__(B) void k_quad(typename Vec<T>::t* __restrict__ st,
       const V s = cmad2(m.m[4 * t + 2], x[j][2], m.m[4 * t + 3], x[j][3]);
       r.x += s.x;
       r.y += s.y;
-      stg(r, &st[base[j] | off[t]]);
+      stx<NT>(r, &st[base[j] | off[t]]);
     }
   }
 }
@@ -400,7 +400,7 @@ __device__ __forceinline__ V quad_row_lane(const Mat4<T>& m, bool ul, bool uh, c
 
 // LOB: the lower position is pb (row bit 0); otherwise pa.  Inputs are named by (bit lo,
 // bit hi); rows are row(l, h) = LOB ? 2h + l : 2l + h, all compile-time.
-template <typename T, bool MOVE, bool LOB, int B, int P>
+template <typename T, bool MOVE, bool LOB, int B, int P, bool NT>
 __device__ __forceinline__ void quad_lane_body(typename Vec<T>::t* __restrict__ st, unsigned lo, unsigned hi,
                                                const Mat4<T>& m)
 {
@@ -416,8 +416,8 @@ __device__ __forceinline__ void quad_lane_body(typename Vec<T>::t* __restrict__ 
 #pragma unroll
     for (int j = 0; j < P; ++j) {
       idx[j] = ins0(r0 + (uint64_t)j * B, hi);
-      a[j] = ldg(&st[idx[j]]);
-      b[j] = ldg(&st[idx[j] | hb]);
+      a[j] = ldx<NT>(&st[idx[j]]);
+      b[j] = ldx<NT>(&st[idx[j] | hb]);
     }
 #pragma unroll
     for (int j = 0; j < P; ++j) {
@@ -439,8 +439,8 @@ __device__ __forceinline__ void quad_lane_body(typename Vec<T>::t* __restrict__ 
         o0 = quad_row_lane<R00, R10, R00, R10>(m, ul, false, x00, i1, i2, x11);
         o1 = quad_row_lane<R01, R11, R01, R11>(m, ul, false, x00, i1, i2, x11);
       }
-      stg(o0, &st[idx[j]]);
-      stg(o1, &st[idx[j] | hb]);
+      stx<NT>(o0, &st[idx[j]]);
+      stx<NT>(o1, &st[idx[j] | hb]);
     }
   } else {
     const int mh = 1 << hi;
@@ -450,7 +450,7 @@ __device__ __forceinline__ void quad_lane_body(typename Vec<T>::t* __restrict__ 
 #pragma unroll
     for (int j = 0; j < P; ++j) {
       idx[j] = r0 + (uint64_t)j * B;
-      v[j] = ldg(&st[idx[j]]);
+      v[j] = ldx<NT>(&st[idx[j]]);
     }
 #pragma unroll
     for (int j = 0; j < P; ++j) {
@@ -472,20 +472,20 @@ __device__ __forceinline__ void quad_lane_body(typename Vec<T>::t* __restrict__ 
         const V x11 = ul ? (uh ? v[j] : xh) : (uh ? xl : xb);
         o = quad_row_lane<R00, R10, R01, R11>(m, ul, uh, x00, LOB ? x10 : x01, LOB ? x01 : x10, x11);
       }
-      stg(o, &st[idx[j]]);
+      stx<NT>(o, &st[idx[j]]);
     }
   }
 }
 
-template <typename T, bool MOVE, int B, int P>
+template <typename T, bool MOVE, int B, int P, bool NT>
 __global__ __launch_bounds__(B) void k_quad_lane(typename Vec<T>::t* __restrict__ st, unsigned pa, unsigned pb,
                                                  Mat4<T> m)
 {
   const unsigned lo = pa < pb ? pa : pb, hi = pa < pb ? pb : pa;
   if (lo == pb)
-    quad_lane_body<T, MOVE, true, B, P>(st, lo, hi, m);
+    quad_lane_body<T, MOVE, true, B, P, NT>(st, lo, hi, m);
   else
-    quad_lane_body<T, MOVE, false, B, P>(st, lo, hi, m);
+    quad_lane_body<T, MOVE, false, B, P, NT>(st, lo, hi, m);
 }
 
 // ---------------------------------------------------------------------------------------

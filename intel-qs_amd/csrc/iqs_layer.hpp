@@ -472,14 +472,6 @@ int layer_m(const LayerArgs& a)
   return IQSH_OK;
 }
 
-// Cache policy by the bytes that the passes go over again and again (psi, and lam in the
-// adjoint).  From 32 to 256 MiB they stay in the 256 MiB last-level cache under ordinary
-// accesses: forward complex128 22 qubits 79 -> 64 us, 24 qubits 298 -> 241 us, complex64 24
-// qubits 159 -> 136, adjoint complex128 22 qubits 198 -> 169.  Above, non-temporal accesses
-// stream faster (26 qubits 1188 against 1236 us); below, stores that stay in the L2s cost
-// more when the kernel ends and writes them back (20 qubits 21 against 30 us).
-inline bool cache_set(uint64_t bytes) { return bytes >= (uint64_t(32) << 20) && bytes <= (uint64_t(256) << 20); }
-
 // Tile size: large tiles (long rows, fewest passes) for registers that fill the chip with
 // them; below that the smallest tile that takes no more passes, for more workgroups (18
 // qubits complex128 takes 14.1 us with 64 tiles of 2^12, 12.6 with 128 of 2^11, but at 20 qubits
@@ -491,7 +483,7 @@ template <typename T, bool ADJ, int F>
 int layer_n(const LayerArgs& a)
 {
   const unsigned n = a.psi->n;
-  const bool cached = cache_set(a.psi->size() * sizeof(typename Vec<T>::t) * (ADJ ? 2 : 1));
+  const bool cached = iqsi::cache_set(a.psi->size() * sizeof(typename Vec<T>::t) * (ADJ ? 2 : 1));
   if constexpr (sizeof(T) == 8) {
     if (n <= 10 || (n > 12 && n <= 16)) return layer_m<T, 10, 4, ADJ, F>(a);
     if (n == 11 || n == 17 || n == 18) return layer_m<T, 11, 4, ADJ, F>(a);
