@@ -590,3 +590,32 @@ def test_controlled_tiled_line_aligned_control(dt, c, t):
     sv.apply_c1q(c, t, [[0, 1], [1, 0]])  # CNOT: exact move
     oracle.apply_c1q(h, c, t, np.array([[0, 1], [1, 0]]))
     assert np.array_equal(sv.download(), h)
+
+
+@pytest.mark.parametrize("dt", ["c128", "c64"])
+@pytest.mark.parametrize("n", [14, 15, 16, 21])
+def test_controlled_phase_with_a_position_inside_a_line(dt, n):
+    """One non-unit diagonal entry with one position inside a 128-byte line and one above it
+    (half of the lines are touched), on both sides of the size from which that kernel runs,
+    and with the cached accesses of a 32 MiB register (21 qubits complex128): each entry, each
+    order of the positions.  One complex product per touched amplitude; the others bit-equal."""
+    r = np.random.default_rng(n)
+    v = r.normal(size=1 << n) + 1j * r.normal(size=1 << n)
+    v = (v / np.linalg.norm(v)).astype(np.complex128 if dt == "c128" else np.complex64)
+    x = np.arange(1 << n)
+    f = np.exp(0.7j)
+    line = 3 if dt == "c128" else 4
+    sv = StateVector(n, dt)
+    for lo, hi in ((0, line), (line - 1, n - 1), (1, n // 2)):
+        for p1, p2 in ((lo, hi), (hi, lo)):
+            for entry in range(4):
+                d = np.ones(4, dtype=np.complex128)
+                d[entry] = f
+                sv.upload(v)
+                sv.apply_diag2(p1, p2, d)
+                got = sv.download()
+                touched = 2 * ((x >> p1) & 1) + ((x >> p2) & 1) == entry
+                assert np.array_equal(got[~touched], v[~touched])
+                want = v[touched].astype(np.complex128) * f
+                eps = 2.0 ** -52 if dt == "c128" else 2.0 ** -23
+                assert np.abs(got[touched] - want).max() < 4 * eps * np.abs(v).max()
