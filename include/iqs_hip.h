@@ -131,6 +131,18 @@ int iqsh_apply_2q(iqsh_handle h, unsigned ph, unsigned pl, const double m[32]);
  * 1 <= k <= 5.  Replaces the reference's fused-gate replay (src/qureg_fusion.cpp:56-94):
  * a run of gates is multiplied into one block on the host and applied in one pass. */
 int iqsh_apply_kq(iqsh_handle h, unsigned k, const unsigned *pos, const double *U);
+/* A list of one- and two-qubit gates (np = 1: a row-major 2x2 on p[0]; np = 2: a 4x4 on (p[0],
+ * p[1]), row index 2*b(p[0]) + b(p[1])), applied together: gates on disjoint positions are
+ * reordered, and every pass over the state applies all gates that become ready on the
+ * positions of one tile, multiplied into dense blocks of at most `block` (1..5) positions.
+ * Registers below 10 qubits take one pass per block.  *launched (may be null) receives the
+ * number of passes.  Replaces the reference's fused-gate replay (src/qureg_fusion.cpp:56-94). */
+typedef struct {
+  unsigned np;
+  unsigned p[2];
+  double m[32];
+} iqsh_gate;
+int iqsh_apply_gates(iqsh_handle h, uint64_t ngates, const iqsh_gate *gates, unsigned block, uint64_t *launched);
 /* Select the kernel for 5-qubit blocks (and 3-/4-qubit blocks padded to 5): 1 (default)
  * matrix cores, three real 32x32 products per block (Ur xr, Ui xi, (Ur+Ui)(xr+xi));
  * 2 matrix cores, one real 64x64 product; 0 vector ALUs.  Process-wide. */

@@ -311,16 +311,18 @@ int launch_scale(iqsh_handle h, const Ins<K>& ins, uint64_t mask, const double* 
 {
   using V = typename Vec<T>::t;
   const uint64_t items = h->size() >> K;
-  if (K == 2 && ins.p[0] < line_bits<T>() && ins.p[1] >= line_bits<T>() && h->size() / 2 >= kTiledMin) {
-    // One position inside a 128-byte line, one above: only the lines that hold touched
-    // amplitudes, half of the state.
-    using D = DiagTile<T>;
-    by_cache_policy(h, [&](auto policy) {
-      k_scale_line<T, D::B, D::P, decltype(policy)::value><<<grid2(h->size() / 2 / (D::B * D::P)), D::B, 0, g_stream>>>(
-          (V*)h->d, ins.p[1], ins.p[0], mask, cx<T>(f));
-    });
-    CHECK_LAUNCH();
-    return IQSH_OK;
+  if constexpr (K == 2) {
+    if (ins.p[0] < line_bits<T>() && ins.p[1] >= line_bits<T>() && h->size() / 2 >= kTiledMin) {
+      // One position inside a 128-byte line, one above: only the lines that hold touched
+      // amplitudes, half of the state.
+      using D = DiagTile<T>;
+      by_cache_policy(h, [&](auto policy) {
+        k_scale_line<T, D::B, D::P, decltype(policy)::value><<<grid2(h->size() / 2 / (D::B * D::P)), D::B, 0, g_stream>>>(
+            (V*)h->d, ins.p[1], ins.p[0], mask, cx<T>(f));
+      });
+      CHECK_LAUNCH();
+      return IQSH_OK;
+    }
   }
   if (K >= 1 && K <= 2 && ins.p[0] < line_bits<T>() && h->size() >= kTiledMin) {
     // Every position inside a 128-byte line: the touched amplitudes share every line with

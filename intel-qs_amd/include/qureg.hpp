@@ -162,16 +162,17 @@ class QubitRegister
   void ApplyCPhaseRotation(unsigned const qubit, unsigned const qubit2, BaseType theta);
 
   // ---- fusion ----
-  /// Gates are queued and applied as dense blocks of up to FusionBlockQubits() qubits,
-  /// one HBM pass per block (the reference's fusion replays queued gates cache block by
-  /// cache block, src/qureg_fusion.cpp).  log2llc is kept for API compatibility.
+  /// Gates are queued, multiplied into dense blocks of up to FusionBlockQubits() qubits and
+  /// applied several blocks to a pass over the state (iqsh_apply_gates; the reference's fusion
+  /// replays queued gates cache block by cache block, src/qureg_fusion.cpp).  log2llc is kept
+  /// for API compatibility.
   void TurnOnFusion(unsigned log2llc = 20);
   void TurnOffFusion();
   bool IsFusionEnabled();
   void ApplyFusedGates();
   void SetFusionBlockQubits(unsigned k);
   unsigned FusionBlockQubits() const { return fuse_k_; }
-  /// (queued gates applied so far, blocks launched for them) since construction.
+  /// (queued gates applied so far, passes launched for them) since construction.
   std::pair<std::size_t, std::size_t> FusionStats() const { return {fused_gates_, fused_blocks_}; }
 
   // ---- specialization ----

@@ -60,6 +60,7 @@ def _sig(L):
         "iqsh_apply_diag2": [P, U, U, P],
         "iqsh_apply_2q": [P, U, U, P],
         "iqsh_apply_kq": [P, U, P, P],
+        "iqsh_apply_gates": [P, U64, P, U, C.POINTER(U64)],
         "iqsh_set_block_mfma": [I],
         "iqsh_scale": [P, D, D],
         "iqsh_axpy": [P, P, D, D],

@@ -49,17 +49,12 @@ void m2(const TM2x2<Type>& m, Type out[4])
   out[3] = m(1, 1);
 }
 
-using cd = std::complex<double>;
-
 }  // namespace
 
 // A queued gate: a 2x2 (np = 1) or 4x4 (np = 2, row index 2*b(p[0]) + b(p[1])) matrix on
 // data positions, resolved when the gate was queued.
 template <class Type>
-struct QubitRegister<Type>::Pending {
-  unsigned np;
-  unsigned p[2];
-  cd m[16];
+struct QubitRegister<Type>::Pending : iqsh_gate {
 };
 
 // ---------------------------------------------------------------------------------------
@@ -393,13 +388,12 @@ void QubitRegister<Type>::cgate1_(unsigned c, unsigned t, const Type m[4], GateS
 template <class Type>
 void QubitRegister<Type>::enqueue_(unsigned np, unsigned p0, unsigned p1, const Type* m)
 {
-  Pending g;
+  queue_->emplace_back();
+  Pending& g = queue_->back();
   g.np = np;
   g.p[0] = p0;
   g.p[1] = p1;
-  const int cnt = np == 1 ? 4 : 16;
-  for (int i = 0; i < cnt; ++i) g.m[i] = cd((double)m[i].real(), (double)m[i].imag());
-  queue_->push_back(g);
+  to_doubles(m, np == 1 ? 4 : 16, g.m);
 }
 
 // The 2x2 (as 8 doubles) a sub-range helper applies: the SpecializeV2 constants when that
@@ -859,7 +853,7 @@ void QubitRegister<Type>::ApplyToffoli(unsigned const c1, unsigned const c2, uns
 }
 
 // ---------------------------------------------------------------------------------------
-// fusion: queued gates are multiplied into dense blocks of <= fuse_k_ positions
+// fusion: queued gates are multiplied into dense blocks and applied together (iqsh_apply_gates)
 
 template <class Type>
 void QubitRegister<Type>::TurnOnFusion(unsigned l2)
@@ -907,130 +901,9 @@ void QubitRegister<Type>::ApplyFusedGates()
   }
   host_valid_ = false;
 
-  // Plan the blocks over the gates' dependency graph (gate j depends on the previous gate on
-  // each of its positions; gates on disjoint positions commute).  A block starts empty and
-  // repeatedly absorbs the ready gate (every predecessor already placed) that adds the fewest
-  // new positions, oldest first, while it stays within fuse_k_ positions; the gates of a
-  // block multiply in absorption order, which respects every dependency.  200 Haar-random
-  // 1q/2q gates on 32 positions (seed 20240603) take 26 blocks of <= 5 positions this way,
-  // against 59 when a block is closed at the first gate that does not fit.
-  const std::size_t ng = q.size();
-  std::vector<std::vector<std::size_t>> succ(ng);
-  std::vector<unsigned> npred(ng, 0);
-  {
-    std::vector<long> last(64, -1);
-    for (std::size_t i = 0; i < ng; ++i) {
-      long prev = -1;
-      for (unsigned j = 0; j < q[i].np; ++j) {
-        const long l = last[q[i].p[j]];
-        if (l >= 0 && l != prev) {
-          succ[(std::size_t)l].push_back(i);
-          ++npred[i];
-          prev = l;
-        }
-        last[q[i].p[j]] = (long)i;
-      }
-    }
-  }
-  std::vector<std::size_t> ready;  // ascending gate index
-  for (std::size_t i = 0; i < ng; ++i)
-    if (!npred[i]) ready.push_back(i);
-  std::vector<std::vector<std::size_t>> plan;
-  while (!ready.empty()) {
-    std::vector<std::size_t> blk;
-    std::vector<unsigned> Q;
-    for (;;) {
-      std::size_t best = ready.size();
-      unsigned best_add = ~0u;
-      for (std::size_t r = 0; r < ready.size() && best_add != 0; ++r) {
-        const Pending& g = q[ready[r]];
-        unsigned add = 0;
-        for (unsigned j = 0; j < g.np; ++j) add += std::find(Q.begin(), Q.end(), g.p[j]) == Q.end();
-        // (a gate wider than fuse_k_ is a block of its own)
-        if ((Q.size() + add <= fuse_k_ || Q.empty()) && add < best_add) {
-          best = r;
-          best_add = add;
-        }
-      }
-      if (best == ready.size()) break;
-      const std::size_t gi = ready[best];
-      ready.erase(ready.begin() + (long)best);
-      for (unsigned j = 0; j < q[gi].np; ++j)
-        if (std::find(Q.begin(), Q.end(), q[gi].p[j]) == Q.end()) Q.push_back(q[gi].p[j]);
-      blk.push_back(gi);
-      for (std::size_t sj : succ[gi])
-        if (--npred[sj] == 0) ready.insert(std::lower_bound(ready.begin(), ready.end(), sj), sj);
-    }
-    plan.push_back(std::move(blk));
-  }
-
-  std::vector<unsigned> S;  // block positions; row-index bit j <-> S[j]
-  std::vector<cd> B;        // 2^|S| x 2^|S| row-major
-  int ngates = 0;
-  auto emit = [&]() {
-    if (S.empty()) return;
-    const unsigned k = (unsigned)S.size();
-    const std::size_t D = std::size_t(1) << k;
-    std::vector<double> md(2 * D * D);
-    for (std::size_t i = 0; i < D * D; ++i) {
-      md[2 * i] = B[i].real();
-      md[2 * i + 1] = B[i].imag();
-    }
-    if (k == 1) ck(iqsh_apply_1q(h_, S[0], md.data()));
-    else if (k == 2) ck(iqsh_apply_2q(h_, S[1], S[0], md.data()));  // row = 2*b(S[1]) + b(S[0])
-    else ck(iqsh_apply_kq(h_, k, S.data(), md.data()));
-    ++fused_blocks_;
-    S.clear();
-    B.clear();
-    ngates = 0;
-  };
-  for (const std::vector<std::size_t>& blk : plan) {
-    for (std::size_t gi : blk) {
-      const Pending& g = q[gi];
-      // Positions of the gate, in its own index order: for np = 2, gate row = 2*b(p[0]) + b(p[1]).
-      std::vector<unsigned> U(S);
-      for (unsigned j = 0; j < g.np; ++j)
-        if (std::find(U.begin(), U.end(), g.p[j]) == U.end()) U.push_back(g.p[j]);
-      // Grow B to the positions U (new positions appended above the old ones: B (x) I).
-      const std::size_t Dold = std::size_t(1) << S.size(), D = std::size_t(1) << U.size();
-      std::vector<cd> Bn(D * D, cd(0, 0));
-      if (S.empty()) {
-        for (std::size_t i = 0; i < D; ++i) Bn[i * D + i] = 1.0;
-      } else {
-        for (std::size_t r = 0; r < D; ++r)
-          for (std::size_t c = 0; c < D; ++c)
-            if ((r / Dold) == (c / Dold)) Bn[r * D + c] = B[(r % Dold) * Dold + (c % Dold)];
-      }
-      S = U;
-      // Left-multiply by the gate expanded to S.
-      unsigned bitof[2];
-      for (unsigned j = 0; j < g.np; ++j)
-        bitof[j] = (unsigned)(std::find(S.begin(), S.end(), g.p[j]) - S.begin());
-      const std::size_t gmask = (g.np == 1) ? (std::size_t(1) << bitof[0])
-                                            : ((std::size_t(1) << bitof[0]) | (std::size_t(1) << bitof[1]));
-      auto gidx = [&](std::size_t r) -> unsigned {
-        if (g.np == 1) return (unsigned)((r >> bitof[0]) & 1);
-        return (unsigned)(2 * ((r >> bitof[0]) & 1) + ((r >> bitof[1]) & 1));
-      };
-      const unsigned gd = g.np == 1 ? 2 : 4;
-      std::vector<cd> R(D * D, cd(0, 0));
-      for (std::size_t r = 0; r < D; ++r) {
-        const unsigned gr = gidx(r);
-        for (unsigned gc = 0; gc < gd; ++gc) {
-          const cd gv = g.m[gr * gd + gc];
-          if (gv == cd(0, 0)) continue;
-          // the index that differs from r only in the gate bits, with gate value gc
-          std::size_t rr = r & ~gmask;
-          if (g.np == 1) rr |= (std::size_t)(gc & 1) << bitof[0];
-          else rr |= ((std::size_t)((gc >> 1) & 1) << bitof[0]) | ((std::size_t)(gc & 1) << bitof[1]);
-          for (std::size_t c = 0; c < D; ++c) R[r * D + c] += gv * Bn[rr * D + c];
-        }
-      }
-      B.swap(R);
-      ++ngates;
-    }
-    emit();
-  }
+  uint64_t launched = 0;
+  ck(iqsh_apply_gates(h_, q.size(), q.data(), fuse_k_, &launched));
+  fused_blocks_ += launched;
 }
 
 // ---------------------------------------------------------------------------------------

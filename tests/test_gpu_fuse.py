@@ -1,0 +1,87 @@
+"""Gate lists applied together (iqsh_apply_gates, TurnOnFusion) against the same gates one by
+one on the GPU: sizes around the tile (2^10 below 12 qubits, 2^12 from there; dense blocks below
+10), every block size, lists that fill more than one slot of the descriptor ring, repeated pairs
+in both orders, gates on fresh and on used qubits, and the cached accesses of a 32 MiB register.
+Tolerances: those of the fused-against-unfused tests (1e-12, 2e-5 absolute)."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from iqs_amd import runner
+from iqs_amd._lib import IqsError, call
+from iqs_amd.circuits import Circuit, SplitMix64, haar_unitary
+from iqs_amd.engine import StateVector
+
+pytestmark = pytest.mark.gpu
+TOL = {"dp": 1e-12, "sp": 2e-5}
+
+
+def _mixed(n, count, seed, precision):
+    """Random one- and two-qubit gates, CNOTs, repeated pairs (both orders) and rotations."""
+    r = SplitMix64(seed)
+    c = Circuit(n, precision=precision, init="plus")
+    pair = (0, 1)
+    for i in range(count):
+        k = r.randint(6)
+        a = r.randint(n)
+        b = (a + 1 + r.randint(n - 1)) % n
+        if k == 0:
+            c.add("Apply1QubitGate", a, haar_unitary(2, r))
+        elif k == 1:
+            c.add("Apply2QubitGate", a, b, haar_unitary(4, r))
+            pair = (a, b)
+        elif k == 2:
+            c.add("ApplyCPauliX", a, b)
+        elif k == 3:
+            c.add("Apply2QubitGate", pair[1], pair[0], haar_unitary(4, r))
+        elif k == 4:
+            c.add("ApplyRotationZ", a, r.uniform(0.0, 6.0))
+        else:
+            c.add("ApplyHadamard", a)
+    return c
+
+
+def _compare(c, block):
+    ref, _ = runner.run(c)
+    reg = runner.new_register(c)
+    reg.SetFusionBlockQubits(block)
+    reg.TurnOnFusion()
+    reg, _ = runner.run(c, reg)
+    assert np.abs(runner.state_of(reg) - runner.state_of(ref)).max() < TOL[c.precision]
+    return reg.FusionStats()
+
+
+@pytest.mark.parametrize("precision", ["dp", "sp"])
+@pytest.mark.parametrize("n", [2, 5, 9, 10, 11, 12, 13, 15, 17, 21, 22])
+def test_gate_lists_match_single_gates(precision, n):
+    for count, seed in ((1, 3), (7, 4), (60, 5)):
+        _compare(_mixed(n, count, 100 * n + seed, precision), 5)
+
+
+@pytest.mark.parametrize("block", [1, 2, 3, 4])
+@pytest.mark.parametrize("n", [8, 10, 14])
+def test_block_sizes(n, block):
+    _compare(_mixed(n, 40, n + block, "dp"), block)
+
+
+def test_long_lists_take_several_launches():
+    gates, passes = _compare(_mixed(12, 900, 8, "dp"), 5)
+    assert gates == 900 and passes >= 2  # one tile, more blocks than one launch holds
+    _compare(_mixed(14, 900, 9, "sp"), 5)
+
+
+def test_bad_gate_lists_are_refused():
+    class Gate(C.Structure):
+        _fields_ = [("np", C.c_uint), ("p", C.c_uint * 2), ("m", C.c_double * 32)]
+
+    sv = StateVector(11, "c128")
+    sv.init_basis(3)
+    passes = C.c_uint64(7)
+    call("iqsh_apply_gates", sv.handle, 0, None, 5, C.byref(passes))
+    assert passes.value == 0
+    for np_, p, block in ((0, (0, 1), 5), (3, (0, 1), 5), (1, (11, 0), 5), (2, (4, 4), 5), (2, (0, 1), 0), (2, (0, 1), 6)):
+        g = Gate(np_, (C.c_uint * 2)(*p))
+        with pytest.raises(IqsError):
+            call("iqsh_apply_gates", sv.handle, 1, C.byref(g), block, None)
+    assert sv.prob1(0) == 1.0 and sv.norm2() == 1.0
