@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <chrono>
 #include <cmath>
 #include <complex>
 #include <cstdarg>
@@ -42,29 +43,27 @@ int fail(int code, const char* fmt, ...)
 
 #define CHECK_LAUNCH() HIP_TRY(hipGetLastError())
 
-// ---- reduction workspace: partial sums [NV][kMaxBlocks] + result [NV], pinned host copy ----
+// ---- reduction workspace: partial results [NV][kMaxRedBlocks] in pinned host memory, written
+// there by the reduction kernels' workgroups and summed by the host (red_finish) ----
 constexpr int kMaxRedBlocks = 2048;
 constexpr int kMaxRedVals = 4;
 struct RedWork {
   double* partial = nullptr;
-  double* result = nullptr;
-  double* host = nullptr;
 };
 RedWork g_red;
 std::mutex g_mu;
 // One reduction at a time uses g_red: a reduction holds this from its first launch until
-// red_finish has synchronized the stream, so host threads sharing the library do not race
-// on the partial sums.
+// red_finish has every partial result, so host threads sharing the library do not race on
+// them.
 std::mutex g_red_mu;
 
-int red_ws(RedWork** out)
+// The workspace, marked for a reduction of `nv` values over `nblocks` workgroups.
+int red_ws(RedWork** out, unsigned nblocks, unsigned nv)
 {
   std::lock_guard<std::mutex> lk(g_mu);
-  if (!g_red.partial) {
-    HIP_TRY(hipMalloc(&g_red.partial, sizeof(double) * kMaxRedVals * kMaxRedBlocks));
-    HIP_TRY(hipMalloc(&g_red.result, sizeof(double) * kMaxRedVals));
-    HIP_TRY(hipHostMalloc((void**)&g_red.host, sizeof(double) * kMaxRedVals, hipHostMallocDefault));
-  }
+  if (!g_red.partial)
+    HIP_TRY(hipHostMalloc((void**)&g_red.partial, sizeof(double) * kMaxRedVals * kMaxRedBlocks, hipHostMallocDefault));
+  for (unsigned r = 0; r < nv; ++r) iqsi::mark_pending(g_red.partial + r * kMaxRedBlocks, nblocks);
   *out = &g_red;
   return IQSH_OK;
 }
@@ -960,17 +959,27 @@ __global__ __launch_bounds__(kBlock) void k_adj_1q(typename Vec<T>::t* __restric
     lam[i0] = cmad2(uinv.m00, l0, uinv.m01, l1);
     lam[i1] = cmad2(uinv.m10, l0, uinv.m11, l1);
   }
-  block_sum_store<1>(v, partial);
+  if (with_grad) block_sum_store<1>(v, partial);  // nobody waits for the sum otherwise
 }
 
-// Finish a reduction: second stage + copy nv doubles to host (synchronizes the stream).
-int red_finish(RedWork* w, unsigned nblocks, unsigned nv, int is_max, double* out)
+// Finish a reduction: out[r] = sum (or max) of the nblocks partial results of value r, in the
+// order of k_red_final.  Read-only reductions wait for the partial results themselves;
+// those that also write a register wait for the stream.
+int red_finish(RedWork* w, unsigned nblocks, unsigned nv, int is_max, double* out, bool read_only = true)
 {
-  k_red_final<<<1, kBlock, 0, g_stream>>>(w->partial, nblocks, nv, is_max, w->result);
-  CHECK_LAUNCH();
-  HIP_TRY(hipMemcpyAsync(w->host, w->result, sizeof(double) * nv, hipMemcpyDeviceToHost, g_stream));
-  HIP_TRY(hipStreamSynchronize(g_stream));
-  for (unsigned r = 0; r < nv; ++r) out[r] = w->host[r];
+  if (!read_only) HIP_TRY(hipStreamSynchronize(g_stream));
+  for (unsigned r = 0; r < nv; ++r) {
+    const double* p = w->partial + r * kMaxRedBlocks;
+    if (int rc = iqsi::await_results(p, nblocks)) return rc;
+    double s[kBlock];
+    for (unsigned t = 0; t < (unsigned)kBlock; ++t) {
+      s[t] = is_max ? -1.0 : 0.0;
+      for (unsigned b = t; b < nblocks; b += kBlock) s[t] = is_max ? std::fmax(s[t], p[b]) : s[t] + p[b];
+    }
+    for (unsigned h = kBlock / 2; h > 0; h >>= 1)
+      for (unsigned t = 0; t < h; ++t) s[t] = is_max ? std::fmax(s[t], s[t + h]) : s[t] + s[t + h];
+    out[r] = s[0];
+  }
   return IQSH_OK;
 }
 
@@ -1031,6 +1040,23 @@ int device_cus()
   if (hipGetDevice(&dev) != hipSuccess) return 0;
   if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
   return cus;
+}
+int await_results(const double* p, uint64_t count)
+{
+  using clock = std::chrono::steady_clock;
+  const auto* q = reinterpret_cast<const uint64_t*>(p);
+  const auto end = clock::now() + std::chrono::microseconds(100);
+  uint64_t i = 0;
+  for (unsigned polls = 1; i < count; ++polls) {
+    while (i < count && __atomic_load_n(q + i, __ATOMIC_ACQUIRE) != kPending) ++i;
+    if (i == count) return IQSH_OK;
+    if (polls % 32 == 0 && clock::now() > end) break;
+  }
+  IQSI_TRY(hipStreamSynchronize(g_stream));
+  for (; i < count; ++i)
+    if (__atomic_load_n(q + i, __ATOMIC_ACQUIRE) == kPending)
+      return fail(IQSH_ERR_HIP, "a reduction kernel left partial result %llu unwritten", (unsigned long long)i);
+  return IQSH_OK;
 }
 int build_cut_spec(iqsh_handle h, unsigned ne, const unsigned* u, const unsigned* v, const double* w, double gamma,
                    iqsk::CutSpec* cs)
@@ -1707,11 +1733,11 @@ template <typename T>
 int do_norm_sub(iqsh_handle h, int K, unsigned pos, double* out)
 {
   RedWork* w;
-  std::lock_guard<std::mutex> red_lk(g_red_mu);  // held until red_finish has synchronized
-  if (int rc = red_ws(&w)) return rc;
+  std::lock_guard<std::mutex> red_lk(g_red_mu);  // held until red_finish has the result
   using V = typename Vec<T>::t;
   if (K == 0) {
     const unsigned g = red_grid(h->size());
+    if (int rc = red_ws(&w, g, 1)) return rc;
     k_red_norm<T, 0><<<g, kBlock, 0, g_stream>>>((const V*)h->d, h->size(), Ins<0>{}, 0, w->partial);
     CHECK_LAUNCH();
     return red_finish(w, g, 1, 0, out);
@@ -1719,6 +1745,7 @@ int do_norm_sub(iqsh_handle h, int K, unsigned pos, double* out)
   Ins<1> ins;
   ins.p[0] = pos;
   const unsigned g = red_grid(h->size() / 2);
+  if (int rc = red_ws(&w, g, 1)) return rc;
   k_red_norm<T, 1><<<g, kBlock, 0, g_stream>>>((const V*)h->d, h->size() / 2, ins, uint64_t(1) << pos, w->partial);
   CHECK_LAUNCH();
   return red_finish(w, g, 1, 0, out);
@@ -1728,10 +1755,10 @@ template <typename T>
 int do_pauli(iqsh_handle h, uint64_t x, uint64_t z, unsigned ny, double* out2)
 {
   RedWork* w;
-  std::lock_guard<std::mutex> red_lk(g_red_mu);  // held until red_finish has synchronized
-  if (int rc = red_ws(&w)) return rc;
+  std::lock_guard<std::mutex> red_lk(g_red_mu);  // held until red_finish has the result
   using V = typename Vec<T>::t;
   const unsigned g = red_grid((x >> 6) ? h->size() / 2 : h->size());
+  if (int rc = red_ws(&w, g, 2)) return rc;
   launch_pauli<T>(g, (const V*)h->d, h->size(), x, z, ny, w->partial);
   CHECK_LAUNCH();
   return red_finish(w, g, 2, 0, out2);
@@ -1741,10 +1768,10 @@ template <typename T>
 int do_two(iqsh_handle h, iqsh_handle x, int kind, double sr, double si, double* out)
 {
   RedWork* w;
-  std::lock_guard<std::mutex> red_lk(g_red_mu);  // held until red_finish has synchronized
-  if (int rc = red_ws(&w)) return rc;
+  std::lock_guard<std::mutex> red_lk(g_red_mu);  // held until red_finish has the result
   using V = typename Vec<T>::t;
   const unsigned g = red_grid(h->size());
+  if (int rc = red_ws(&w, g, 2)) return rc;
   if (kind == 0) {
     k_red_overlap<T><<<g, kBlock, 0, g_stream>>>((const V*)h->d, (const V*)x->d, h->size(), w->partial);
     CHECK_LAUNCH();
@@ -1773,11 +1800,11 @@ template <typename T>
 int do_maxnorm_half(iqsh_handle h, unsigned pos, int value, double* out)
 {
   RedWork* w;
-  std::lock_guard<std::mutex> red_lk(g_red_mu);  // held until red_finish has synchronized
-  if (int rc = red_ws(&w)) return rc;
+  std::lock_guard<std::mutex> red_lk(g_red_mu);  // held until red_finish has the result
   Ins<1> ins;
   ins.p[0] = pos;
   const unsigned g = red_grid(h->size() / 2);
+  if (int rc = red_ws(&w, g, 1)) return rc;
   k_red_maxnorm<T><<<g, kBlock, 0, g_stream>>>((const typename Vec<T>::t*)h->d, h->size() / 2, ins,
                                                value ? (uint64_t(1) << pos) : 0, w->partial);
   CHECK_LAUNCH();
@@ -1930,9 +1957,9 @@ template <typename T>
 int do_qaoa_cost(iqsh_handle h, iqsh_handle lam, const CutSpec& cs, double* out)
 {
   RedWork* w;
-  std::lock_guard<std::mutex> red_lk(g_red_mu);  // held until red_finish has synchronized
-  if (int rc = red_ws(&w)) return rc;
+  std::lock_guard<std::mutex> red_lk(g_red_mu);  // held until red_finish has the result
   const unsigned g = red_grid(h->size());
+  if (int rc = red_ws(&w, g, 1)) return rc;
   if (!cs.weighted && h->size() >= kDiagRow)
     k_qaoa_diag_rows<T, 1><<<g, kBlock, 0, g_stream>>>((typename Vec<T>::t*)h->d,
                                                        lam ? (typename Vec<T>::t*)lam->d : nullptr, h->size(), cs,
@@ -1942,21 +1969,21 @@ int do_qaoa_cost(iqsh_handle h, iqsh_handle lam, const CutSpec& cs, double* out)
                                                lam ? (typename Vec<T>::t*)lam->d : nullptr, h->size(), cs, lam != nullptr,
                                                w->partial);
   CHECK_LAUNCH();
-  return red_finish(w, g, 1, 0, out);
+  return red_finish(w, g, 1, 0, out, lam == nullptr);
 }
 
 template <typename T>
 int do_qaoa_phase_adj(iqsh_handle h, iqsh_handle lam, const CutSpec& cs, double* out)
 {
   RedWork* w;
-  std::lock_guard<std::mutex> red_lk(g_red_mu);  // held until red_finish has synchronized
-  if (int rc = red_ws(&w)) return rc;
+  std::lock_guard<std::mutex> red_lk(g_red_mu);  // held until red_finish has the result
   const unsigned g = red_grid(h->size());
+  if (int rc = red_ws(&w, g, 1)) return rc;
   k_qaoa_phase_adj<T><<<g, kBlock, 0, g_stream>>>((typename Vec<T>::t*)h->d, (typename Vec<T>::t*)lam->d, h->size(), cs,
                                                   w->partial);
   CHECK_LAUNCH();
   double s;
-  if (int rc = red_finish(w, g, 1, 0, &s)) return rc;
+  if (int rc = red_finish(w, g, 1, 0, &s, false)) return rc;
   *out = 2.0 * s;
   return IQSH_OK;
 }
@@ -1965,12 +1992,12 @@ template <typename T>
 int do_maxcut_fill(iqsh_handle h, const CutSpec& cs, int accumulate, double* out)
 {
   RedWork* w;
-  std::lock_guard<std::mutex> red_lk(g_red_mu);  // held until red_finish has synchronized
-  if (int rc = red_ws(&w)) return rc;
+  std::lock_guard<std::mutex> red_lk(g_red_mu);  // held until red_finish has the result
   const unsigned g = red_grid(h->size());
+  if (int rc = red_ws(&w, g, 1)) return rc;
   k_maxcut_fill<T><<<g, kBlock, 0, g_stream>>>((typename Vec<T>::t*)h->d, h->size(), cs, accumulate, w->partial);
   CHECK_LAUNCH();
-  return red_finish(w, g, 1, 1, out);
+  return red_finish(w, g, 1, 1, out, false);
 }
 
 template <typename T>
@@ -1987,9 +2014,9 @@ template <typename T>
 int do_qaoa_diag_expect(iqsh_handle psi, iqsh_handle diag, int squared, double* out)
 {
   RedWork* w;
-  std::lock_guard<std::mutex> red_lk(g_red_mu);  // held until red_finish has synchronized
-  if (int rc = red_ws(&w)) return rc;
+  std::lock_guard<std::mutex> red_lk(g_red_mu);  // held until red_finish has the result
   const unsigned g = red_grid(psi->size());
+  if (int rc = red_ws(&w, g, 1)) return rc;
   k_qaoa_diag_expect<T><<<g, kBlock, 0, g_stream>>>((const typename Vec<T>::t*)psi->d,
                                                     (const typename Vec<T>::t*)diag->d, psi->size(), squared, w->partial);
   CHECK_LAUNCH();
@@ -2000,17 +2027,17 @@ template <typename T>
 int do_adj_1q(iqsh_handle h, iqsh_handle lam, unsigned pos, const double* uinv, const double* G, double* out)
 {
   RedWork* w;
-  std::lock_guard<std::mutex> red_lk(g_red_mu);  // held until red_finish has synchronized
-  if (int rc = red_ws(&w)) return rc;
+  std::lock_guard<std::mutex> red_lk(g_red_mu);  // held until red_finish has the result
   const uint64_t items = h->size() / 2;
   const unsigned g = red_grid(items);
+  if (int rc = red_ws(&w, g, 1)) return rc;
   const double zero[8] = {0, 0, 0, 0, 0, 0, 0, 0};
   k_adj_1q<T><<<g, kBlock, 0, g_stream>>>((typename Vec<T>::t*)h->d, (typename Vec<T>::t*)lam->d, items, pos,
                                           mat2<T>(uinv), mat2<double>(G ? G : zero), G != nullptr, w->partial);
   CHECK_LAUNCH();
   if (!G) return IQSH_OK;
   double s;
-  if (int rc = red_finish(w, g, 1, 0, &s)) return rc;
+  if (int rc = red_finish(w, g, 1, 0, &s, false)) return rc;
   *out = 2.0 * s;
   return IQSH_OK;
 }

@@ -5,15 +5,15 @@
 // 4x4 matrix per state (noise gates, 1- and 2-qubit channel branches), and reductions with
 // one result per state.
 //
-// Reductions: a workgroup reduces one chunk of C = min(2^state_qubits, 2^14) contiguous
-// amplitudes (never straddling two states) in FP64 with a fixed lane/wave order; the
-// per-chunk partials are summed per state on the host, in chunk order, so every result is
-// bitwise reproducible.
+// Reductions: a workgroup reduces one chunk of at most 2^14 contiguous amplitudes (never
+// straddling two states) in FP64 with a fixed lane/wave order; the per-chunk partials are
+// summed per state on the host, in chunk order, so every result is bitwise reproducible.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
 #include <cmath>
 #include <mutex>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/iqs_hip.h"
@@ -25,18 +25,28 @@ using namespace iqsk;
 namespace {
 
 constexpr int kPB = 256;              // threads per workgroup
-constexpr unsigned kChunkLog = 14;    // at most 2^14 amplitudes per reduction workgroup
+constexpr unsigned kChunkLog = 14;    // at most 2^14 amplitudes per reduction workgroup, and down to
+constexpr unsigned kChunkLogMin = 11; // 2^11 while there are fewer than kFillGrid workgroups
+constexpr uint64_t kFillGrid = 1024;
 constexpr uint64_t kMaxGrid = 1u << 20;
 constexpr int kRU = 8;                // loads in flight per thread in the chunk reductions
 
-// Device buffers shared by the pool entry points (guarded; grown on demand).
+// Per-state matrices on their way to the device: kSlots pinned slots and their device copies,
+// each reused when the launch that reads it has finished; grown on demand, together.
+constexpr int kSlots = 4;
 struct PoolWork {
-  void* mats = nullptr;
-  size_t mats_bytes = 0;
-  double* part = nullptr;
-  size_t part_count = 0;
+  char *mats_host = nullptr, *mats = nullptr;
+  size_t slot_bytes = 0;
+  hipEvent_t done[kSlots];
+  bool events = false, used[kSlots] = {};
+  int next = 0;
+  double* pinned = nullptr;  // kHostParts partial sums written by the kernels
+  double* part = nullptr;    // more than that: on the device
+  size_t part_bytes = 0;
   std::vector<double> host;
 };
+// Chunk sums up to this many go straight to pinned host memory (512 KiB).
+constexpr uint64_t kHostParts = 65536;
 PoolWork g_pw;
 std::mutex g_pm;
 
@@ -50,6 +60,73 @@ int grow(void** p, size_t* have, size_t need)
   *have = 0;
   if (hipMalloc(p, need) != hipSuccess) return iqsi::fail(IQSH_ERR_ALLOC, "pool work buffer of %zu bytes", need);
   *have = need;
+  return IQSH_OK;
+}
+
+// A free slot of at least `bytes` for matrices.
+int mats_slot(size_t bytes, int* slot)
+{
+  if (!g_pw.events) {
+    for (int i = 0; i < kSlots; ++i) IQSI_TRY(hipEventCreateWithFlags(&g_pw.done[i], hipEventDisableTiming));
+    g_pw.events = true;
+  }
+  if (g_pw.slot_bytes < bytes) {
+    const size_t want = std::max<size_t>(4096, (bytes + 255) & ~size_t(255));
+    IQSI_TRY(hipStreamSynchronize(iqsi::stream()));
+    g_pw.slot_bytes = 0;
+    if (g_pw.mats_host) IQSI_TRY(hipHostFree(g_pw.mats_host));
+    g_pw.mats_host = nullptr;
+    if (g_pw.mats) IQSI_TRY(hipFree(g_pw.mats));
+    g_pw.mats = nullptr;
+    if (hipHostMalloc((void**)&g_pw.mats_host, want * kSlots, hipHostMallocDefault) != hipSuccess ||
+        hipMalloc((void**)&g_pw.mats, want * kSlots) != hipSuccess)
+      return iqsi::fail(IQSH_ERR_ALLOC, "pool matrices of %zu bytes", bytes);
+    g_pw.slot_bytes = want;
+    std::fill(g_pw.used, g_pw.used + kSlots, false);
+  }
+  *slot = g_pw.next;
+  g_pw.next = (g_pw.next + 1) % kSlots;
+  if (g_pw.used[*slot]) IQSI_TRY(hipEventSynchronize(g_pw.done[*slot]));
+  return IQSH_OK;
+}
+
+// Where a kernel finds the matrix of a state: in device memory, or in its own arguments for
+// pools whose matrices fit them (no copy at all: a noise gate on 32 states of 16 qubits 24 ->
+// 8 us, against 24 -> 14 with an asynchronous copy).
+constexpr size_t kArgBytes = 2048;
+template <typename MT>
+struct MatsAt {
+  const MT* m;
+  __device__ __forceinline__ const MT& operator[](uint64_t s) const { return m[s]; }
+};
+template <typename MT>
+struct MatsArg {
+  MT m[kArgBytes / sizeof(MT)];
+  __device__ __forceinline__ const MT& operator[](uint64_t s) const { return m[s]; }
+};
+
+// Calls launch(source) with the matrices of `nstates` states, each converted by fill(s, &m).
+template <typename MT, typename Fill, typename Launch>
+int with_mats(uint64_t nstates, Fill fill, Launch launch)
+{
+  const size_t bytes = sizeof(MT) * nstates;
+  if (bytes <= kArgBytes) {
+    MatsArg<MT> a;
+    for (uint64_t s = 0; s < nstates; ++s) fill(s, &a.m[s]);
+    launch(a);
+    IQSI_TRY(hipGetLastError());
+    return IQSH_OK;
+  }
+  int slot;
+  if (int rc = mats_slot(bytes, &slot)) return rc;
+  MT* host = (MT*)(g_pw.mats_host + slot * g_pw.slot_bytes);
+  for (uint64_t s = 0; s < nstates; ++s) fill(s, &host[s]);
+  MT* dev = (MT*)(g_pw.mats + slot * g_pw.slot_bytes);
+  IQSI_TRY(hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, iqsi::stream()));
+  launch(MatsAt<MT>{dev});
+  IQSI_TRY(hipGetLastError());
+  IQSI_TRY(hipEventRecord(g_pw.done[slot], iqsi::stream()));
+  g_pw.used[slot] = true;
   return IQSH_OK;
 }
 
@@ -103,9 +180,9 @@ __global__ __launch_bounds__(kPB) void k_pool_init(typename Vec<T>::t* __restric
 }
 
 // (psi_{b}, psi_{b | 2^pos}) <- M_s (psi_b, psi_{b | 2^pos}) with s = b >> sbits.
-template <typename T>
+template <typename T, typename Mats>
 __global__ __launch_bounds__(kPB) void k_pool_1q(typename Vec<T>::t* __restrict__ st, uint64_t items, unsigned pos,
-                                                 unsigned sbits, const Mat2<T>* __restrict__ mats, uint64_t nstates)
+                                                 unsigned sbits, Mats mats, uint64_t nstates)
 {
   using V = typename Vec<T>::t;
   const uint64_t hb = uint64_t(1) << pos;
@@ -133,9 +210,9 @@ __device__ __forceinline__ uint64_t pool_tile() {
   return (G & 7) ? b : xcd_block(b, G);
 }
 
-template <typename T, bool NT, int TB = kTB, int TP = kTP>
+template <typename T, bool NT, int TB, int TP, typename Mats>
 __global__ __launch_bounds__(TB) void k_pool_1q_t(typename Vec<T>::t* __restrict__ st, unsigned pos, unsigned sbits,
-                                                  const Mat2<T>* __restrict__ mats, uint64_t nstates)
+                                                  Mats mats, uint64_t nstates)
 {
   using V = typename Vec<T>::t;
   const uint64_t hb = uint64_t(1) << pos, k0 = pool_tile() * (TB * TP) + threadIdx.x;
@@ -168,10 +245,9 @@ __global__ __launch_bounds__(TB) void k_pool_1q_t(typename Vec<T>::t* __restrict
 // written.
 constexpr int kLB = 256, kLP = 2;
 constexpr unsigned kLaneMinBits = 9;  // 2^9 = kLB * kLP
-template <typename T>
+template <typename T, bool NT, typename Mats>
 __global__ __launch_bounds__(kLB) void k_pool_1q_lane(typename Vec<T>::t* __restrict__ st, unsigned pos,
-                                                      unsigned sbits, const Mat2<T>* __restrict__ mats,
-                                                      uint64_t nstates)
+                                                      unsigned sbits, Mats mats, uint64_t nstates)
 {
   using V = typename Vec<T>::t;
   const uint64_t t0 = pool_tile() * (kLB * kLP), s = t0 >> sbits;
@@ -182,13 +258,13 @@ __global__ __launch_bounds__(kLB) void k_pool_1q_lane(typename Vec<T>::t* __rest
   const bool up = (threadIdx.x >> pos) & 1;  // this amplitude's bit pos
   V a[kLP];
 #pragma unroll
-  for (int j = 0; j < kLP; ++j) a[j] = ldg(&st[i0 + (uint64_t)j * kLB]);
+  for (int j = 0; j < kLP; ++j) a[j] = ldx<NT>(&st[i0 + (uint64_t)j * kLB]);
 #pragma unroll
   for (int j = 0; j < kLP; ++j) {
     V b;  // the partner amplitude
     b.x = __shfl_xor(a[j].x, ml);
     b.y = __shfl_xor(a[j].y, ml);
-    stg(up ? cmad2(m.m10, b, m.m11, a[j]) : cmad2(m.m00, a[j], m.m01, b), &st[i0 + (uint64_t)j * kLB]);
+    stx<NT>(up ? cmad2(m.m10, b, m.m11, a[j]) : cmad2(m.m00, a[j], m.m01, b), &st[i0 + (uint64_t)j * kLB]);
   }
 }
 
@@ -196,10 +272,9 @@ __global__ __launch_bounds__(kLB) void k_pool_1q_lane(typename Vec<T>::t* __rest
 // a lane holds the amplitude whose row is r = 2 b(ph) + b(pl) and receives rows r ^ 1,
 // r ^ 2, r ^ 3 from lanes ^ 2^pl, ^ 2^ph, ^ both; its output is row r of the state's
 // matrix, the coefficients m[r][r ^ k] selected per lane from the uniform matrix.
-template <typename T>
+template <typename T, bool NT, typename Mats>
 __global__ __launch_bounds__(kLB) void k_pool_2q_lane(typename Vec<T>::t* __restrict__ st, unsigned ph, unsigned pl,
-                                                      unsigned sbits, const Mat4<T>* __restrict__ mats,
-                                                      uint64_t nstates)
+                                                      unsigned sbits, Mats mats, uint64_t nstates)
 {
   using V = typename Vec<T>::t;
   const uint64_t t0 = pool_tile() * (kLB * kLP), s = t0 >> sbits;
@@ -217,7 +292,7 @@ __global__ __launch_bounds__(kLB) void k_pool_2q_lane(typename Vec<T>::t* __rest
   const uint64_t i0 = t0 + threadIdx.x;
   V a[kLP];
 #pragma unroll
-  for (int j = 0; j < kLP; ++j) a[j] = ldg(&st[i0 + (uint64_t)j * kLB]);
+  for (int j = 0; j < kLP; ++j) a[j] = ldx<NT>(&st[i0 + (uint64_t)j * kLB]);
 #pragma unroll
   for (int j = 0; j < kLP; ++j) {
     V xl, xh, xb;
@@ -231,14 +306,13 @@ __global__ __launch_bounds__(kLB) void k_pool_2q_lane(typename Vec<T>::t* __rest
     const V u = cmad2(c[2], xh, c[3], xb);
     r.x += u.x;
     r.y += u.y;
-    stg(r, &st[i0 + (uint64_t)j * kLB]);
+    stx<NT>(r, &st[i0 + (uint64_t)j * kLB]);
   }
 }
 
-template <typename T, bool NT, int TB = kTB>
+template <typename T, bool NT, int TB, typename Mats>
 __global__ __launch_bounds__(TB) void k_pool_2q_t(typename Vec<T>::t* __restrict__ st, unsigned lo, unsigned hi,
-                                                  uint64_t dh, uint64_t dl, unsigned sbits,
-                                                  const Mat4<T>* __restrict__ mats, uint64_t nstates)
+                                                  uint64_t dh, uint64_t dl, unsigned sbits, Mats mats, uint64_t nstates)
 {
   using V = typename Vec<T>::t;
   const uint64_t k0 = pool_tile() * (TB * kTP2) + threadIdx.x;
@@ -279,10 +353,10 @@ dim3 tile_grid(uint64_t tiles)
 
 // Dense 4x4 per state on (ph, pl), rows 2 b(ph) + b(pl): with lo < hi the two positions in
 // ascending order, item k enumerates the indices with both bits clear; s = index >> sbits.
-template <typename T>
+template <typename T, typename Mats>
 __global__ __launch_bounds__(kPB) void k_pool_2q(typename Vec<T>::t* __restrict__ st, uint64_t items, unsigned lo,
-                                                 unsigned hi, uint64_t dh, uint64_t dl, unsigned sbits,
-                                                 const Mat4<T>* __restrict__ mats, uint64_t nstates)
+                                                 unsigned hi, uint64_t dh, uint64_t dl, unsigned sbits, Mats mats,
+                                                 uint64_t nstates)
 {
   using V = typename Vec<T>::t;
   for (uint64_t k = (uint64_t)blockIdx.x * kPB + threadIdx.x; k < items; k += (uint64_t)gridDim.x * kPB) {
@@ -318,7 +392,21 @@ __global__ __launch_bounds__(kPB) void k_pool_red(const typename Vec<T>::t* __re
     else if (KIND == 1) v[0] += ((i >> arg) & 1) ? p : 0.0;
     else v[0] += (__popcll(i & arg) & 1) ? -p : p;
   };
-  if (C >= kRU * kPB) {
+  if (KIND == 1 && arg >= pool_line_bits(sizeof(typename Vec<T>::t)) && ((uint64_t(1) << arg) >= C || C >= 2 * kRU * kPB)) {
+    // Only the lines with the bit set: half of the chunk, or all or nothing of it.
+    const bool inside = (uint64_t(1) << arg) < C;
+    const uint64_t items = inside ? C / 2 : (((base >> arg) & 1) ? C : 0);
+    auto at = [&](uint64_t j) { return base + (inside ? ins0(j, (unsigned)arg) | (uint64_t(1) << arg) : j); };
+    uint64_t j = threadIdx.x;
+    for (; j + (kRU - 1) * kPB < items; j += kRU * kPB) {
+      typename Vec<T>::t a[kRU];
+#pragma unroll
+      for (int u = 0; u < kRU; ++u) a[u] = ldg(&st[at(j + u * kPB)]);
+#pragma unroll
+      for (int u = 0; u < kRU; ++u) v[0] += nrm2(a[u]);
+    }
+    for (; j < items; j += kPB) v[0] += nrm2(ldg(&st[at(j)]));
+  } else if (C >= kRU * kPB) {
     // C is a power of two: whole batches of kRU loads per thread, in flight together
     for (uint64_t j = threadIdx.x; j < C; j += kRU * kPB) {
       typename Vec<T>::t a[kRU];
@@ -389,105 +477,115 @@ int do_init(iqsh_handle h, unsigned sbits, int style, uint64_t index, uint64_t n
   return IQSH_OK;
 }
 
+// Cache policy by the pool's size (iqsi::cache_set): f(std::true_type) for non-temporal accesses.
+template <typename F>
+void by_cache_policy(iqsh_handle h, F f)
+{
+  if (iqsi::cache_set(h->size() * h->esz())) f(std::false_type{});
+  else f(std::true_type{});
+}
+
 template <typename T>
 int do_1q_each(iqsh_handle h, unsigned sbits, unsigned pos, const double* mats, uint64_t nstates)
 {
-  std::vector<Mat2<T>> m(nstates);
-  for (uint64_t s = 0; s < nstates; ++s) {
-    const double* p = mats + 8 * s;
-    m[s] = Mat2<T>{{(T)p[0], (T)p[1]}, {(T)p[2], (T)p[3]}, {(T)p[4], (T)p[5]}, {(T)p[6], (T)p[7]}};
-  }
-  const size_t bytes = sizeof(Mat2<T>) * nstates;
-  if (int rc = grow(&g_pw.mats, &g_pw.mats_bytes, bytes)) return rc;
-  // Earlier launches may still read the matrix buffer: wait for them before refilling it.
-  IQSI_TRY(hipStreamSynchronize(iqsi::stream()));
-  IQSI_TRY(hipMemcpy(g_pw.mats, m.data(), bytes, hipMemcpyHostToDevice));
-  const uint64_t items = h->size() >> 1;
   using V = typename Vec<T>::t;
-  if (pos < pool_line_bits(sizeof(V)) && sbits >= kLaneMinBits) {
-    k_pool_1q_lane<T><<<tile_grid(h->size() / (kLB * kLP)), kLB, 0, iqsi::stream()>>>(
-        (V*)h->d, pos, sbits, (const Mat2<T>*)g_pw.mats, nstates);
-  } else if (items % (kTB * kTP) == 0) {
-    // items is a power of two: a whole number of tiles, 8 or more from 2^12 amplitudes up
-    const dim3 g = tile_grid(items / (kTB * kTP));
-    // complex64 from the line width up: 256 x 1 tiles (8 x 28 qubits: position 5 6.25 ->
-    // 6.47 TB/s, 13 6.43 -> 6.54, top equal)
-    if (pos >= pool_line_bits(sizeof(V)) && sizeof(T) == 4)
-      k_pool_1q_t<T, true, 2 * kTB, 1><<<tile_grid(items / (2 * kTB)), 2 * kTB, 0, iqsi::stream()>>>(
-          (V*)h->d, pos, sbits, (const Mat2<T>*)g_pw.mats, nstates);
-    else if (pos >= pool_line_bits(sizeof(V)))
-      k_pool_1q_t<T, true><<<g, kTB, 0, iqsi::stream()>>>((V*)h->d, pos, sbits, (const Mat2<T>*)g_pw.mats, nstates);
-    else
-      k_pool_1q_t<T, false><<<g, kTB, 0, iqsi::stream()>>>((V*)h->d, pos, sbits, (const Mat2<T>*)g_pw.mats, nstates);
-  } else {
-    k_pool_1q<T><<<grid_of(items), kPB, 0, iqsi::stream()>>>((V*)h->d, items, pos, sbits, (const Mat2<T>*)g_pw.mats,
-                                                              nstates);
-  }
-  IQSI_TRY(hipGetLastError());
-  return IQSH_OK;
+  const uint64_t items = h->size() >> 1;
+  V* st = (V*)h->d;
+  hipStream_t q = iqsi::stream();
+  auto fill = [&](uint64_t s, Mat2<T>* m) {
+    const double* p = mats + 8 * s;
+    *m = Mat2<T>{{(T)p[0], (T)p[1]}, {(T)p[2], (T)p[3]}, {(T)p[4], (T)p[5]}, {(T)p[6], (T)p[7]}};
+  };
+  return with_mats<Mat2<T>>(nstates, fill, [&](auto src) {
+    using S = decltype(src);
+    by_cache_policy(h, [&](auto policy) {
+      constexpr bool NT = decltype(policy)::value;
+      if (pos < pool_line_bits(sizeof(V)) && sbits >= kLaneMinBits) {
+        k_pool_1q_lane<T, NT, S><<<tile_grid(h->size() / (kLB * kLP)), kLB, 0, q>>>(st, pos, sbits, src, nstates);
+      } else if (items % (kTB * kTP) == 0) {
+        // items is a power of two: a whole number of tiles, 8 or more from 2^12 amplitudes up
+        const dim3 g = tile_grid(items / (kTB * kTP));
+        // complex64 from the line width up: 256 x 1 tiles (8 x 28 qubits: position 5 6.25 ->
+        // 6.47 TB/s, 13 6.43 -> 6.54, top equal)
+        if (pos < pool_line_bits(sizeof(V)))
+          k_pool_1q_t<T, false, kTB, kTP, S><<<g, kTB, 0, q>>>(st, pos, sbits, src, nstates);
+        else if (sizeof(T) == 4)
+          k_pool_1q_t<T, NT, 2 * kTB, 1, S><<<tile_grid(items / (2 * kTB)), 2 * kTB, 0, q>>>(st, pos, sbits, src, nstates);
+        else
+          k_pool_1q_t<T, NT, kTB, kTP, S><<<g, kTB, 0, q>>>(st, pos, sbits, src, nstates);
+      } else {
+        k_pool_1q<T, S><<<grid_of(items), kPB, 0, q>>>(st, items, pos, sbits, src, nstates);
+      }
+    });
+  });
 }
 
 template <typename T>
 int do_2q_each(iqsh_handle h, unsigned sbits, unsigned ph, unsigned pl, const double* mats, uint64_t nstates)
 {
-  std::vector<Mat4<T>> m(nstates);
-  for (uint64_t s = 0; s < nstates; ++s)
-    for (int e = 0; e < 16; ++e) m[s].m[e] = Cx<T>{(T)mats[32 * s + 2 * e], (T)mats[32 * s + 2 * e + 1]};
-  const size_t bytes = sizeof(Mat4<T>) * nstates;
-  if (int rc = grow(&g_pw.mats, &g_pw.mats_bytes, bytes)) return rc;
-  IQSI_TRY(hipStreamSynchronize(iqsi::stream()));
-  IQSI_TRY(hipMemcpy(g_pw.mats, m.data(), bytes, hipMemcpyHostToDevice));
-  const uint64_t items = h->size() >> 2;
   using V = typename Vec<T>::t;
+  const uint64_t items = h->size() >> 2, dh = uint64_t(1) << ph, dl = uint64_t(1) << pl;
   const unsigned lo = std::min(ph, pl), hi = std::max(ph, pl);
-  if (hi < pool_line_bits(sizeof(V)) && sbits >= kLaneMinBits) {
-    k_pool_2q_lane<T><<<tile_grid(h->size() / (kLB * kLP)), kLB, 0, iqsi::stream()>>>(
-        (V*)h->d, ph, pl, sbits, (const Mat4<T>*)g_pw.mats, nstates);
-  } else if (items % (kTB * kTP2) == 0) {
-    const dim3 g = tile_grid(items / (kTB * kTP2));
-    // complex64 from the line width up: 256-thread tiles (8 x 28 qubits: (27,26) 4.88 ->
-    // 5.55 TB/s, (5,20) 5.40 -> 5.52; complex128 within 1% either way)
-    if (lo >= pool_line_bits(sizeof(V)) && sizeof(T) == 4 && items % (2 * kTB * kTP2) == 0)
-      k_pool_2q_t<T, true, 2 * kTB><<<tile_grid(items / (2 * kTB * kTP2)), 2 * kTB, 0, iqsi::stream()>>>(
-          (V*)h->d, lo, hi, uint64_t(1) << ph, uint64_t(1) << pl, sbits, (const Mat4<T>*)g_pw.mats, nstates);
-    else if (lo >= pool_line_bits(sizeof(V)))
-      k_pool_2q_t<T, true><<<g, kTB, 0, iqsi::stream()>>>((V*)h->d, lo, hi, uint64_t(1) << ph, uint64_t(1) << pl, sbits,
-                                                          (const Mat4<T>*)g_pw.mats, nstates);
-    else
-      k_pool_2q_t<T, false><<<g, kTB, 0, iqsi::stream()>>>((V*)h->d, lo, hi, uint64_t(1) << ph, uint64_t(1) << pl,
-                                                           sbits, (const Mat4<T>*)g_pw.mats, nstates);
-  } else {
-    k_pool_2q<T><<<grid_of(items), kPB, 0, iqsi::stream()>>>((V*)h->d, items, lo, hi, uint64_t(1) << ph,
-                                                              uint64_t(1) << pl, sbits, (const Mat4<T>*)g_pw.mats,
-                                                              nstates);
-  }
-  IQSI_TRY(hipGetLastError());
-  return IQSH_OK;
+  V* st = (V*)h->d;
+  hipStream_t q = iqsi::stream();
+  auto fill = [&](uint64_t s, Mat4<T>* m) {
+    for (int e = 0; e < 16; ++e) m->m[e] = Cx<T>{(T)mats[32 * s + 2 * e], (T)mats[32 * s + 2 * e + 1]};
+  };
+  return with_mats<Mat4<T>>(nstates, fill, [&](auto src) {
+    using S = decltype(src);
+    by_cache_policy(h, [&](auto policy) {
+      constexpr bool NT = decltype(policy)::value;
+      if (hi < pool_line_bits(sizeof(V)) && sbits >= kLaneMinBits) {
+        k_pool_2q_lane<T, NT, S><<<tile_grid(h->size() / (kLB * kLP)), kLB, 0, q>>>(st, ph, pl, sbits, src, nstates);
+      } else if (items % (kTB * kTP2) == 0) {
+        const dim3 g = tile_grid(items / (kTB * kTP2));
+        // complex64 from the line width up: 256-thread tiles (8 x 28 qubits: (27,26) 4.88 ->
+        // 5.55 TB/s, (5,20) 5.40 -> 5.52; complex128 within 1% either way)
+        if (lo < pool_line_bits(sizeof(V)))
+          k_pool_2q_t<T, false, kTB, S><<<g, kTB, 0, q>>>(st, lo, hi, dh, dl, sbits, src, nstates);
+        else if (sizeof(T) == 4 && items % (2 * kTB * kTP2) == 0)
+          k_pool_2q_t<T, NT, 2 * kTB, S><<<tile_grid(items / (2 * kTB * kTP2)), 2 * kTB, 0, q>>>(st, lo, hi, dh, dl, sbits,
+                                                                                             src, nstates);
+        else
+          k_pool_2q_t<T, NT, kTB, S><<<g, kTB, 0, q>>>(st, lo, hi, dh, dl, sbits, src, nstates);
+      } else {
+        k_pool_2q<T, S><<<grid_of(items), kPB, 0, q>>>(st, items, lo, hi, dh, dl, sbits, src, nstates);
+      }
+    });
+  });
 }
 
 // Launch `nchunks` chunk reductions with NV values each, then sum them per state on the host.
 template <typename Launch>
 int reduce_per_state(unsigned sbits, uint64_t nstates, int nv, double* out, Launch launch)
 {
-  const unsigned clog = std::min(sbits, kChunkLog);
+  // 32 states of 16 qubits: 1024 workgroups of 2^11 amplitudes instead of 128 of 2^14.
+  unsigned clog = std::min(sbits, kChunkLog);
+  while (clog > kChunkLogMin && (nstates << (sbits - clog)) < kFillGrid) --clog;
   const uint64_t per_state = uint64_t(1) << (sbits - clog);
   const uint64_t nchunks = nstates * per_state;
   if (nchunks > 0x7fffffffull) return iqsi::fail(IQSH_ERR_NOTSUP, "pool reduction needs %llu workgroups", (unsigned long long)nchunks);
-  size_t have = g_pw.part_count * sizeof(double);
-  void* p = g_pw.part;
-  if (int rc = grow(&p, &have, nchunks * nv * sizeof(double))) return rc;
-  g_pw.part = (double*)p;
-  g_pw.part_count = have / sizeof(double);
-  launch((unsigned)nchunks, clog, g_pw.part);
-  IQSI_TRY(hipGetLastError());
-  g_pw.host.resize(nchunks * nv);
-  IQSI_TRY(hipMemcpyAsync(g_pw.host.data(), g_pw.part, nchunks * nv * sizeof(double), hipMemcpyDeviceToHost,
-                          iqsi::stream()));
-  IQSI_TRY(hipStreamSynchronize(iqsi::stream()));
+  const double* sums;
+  if (nchunks * nv <= kHostParts) {
+    if (!g_pw.pinned) IQSI_TRY(hipHostMalloc((void**)&g_pw.pinned, kHostParts * sizeof(double), hipHostMallocDefault));
+    iqsi::mark_pending(g_pw.pinned, nchunks * nv);
+    launch((unsigned)nchunks, clog, g_pw.pinned);
+    IQSI_TRY(hipGetLastError());
+    if (int rc = iqsi::await_results(g_pw.pinned, nchunks * nv)) return rc;
+    sums = g_pw.pinned;
+  } else {
+    if (int rc = grow((void**)&g_pw.part, &g_pw.part_bytes, nchunks * nv * sizeof(double))) return rc;
+    launch((unsigned)nchunks, clog, g_pw.part);
+    IQSI_TRY(hipGetLastError());
+    g_pw.host.resize(nchunks * nv);
+    IQSI_TRY(hipMemcpyAsync(g_pw.host.data(), g_pw.part, nchunks * nv * sizeof(double), hipMemcpyDeviceToHost, iqsi::stream()));
+    IQSI_TRY(hipStreamSynchronize(iqsi::stream()));
+    sums = g_pw.host.data();
+  }
   for (uint64_t s = 0; s < nstates; ++s)
     for (int r = 0; r < nv; ++r) {
       double acc = 0;
-      for (uint64_t c = 0; c < per_state; ++c) acc += g_pw.host[(s * per_state + c) * nv + r];
+      for (uint64_t c = 0; c < per_state; ++c) acc += sums[(s * per_state + c) * nv + r];
       out[s * nv + r] = acc;
     }
   return IQSH_OK;

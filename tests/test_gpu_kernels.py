@@ -619,3 +619,31 @@ def test_controlled_phase_with_a_position_inside_a_line(dt, n):
                 want = v[touched].astype(np.complex128) * f
                 eps = 2.0 ** -52 if dt == "c128" else 2.0 ** -23
                 assert np.abs(got[touched] - want).max() < 4 * eps * np.abs(v).max()
+
+
+@pytest.mark.parametrize("dt", ["c128", "c64"])
+@pytest.mark.parametrize("n", [1, 5, 10, 12, 20, 23])
+def test_reductions_between_unfinished_work(dt, n):
+    """Values read back right after the launch, between gates and adjoint steps that nobody waits
+    for: every read sees exactly the state before it (norms, probabilities, overlaps and maxima
+    against numpy), and two reads in a row agree bit for bit."""
+    r = np.random.default_rng(n)
+    v = r.normal(size=1 << n) + 1j * r.normal(size=1 << n)
+    v = (v / np.linalg.norm(v)).astype(np.complex128 if dt == "c128" else np.complex64)
+    a, b = StateVector(n, dt), StateVector(n, dt)
+    a.upload(v)
+    b.upload(v)
+    tol = 1e-12 if dt == "c128" else 1e-5
+    x = np.array([[0, 1], [1, 0]])
+    for k in range(8):
+        a.apply_1q(k % n, x)  # a pure move
+        a.adjoint_1q(b, 0, np.eye(2))  # writes both, returns nothing
+        m = np.moveaxis(v.reshape(-1, 2, 1 << (k % n)), 1, 0)
+        v = np.stack((m[1], m[0]), axis=1).reshape(-1)
+        p = np.abs(v.astype(np.complex128)) ** 2
+        got = a.prob1(n - 1)
+        assert abs(got - p[1 << (n - 1):].sum()) < tol and a.prob1(n - 1) == got
+        assert abs(a.norm2() - p.sum()) < tol
+        o = np.vdot(b.download().astype(np.complex128), v.astype(np.complex128))
+        assert abs(a.overlap(b) - o) < tol
+    assert a.maxabsdiff(a) == 0.0

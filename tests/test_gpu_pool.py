@@ -261,3 +261,47 @@ def test_per_state_kernels_every_form(dt):
     call("iqsh_pool_overlap", sv.handle, sq, ref.handle, out, ns)
     wov = [np.vdot(ref_h.astype(np.complex128), got[s]) for s in range(ns)]
     assert np.max(np.abs(np.array(out[0::2]) + 1j * np.array(out[1::2]) - wov)) < 1e-11
+
+
+@pytest.mark.parametrize("dt", ["c128", "c64"])
+@pytest.mark.parametrize("sbits,nstates", [(3, 5), (9, 3), (11, 2), (12, 7), (14, 33), (15, 3), (16, 40)])
+def test_per_state_matrices_and_probabilities_over_sizes(dt, sbits, nstates):
+    """Matrices in the kernel's arguments and in the slot ring (more of them than 2048 bytes
+    hold, several calls in a row), chunks of every size, and P(qubit) on every position, against
+    numpy on the host.  Tolerances: one 2x2 product per call (4 roundings), sums of at most 2^16
+    terms in FP64."""
+    import ctypes as C
+
+    from iqs_amd._lib import call
+    from iqs_amd.engine import StateVector
+    n = sbits + max(1, (nstates - 1).bit_length())
+    r = np.random.default_rng(sbits)
+    v = r.normal(size=1 << n) + 1j * r.normal(size=1 << n)
+    v = (v / np.linalg.norm(v)).astype(np.complex128 if dt == "c128" else np.complex64)
+    sv = StateVector(n, dt)
+    sv.upload(v)
+    want = v.astype(np.complex128).reshape(-1, 1 << sbits)
+    for call_no in range(6):
+        pos = (call_no * 5) % sbits
+        th = r.uniform(0, 6, nstates)
+        m = np.zeros((nstates, 2, 2), dtype=np.complex128)
+        m[:, 0, 0] = m[:, 1, 1] = np.cos(th)
+        m[:, 0, 1], m[:, 1, 0] = -np.sin(th), np.sin(th)
+        call("iqsh_pool_apply_1q_each", sv.handle, C.c_uint(sbits), C.c_uint(pos), C.c_void_p(m.ctypes.data), C.c_uint64(nstates))
+        w = want[:nstates].reshape(nstates, -1, 2, 1 << pos)
+        a, b = w[:, :, 0].copy(), w[:, :, 1].copy()
+        w[:, :, 0] = m[:, 0, 0, None, None] * a + m[:, 0, 1, None, None] * b
+        w[:, :, 1] = m[:, 1, 0, None, None] * a + m[:, 1, 1, None, None] * b
+    got = sv.download().reshape(-1, 1 << sbits)
+    eps = 2.0 ** -52 if dt == "c128" else 2.0 ** -23
+    assert np.abs(got - want).max() < 6 * 4 * eps * np.abs(v).max() * 2
+    assert np.array_equal(got[nstates:], v.reshape(-1, 1 << sbits)[nstates:])
+    p = np.abs(got.astype(np.complex128)) ** 2
+    out = np.zeros(nstates)
+    for pos in range(sbits):
+        call("iqsh_pool_reduce", sv.handle, C.c_uint(sbits), C.c_int(1), C.c_uint64(pos), C.c_void_p(out.ctypes.data),
+             C.c_uint64(nstates))
+        assert np.abs(out - p[:nstates].reshape(nstates, -1, 2, 1 << pos)[:, :, 1].sum(axis=(1, 2))).max() < 1e-13
+    call("iqsh_pool_reduce", sv.handle, C.c_uint(sbits), C.c_int(0), C.c_uint64(0), C.c_void_p(out.ctypes.data),
+         C.c_uint64(nstates))
+    assert np.abs(out - p[:nstates].sum(axis=1)).max() < 1e-13
