@@ -252,6 +252,18 @@ int iqsh_qaoa_layer_adjoint(iqsh_handle psi, iqsh_handle lam, unsigned ne, const
                             const double *w, double gamma, const double mixer_inv[8], const double *G,
                             double *dgamma, double *dmixer);
 
+/* A whole QAOA circuit: psi := |+>^n, then iqsh_qaoa_layer with exp(-i gammas[l] C) and the mixer
+ * RX(2 betas[l]) on every qubit, l = 0 .. layers-1.  n >= 10. */
+int iqsh_qaoa_run(iqsh_handle psi, unsigned layers, unsigned ne, const unsigned *u, const unsigned *v, const double *w,
+                  const double *gammas, const double *betas);
+/* From that circuit's final state: lam := C psi with *cost := <C>, then every backward step
+ * (iqsh_qaoa_layer_adjoint with G = X) down to |+>^n, with dgammas[l] and dbetas[l] the derivatives
+ * of *cost.  The steps follow each other on the stream; the host waits once, for all sums.
+ * n >= 10. */
+int iqsh_qaoa_gradient(iqsh_handle psi, iqsh_handle lam, unsigned layers, unsigned ne, const unsigned *u,
+                       const unsigned *v, const double *w, const double *gammas, const double *betas, double *cost,
+                       double *dgammas, double *dbetas);
+
 /* ---- batches of hardware-efficient-ansatz circuits ------------------------------------
  * No counterpart in the reference; the nearest is its pool of independent states
  * (src/mpi_env.cpp:239-404, one state per MPI rank group).  A batch holds `count`

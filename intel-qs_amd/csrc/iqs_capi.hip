@@ -1954,21 +1954,26 @@ int do_qaoa_phase(iqsh_handle h, const CutSpec& cs)
 }
 
 template <typename T>
+int launch_qaoa_cost(iqsh_handle h, iqsh_handle lam, const CutSpec& cs, unsigned g, double* partial)
+{
+  using V = typename Vec<T>::t;
+  V* lp = lam ? (V*)lam->d : nullptr;
+  if (!cs.weighted && h->size() >= kDiagRow)
+    k_qaoa_diag_rows<T, 1><<<g, kBlock, 0, g_stream>>>((V*)h->d, lp, h->size(), cs, lam != nullptr, partial);
+  else
+    k_qaoa_cost<T><<<g, kBlock, 0, g_stream>>>((const V*)h->d, lp, h->size(), cs, lam != nullptr, partial);
+  CHECK_LAUNCH();
+  return IQSH_OK;
+}
+
+template <typename T>
 int do_qaoa_cost(iqsh_handle h, iqsh_handle lam, const CutSpec& cs, double* out)
 {
   RedWork* w;
   std::lock_guard<std::mutex> red_lk(g_red_mu);  // held until red_finish has the result
   const unsigned g = red_grid(h->size());
   if (int rc = red_ws(&w, g, 1)) return rc;
-  if (!cs.weighted && h->size() >= kDiagRow)
-    k_qaoa_diag_rows<T, 1><<<g, kBlock, 0, g_stream>>>((typename Vec<T>::t*)h->d,
-                                                       lam ? (typename Vec<T>::t*)lam->d : nullptr, h->size(), cs,
-                                                       lam != nullptr, w->partial);
-  else
-    k_qaoa_cost<T><<<g, kBlock, 0, g_stream>>>((const typename Vec<T>::t*)h->d,
-                                               lam ? (typename Vec<T>::t*)lam->d : nullptr, h->size(), cs, lam != nullptr,
-                                               w->partial);
-  CHECK_LAUNCH();
+  if (int rc = launch_qaoa_cost<T>(h, lam, cs, g, w->partial)) return rc;
   return red_finish(w, g, 1, 0, out, lam == nullptr);
 }
 
@@ -2042,6 +2047,14 @@ int do_adj_1q(iqsh_handle h, iqsh_handle lam, unsigned pos, const double* uinv, 
   return IQSH_OK;
 }
 }  // namespace
+
+namespace iqsi {
+unsigned cost_blocks(iqsh_handle psi) { return red_grid(psi->size()); }
+int launch_cost(iqsh_handle psi, iqsh_handle lam, const iqsk::CutSpec& cs, double* partial)
+{
+  return DISPATCH(psi, launch_qaoa_cost)(psi, lam, cs, red_grid(psi->size()), partial);
+}
+}  // namespace iqsi
 
 int iqsh_qaoa_phase(iqsh_handle h, unsigned ne, const unsigned* u, const unsigned* v, const double* w, double gamma)
 {

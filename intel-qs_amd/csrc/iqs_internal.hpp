@@ -56,6 +56,10 @@ inline bool cache_set(uint64_t bytes) { return bytes >= (uint64_t(32) << 20) && 
 // the phase exp(-i gamma cut) per amplitude.
 int build_cut_spec(iqsh_handle h, unsigned ne, const unsigned* u, const unsigned* v, const double* w, double gamma,
                    iqsk::CutSpec* cs);
+// lam := C psi with cost_blocks(psi) partial sums of cut |psi|^2 (iqsh_qaoa_cost_apply without
+// the sum).
+unsigned cost_blocks(iqsh_handle psi);
+int launch_cost(iqsh_handle psi, iqsh_handle lam, const iqsk::CutSpec& cs, double* partial);
 
 }  // namespace iqsi
 

@@ -365,24 +365,46 @@ __global__ __launch_bounds__((LTile<T, M, LR>::NT), (ADJ ? (sizeof(T) == 8 ? 2 :
   }
 }
 
+// Sums over workgroups, taken on the way: a pass reserves a run of partials on the device, a
+// kernel sums pending runs in a fixed order into pinned host memory when the buffer or its
+// argument list is full, and the host waits once, at the end (iqs_layer.hip).
+constexpr int kMaxSums = 32;
+struct SumRuns {
+  uint64_t off[kMaxSums], len[kMaxSums];
+};
+class LayerSums {
+ public:
+  // For passes of at most `run` partials in groups of at most `group` runs, `total` runs in all.
+  int begin(uint64_t run, int group, uint64_t total);
+  // Space for `count` (<= kMaxSums) consecutive runs of `run` partials each; their sums become
+  // results [taken(), taken() + count).
+  int take(uint64_t run, int count, double** part);
+  uint64_t taken() const { return done_ + n_; }
+  int flush();
+  // Every result, after the stream has been waited for.
+  int finish(const double** results);
+
+ private:
+  SumRuns runs_;
+  uint64_t used_ = 0, done_ = 0;
+  int n_ = 0;
+};
+
 // One layer's operands.
 struct LayerArgs {
   iqsh_handle psi, lam;  // lam: adjoint only
   const double* u;       // 2x2 (adjoint: the inverse)
   const double* g;       // generator (adjoint)
   const CutSpec* cs;     // QAOA phase, or null
-  double* grad;          // adjoint: sum_q 2 Im <lam| G_q |psi>
-  double* grad_phase;    // adjoint with cs: 2 Im <lam| C |psi>
+  // Adjoint: results of sum_q Im <lam| G_q |psi>, one per pass, then with cs Im <lam| C |psi>.
+  LayerSums* sums;
 };
 
-// Partial-sum buffer of at least `count` doubles, and the sums of `nsum` runs of partials
-// (offset, length) in a fixed order into out[] (synchronizes).  In iqs_layer.hip.
-int layer_parts(uint64_t count, double** part);
-constexpr int kMaxSums = 32;
-struct SumRuns {
-  uint64_t off[kMaxSums], len[kMaxSums];
+// Passes of a layer, and the partials of one.
+struct LayerShape {
+  unsigned passes;
+  uint64_t run;
 };
-int layer_sums(const SumRuns& runs, int nsum, double* out);
 
 // The window data of a weighted cut when the registers hold positions a .. a+LR-1.
 inline void build_cut_window(const CutSpec& cs, unsigned a, unsigned lr, CutWin* cw)
@@ -410,7 +432,7 @@ inline void build_cut_window(const CutSpec& cs, unsigned a, unsigned lr, CutWin*
 inline dim3 tile_grid(uint64_t G) { return dim3((unsigned)std::min<uint64_t>(G, 65536), (unsigned)((G + 65535) / 65536), 1); }
 
 template <typename T, int M, int LR, bool ADJ, int F, bool NT = true>
-int layer_m(const LayerArgs& a)
+int layer_m(const LayerArgs& a, LayerShape* shape)
 {
   using V = typename Vec<T>::t;
   using LT = LTile<T, M, LR>;
@@ -423,24 +445,18 @@ int layer_m(const LayerArgs& a)
   V* lam = ADJ ? (V*)a.lam->d : nullptr;
   const unsigned n = a.psi->n, rest = n - M, high = (rest + (M - LR) - 1) / (M - LR);
   const uint64_t G = uint64_t(1) << (n - M);
+  if (shape) {
+    *shape = {high + 1, G};
+    return IQSH_OK;
+  }
   const dim3 grid = tile_grid(G);
-  double* part = nullptr;
-  SumRuns runs;
-  int nsum = 0;
-  if (ADJ)
-    if (int rc = layer_parts(G * (high + 2), &part)) return rc;
-  auto next_run = [&]() -> double* {
-    if (!ADJ) return nullptr;
-    runs.off[nsum] = (uint64_t)nsum * G;
-    runs.len[nsum] = G;
-    return part + (uint64_t)nsum++ * G;
-  };
   // Forward: the low pass first (it carries the phase layer, applied before the mixer);
   // adjoint: last (the phase is undone after the whole mixer).
-  auto low_pass = [&]() {
+  auto low_pass = [&]() -> int {
     const TilePass tp{M, M};
-    double* p = next_run();
-    if (ADJ && a.cs) (void)next_run();  // the phase terms follow the generator terms
+    double* p = nullptr;
+    if (ADJ)  // with a phase its terms follow the generator terms
+      if (int rc = a.sums->take(G, a.cs ? 2 : 1, &p)) return rc;
     if (!a.cs) {
       k_layer_tile<T, M, LR, ADJ, true, F, kCutNone, NT><<<grid, LT::NT, 0, iqsi::stream()>>>(psi, lam, tp, u, g, NoCut{}, NoCut{}, p);
     } else if (!a.cs->weighted) {
@@ -450,25 +466,23 @@ int layer_m(const LayerArgs& a)
       build_cut_window(*a.cs, ADJ ? LR : M - LR, LR, &cw);
       k_layer_tile<T, M, LR, ADJ, true, F, kCutWeighted, NT><<<grid, LT::NT, 0, iqsi::stream()>>>(psi, lam, tp, u, g, *a.cs, cw, p);
     }
+    return IQSH_OK;
   };
-  if (!ADJ) low_pass();
+  if (!ADJ)
+    if (int rc = low_pass()) return rc;
   // Positions above the low pass in passes of as equal a size as possible.
   for (unsigned i = 0, p = M; i < high; ++i) {
     const unsigned m = rest / high + (i < rest % high ? 1 : 0);
     const TilePass tp{M - m, p};
-    k_layer_tile<T, M, LR, ADJ, false, F, kCutNone, NT><<<grid, LT::NT, 0, iqsi::stream()>>>(psi, lam, tp, u, g, NoCut{}, NoCut{}, next_run());
+    double* part = nullptr;
+    if (ADJ)
+      if (int rc = a.sums->take(G, 1, &part)) return rc;
+    k_layer_tile<T, M, LR, ADJ, false, F, kCutNone, NT><<<grid, LT::NT, 0, iqsi::stream()>>>(psi, lam, tp, u, g, NoCut{}, NoCut{}, part);
     p += m;
   }
-  if (ADJ) low_pass();
+  if (ADJ)
+    if (int rc = low_pass()) return rc;
   IQSI_TRY(hipGetLastError());
-  if (!ADJ) return IQSH_OK;
-  double s[kMaxSums];
-  if (int rc = layer_sums(runs, nsum, s)) return rc;
-  const int nmix = a.cs ? nsum - 1 : nsum;
-  double acc = 0;
-  for (int i = 0; i < nmix; ++i) acc += s[i];
-  *a.grad = 2.0 * acc;
-  if (a.cs) *a.grad_phase = 2.0 * s[nsum - 1];
   return IQSH_OK;
 }
 
@@ -480,37 +494,37 @@ int layer_m(const LayerArgs& a)
 // psi and lambda of 32 amplitudes left two waves per SIMD and spilled (25 qubits weighted
 // low pass 535 against 287 us).
 template <typename T, bool ADJ, int F>
-int layer_n(const LayerArgs& a)
+int layer_n(const LayerArgs& a, LayerShape* shape)
 {
   const unsigned n = a.psi->n;
   const bool cached = iqsi::cache_set(a.psi->size() * sizeof(typename Vec<T>::t) * (ADJ ? 2 : 1));
   if constexpr (sizeof(T) == 8) {
-    if (n <= 10 || (n > 12 && n <= 16)) return layer_m<T, 10, 4, ADJ, F>(a);
-    if (n == 11 || n == 17 || n == 18) return layer_m<T, 11, 4, ADJ, F>(a);
-    return cached ? layer_m<T, 12, 4, ADJ, F, false>(a) : layer_m<T, 12, 4, ADJ, F>(a);
+    if (n <= 10 || (n > 12 && n <= 16)) return layer_m<T, 10, 4, ADJ, F>(a, shape);
+    if (n == 11 || n == 17 || n == 18) return layer_m<T, 11, 4, ADJ, F>(a, shape);
+    return cached ? layer_m<T, 12, 4, ADJ, F, false>(a, shape) : layer_m<T, 12, 4, ADJ, F>(a, shape);
   } else if constexpr (ADJ) {
-    if (n <= 11 || (n > 12 && n <= 16)) return layer_m<T, 10, 4, ADJ, F>(a);
-    return cached ? layer_m<T, 12, 4, ADJ, F, false>(a) : layer_m<T, 12, 4, ADJ, F>(a);
+    if (n <= 11 || (n > 12 && n <= 16)) return layer_m<T, 10, 4, ADJ, F>(a, shape);
+    return cached ? layer_m<T, 12, 4, ADJ, F, false>(a, shape) : layer_m<T, 12, 4, ADJ, F>(a, shape);
   } else {
-    if (n <= 10) return layer_m<T, 10, 4, ADJ, F>(a);
-    if (n <= 12 || (n > 13 && n <= 17)) return layer_m<T, 11, 5, ADJ, F>(a);
-    return cached ? layer_m<T, 13, 5, ADJ, F, false>(a) : layer_m<T, 13, 5, ADJ, F>(a);
+    if (n <= 10) return layer_m<T, 10, 4, ADJ, F>(a, shape);
+    if (n <= 12 || (n > 13 && n <= 17)) return layer_m<T, 11, 5, ADJ, F>(a, shape);
+    return cached ? layer_m<T, 13, 5, ADJ, F, false>(a, shape) : layer_m<T, 13, 5, ADJ, F>(a, shape);
   }
 }
 
-// The RX-form kernels when the 2x2 has a real diagonal and an imaginary off-diagonal (the
+// With `shape` only that is filled in.  The RX-form kernels when the 2x2 has a real diagonal and an imaginary off-diagonal (the
 // QAOA mixer and its inverse) and, in the adjoint, the generator is exactly X.
 template <typename T>
-int do_layer(const LayerArgs& a)
+int do_layer(const LayerArgs& a, LayerShape* shape)
 {
   static const double X[8] = {0, 0, 1, 0, 1, 0, 0, 0};
   const bool rx = a.u[1] == 0 && a.u[2] == 0 && a.u[4] == 0 && a.u[7] == 0;
-  if (!a.lam) return rx ? layer_n<T, false, kFormRX>(a) : layer_n<T, false, 0>(a);
+  if (!a.lam) return rx ? layer_n<T, false, kFormRX>(a, shape) : layer_n<T, false, 0>(a, shape);
   const bool gx = std::equal(a.g, a.g + 8, X);
-  return rx && gx ? layer_n<T, true, kFormGX | kFormRX>(a) : layer_n<T, true, 0>(a);
+  return rx && gx ? layer_n<T, true, kFormGX | kFormRX>(a, shape) : layer_n<T, true, 0>(a, shape);
 }
 
-extern template int do_layer<float>(const LayerArgs&);
-extern template int do_layer<double>(const LayerArgs&);
+extern template int do_layer<float>(const LayerArgs&, LayerShape*);
+extern template int do_layer<double>(const LayerArgs&, LayerShape*);
 
 }  // namespace iqsl

@@ -33,6 +33,13 @@ def _edges(edges) -> Tuple[int, object, object, object, tuple]:
     return len(e), u, v, w, (u, v, w)
 
 
+def _angles(gammas, betas) -> Tuple[np.ndarray, np.ndarray]:
+    g, b = (np.ascontiguousarray(x, dtype=np.float64).reshape(-1) for x in (gammas, betas))
+    if g.size != b.size:
+        raise ValueError(f"{g.size} gammas but {b.size} betas")
+    return g, b
+
+
 class StateVector:
     def __init__(self, num_qubits: int, dtype="c128", *, _handle=None):
         self.num_qubits = int(num_qubits)
@@ -237,6 +244,22 @@ class StateVector:
         call("iqsh_qaoa_layer_adjoint", self._h, lam._h, ne, u, v, w, float(gamma), a.ctypes.data, g.ctypes.data,
              C.byref(dg), C.byref(dm))
         return dg.value, dm.value
+
+    def qaoa_run(self, edges, gammas, betas) -> None:
+        """|+>^n, then every QAOA layer of the angles (>= 10 qubits)."""
+        ne, u, v, w, _keep = _edges(edges)
+        g, b = _angles(gammas, betas)
+        call("iqsh_qaoa_run", self._h, g.size, ne, u, v, w, g.ctypes.data, b.ctypes.data)
+
+    def qaoa_gradient(self, lam: "StateVector", edges, gammas, betas) -> Tuple[float, np.ndarray, np.ndarray]:
+        """Cost and its derivatives by every angle from the final state of `qaoa_run`, which is
+        walked back to |+>^n; lam is the second state of the adjoint method."""
+        ne, u, v, w, _keep = _edges(edges)
+        g, b = _angles(gammas, betas)
+        dg, db, cost = np.zeros(g.size), np.zeros(g.size), C.c_double()
+        call("iqsh_qaoa_gradient", self._h, lam._h, g.size, ne, u, v, w, g.ctypes.data, b.ctypes.data, C.byref(cost),
+             dg.ctypes.data, db.ctypes.data)
+        return cost.value, dg, db
 
     def adjoint_1q_all(self, lam: "StateVector", uinv, G) -> float:
         """Backward step through a layer of the same gate on every qubit: returns

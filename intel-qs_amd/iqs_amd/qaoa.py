@@ -71,8 +71,12 @@ class MaxCutQaoa:
         """Run the circuit; `shift` = (kind, layer, index, delta) adds one extra rotation
         (an edge phase or a qubit RX) used by the parameter-shift rule."""
         psi = self._state("_psi")
-        self._prepare(psi)
         fused = self.num_qubits >= LAYER_MIN_QUBITS
+        if fused and not shift and not self.renorm_every:
+            layers = min(len(gammas), len(betas))
+            psi.qaoa_run(self.edges, gammas[:layers], betas[:layers])
+            return psi
+        self._prepare(psi)
         for l, (g, b) in enumerate(zip(gammas, betas)):
             if shift and shift[0] == "edge" and shift[1] == l:
                 # diagonal phases commute: the extra edge phase may precede the layer
@@ -101,13 +105,12 @@ class MaxCutQaoa:
         p = len(gammas)
         psi = self._state("_psi")
         lam = self._state("_lam")
+        if self.num_qubits >= LAYER_MIN_QUBITS:
+            return psi.qaoa_gradient(lam, self.edges, gammas, betas[:p])
         cost = psi.qaoa_cost_apply(lam, self.edges)
         dg, db = np.zeros(p), np.zeros(p)
         for l in reversed(range(p)):
             uinv = G.rx(-2.0 * betas[l])
-            if self.num_qubits >= LAYER_MIN_QUBITS:
-                dg[l], db[l] = psi.qaoa_layer_adjoint(lam, self.edges, gammas[l], uinv, X)
-                continue
             s = 0.0
             for q in reversed(range(self.num_qubits)):
                 s += psi.adjoint_1q(lam, q, uinv, X)
