@@ -317,7 +317,7 @@ int iqsh_hea_variants(int dtype, int *count);
 int iqsh_hea_variant_info(int dtype, int variant, int *tile_qubits, int *amps_per_thread,
                           int *threads, int *for_tests);
 /* Create a batch (allocates every state and work buffer); tune NULL = default variant 0,
- * as many workers as fit, order 0. */
+ * as many workers as fit and find work, order 0. */
 int iqsh_hea_create(int dtype, int count, const int *nqubits, const int *depth,
                     const iqsh_hea_tune *tune, iqsh_hea_handle *out);
 int iqsh_hea_destroy(iqsh_hea_handle h);

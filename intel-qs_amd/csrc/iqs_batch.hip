@@ -36,6 +36,13 @@
 //    s-1 of its instance have arrived.  Every task waits only on tasks earlier in the
 //    queue, which were taken by running workgroups, so the queue always drains; waits are
 //    bounded and set an abort flag instead of hanging.
+//  * Bounds (64 registers of 10..22 qubits, complex64, cost and gradient, 2.0e9 amplitude-layers):
+//    43.6 ms, of which the vector instructions take 24 (480 per amplitude and layer; the
+//    SIMDs' vector units are busy for 55%) and the traffic of the passes, 48 bytes per amplitude
+//    and layer, 15 at the rate of a copy; the rest is scalar work and waits that two workgroups per
+//    compute unit do not cover.  Before, with RY as four products, the CZ signs computed per
+//    amplitude, one workgroup per compute unit and loop bounds in vector registers: 66.3 ms (740
+//    vector instructions).
 //  * Gradient sums are FP64 (products of FP32 amplitudes are formed in FP32): per gate a DPP
 //    wave sum, per tile a fixed-order sum over waves, written as per-tile partials and
 //    reduced in tile order by an epilogue kernel.
@@ -67,7 +74,7 @@ struct HeaInst {
   uint64_t part;      // tiled: gradient partials [depth][n][2 (theta, phi)][tiles]
   uint64_t cpart;     // tiled: cost partials [tiles]
   uint32_t arrive;    // tiled: arrival counter of step 0 (one counter per step)
-  uint32_t pad;
+  uint32_t lay;       // first layer of the instance in flips
 };
 
 struct HeaTask {
@@ -81,6 +88,30 @@ constexpr int kQueues = 8;
 constexpr int kCtlAbort = kQueues;       // ctl[0..7]: queue heads, ctl[8]: abort flag
 constexpr int kCtlArrive = kQueues + 1;  // ctl[9 + i]: arrival counter i
 
+// A value that is the same in every lane, as a scalar: what is computed from it (loop bounds,
+// branches, addresses of gate factors) then is scalar as well, which the compiler cannot know of
+// values read from LDS.
+template <typename S>
+__device__ __forceinline__ S uniform(S v)
+{
+  static_assert(sizeof(S) % 4 == 0, "whole registers");
+  uint32_t w[sizeof(S) / 4];
+  __builtin_memcpy(w, &v, sizeof(S));
+#pragma unroll
+  for (size_t i = 0; i < sizeof(S) / 4; ++i) w[i] = __builtin_amdgcn_readfirstlane(w[i]);
+  __builtin_memcpy(&v, w, sizeof(S));
+  return v;
+}
+
+// Factors of one (layer, qubit) pair (see the scaled rotations below).
+template <typename T> struct HeaGate {
+  T tan;       // of the rotation of the bit
+  T far;       // 1: the rotation inverts the bit
+  V<T> rz;     // kap (cos phi/2, sin phi/2)
+  double ik2;  // 1 / kap^2
+  double pad;
+};
+
 template <typename T> struct HeaArgs {
   const HeaInst* inst;
   const HeaTask* task;  // the queues, back to back
@@ -88,7 +119,8 @@ template <typename T> struct HeaArgs {
   uint32_t flags;
   uint32_t* ctl;
   V<T>* arena;
-  const V<T>* mats;  // 4 entries per pair: (cos, sin) of theta/2 and of phi/2, then 2 unused
+  const HeaGate<T>* gates;
+  const uint32_t* flips;
   double* grad;
   double* cost;
   double* part;
@@ -221,83 +253,146 @@ __device__ __forceinline__ C cx_mulc(const C& a, const C& b)  // a * conj(b)
 // diagonal.  Gradients: dC/dtheta = Im<lam|Y_q|psi> just after the RY (one sum per pair),
 // dC/dphi = Im<lam|Z_q|psi> at the diagonal that holds the RZ (one product per amplitude,
 // signed by the qubit's bit), both from partial sums over a thread's registers.
-// mats: 4 entries per (layer, qubit): (cos theta/2, sin theta/2), (cos phi/2, sin phi/2), 0, 0.
+//
+// Scaled rotations.  RY(theta) = c [[1, -t], [t, 1]] with t = tan(theta/2): without its scale a
+// rotation is one FMA per real number instead of a product and an FMA, and rounds once instead of
+// twice.  Where |t| > 1, RY(theta) = RY(pi) RY(theta - pi): the second factor has a t of at most 1,
+// and RY(pi) is a sign and an exchange of the two values of the qubit, which is not carried out: from
+// there on the qubit's bit in the index of an amplitude holds the opposite of its value.  So
+//  * the scale kap = c (or s, of theta - pi) is part of the qubit's RZ factor, kap e^{-+i phi/2}: on
+//    the way forward the diagonal brings the amplitudes back to their size after the rotations, on
+//    the way back it scales them before the transposed rotations.  Between a rotation and its
+//    diagonal the amplitudes are larger by up to sqrt(2) per rotation (2^(M/2) over a pass), and
+//    the gradient sums formed there are divided by the kap^2 of the rotations still to come
+//    (HeaGate::ik2);
+//  * flips[l] has the qubits whose bits are inverted after layer l's rotations: an inverted
+//    qubit rotates by -t, diagonals, costs and kept states take value = bit ^ flip, and
+//    sums over Y_q and Z_q change their sign.  The sign of RY(pi) (value 0 gets -1) is in the
+//    diagonal of the qubit's RZ.
+// (Branches to a cot form for |t| > 1 instead took 60 registers more: each form's results get
+// registers of their own.)
 template <typename T, int M, int R>
 struct Tile {
   static constexpr int LR = ilog2(R);
   static constexpr int NT = (1 << M) / R;
   static constexpr int NW = NT / 64;
-  static constexpr int KMAX = M;       // register phases of one sweep (at most)
+  static constexpr int KMAX = 1 + (M - 2) / (LR - 1);  // register phases of one sweep (at most)
   static constexpr int SLOTS = 4 * M;  // dtheta of two layers' gated bits, dphi of <= 2M qubits
   static_assert(R >= 4 && (R & (R - 1)) == 0, "R must be a power of two >= 4");
   static_assert(NT >= 64 && NT <= 1024, "workgroup of 1..16 wavefronts");
-  static_assert(KMAX * R <= NT, "one table entry per thread");
   using G = Geo<M, LR>;
   using C = V<T>;
 
-  static __device__ void relayout(C* v, C* lds, int from, int to)
+  // Tables of one sweep in LDS.
+  static constexpr int CH = 16 / sizeof(C);  // diagonal entries per 16-byte read
+  struct Tab {
+    C zt[KMAX * 8 * R];  // diagonals: phase, CH registers, variant (see diag_variant), register
+    T ry[2][M];          // rotations of row_pre and row_post by local bit
+    C rz[2 * M];         // row_pre by qubit
+    double ik2[3 * M];   // row_pre by qubit, then row_post by local bit
+  };
+
+  // The thread's index, computed anew where it is used: what follows from it is not kept in
+  // registers across the passes.
+  static __device__ __forceinline__ uint32_t thread()
   {
-    const uint32_t tid = threadIdx.x;
-#pragma unroll
-    for (int k = 0; k < R; ++k) lds[phys<LR>(lidx<LR>(tid, k, from))] = v[k];
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < R; ++k) v[k] = lds[phys<LR>(lidx<LR>(tid, k, to))];
-    __syncthreads();
+    uint32_t t = threadIdx.x;
+    __asm__ volatile("" : "+v"(t));
+    return t;
   }
 
-  // RY_q (real) on the register bits in rmask; `row` = matrices of qubit 0 of the layer.
-  static __device__ void ry_fwd(C* x, uint32_t rmask, const C* row, int a, const G& g)
+  // Registers <-> LDS.  The slot of (thread, register k) is linear over XOR in both, so the
+  // registers are visited in Gray-code order with one XOR by a scalar per access.
+  template <typename F>
+  static __device__ void visit_lds(C* lds, int a, F f)
+  {
+    uint32_t at = phys<LR>(lidx<LR>(thread(), 0, a)) * (uint32_t)sizeof(C);
+    uint32_t step[LR];
+#pragma unroll
+    for (int j = 0; j < LR; ++j) step[j] = phys<LR>(1u << (a + j)) * (uint32_t)sizeof(C);
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+      f(*reinterpret_cast<C*>(reinterpret_cast<char*>(lds) + at), i ^ (i >> 1));
+      if (i + 1 < R) at ^= step[__builtin_ctz(i + 1)];
+    }
+  }
+  // Layouts a <= 6 have the same highest local bits on the bits of the wavefront's number, and
+  // their exchange stays within each wavefront: its LDS accesses are in order, no barrier is needed.
+  static __device__ void relayout(C* v, C* lds, int from, int to)
+  {
+    const bool in_wave = from <= 6 && to <= 6;
+    visit_lds(lds, from, [&](C& s, int k) { s = v[k]; });
+    if (in_wave)
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    else
+      __syncthreads();
+    visit_lds(lds, to, [&](C& s, int k) { v[k] = s; });
+    if (in_wave)
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    else
+      __syncthreads();
+  }
+
+  // The rotation of register bit j without its scale (its transpose: -t).
+  static __device__ __forceinline__ void rotate(C* x, int j, T t)
   {
 #pragma unroll
-    for (int j = 0; j < LR; ++j) {
-      if ((rmask >> j) & 1u) {
-        const C cs = row[4 * g.gq(a + j)];
-        const T c = cs.x, sn = cs.y;
-#pragma unroll
-        for (int k = 0; k < R; ++k) {
-          if ((k >> j) & 1) continue;
-          const int k1 = k | (1 << j);
-          const C p0 = x[k], p1 = x[k1];
-          x[k].x = c * p0.x - sn * p1.x;
-          x[k].y = c * p0.y - sn * p1.y;
-          x[k1].x = sn * p0.x + c * p1.x;
-          x[k1].y = sn * p0.y + c * p1.y;
-        }
-      }
+    for (int k = 0; k < R; ++k) {
+      if ((k >> j) & 1) continue;
+      const int k1 = k | (1 << j);
+      const C p0 = x[k], p1 = x[k1];
+      x[k].x = p0.x - t * p1.x;
+      x[k].y = p0.y - t * p1.y;
+      x[k1].x = p1.x + t * p0.x;
+      x[k1].y = p1.y + t * p0.y;
     }
   }
 
-  // Backward through RY_q for psi (x) and lam (y): Im<lam|Y_q|psi> (summed over this thread's
-  // pairs, then the wavefront) into redw[slot0 + lbit - la], then RY_q^T on both.
-  static __device__ void ry_bwd(C* x, C* y, uint32_t rmask, const C* row, int a, const G& g, double* redw, int slot0)
+  // The rotation of register bit j, or none if the bit is not in rmask.
+  static __device__ T tan_of(const T* ry, int j, uint32_t rmask)
   {
-    const bool lane63 = (threadIdx.x & 63) == 63;
+    const T t = uniform(ry[j]);
+    return (rmask >> j) & 1u ? t : T(0);
+  }
+
+  // Rotations on the register bits in rmask; ry[j] = rotation of register bit j.  Only bit RARE
+  // (the one that a single phase of the sweep rotates) is branched around: where a path leaves
+  // all registers as they are, the compiler copies every one of them on the other path.
+  template <int RARE>
+  static __device__ void ry_fwd(C* x, uint32_t rmask, const T* ry)
+  {
 #pragma unroll
     for (int j = 0; j < LR; ++j) {
+      if (j == RARE && !((rmask >> j) & 1u)) continue;
+      rotate(x, j, tan_of(ry, j, rmask));
+    }
+  }
+
+  // Backward through the rotations for psi (x) and lam (y), in reverse order:
+  // Im<lam|Y_q|psi> (summed over this thread's pairs, then the wavefront) into redw[j], then the
+  // transposed rotation on both.
+  template <int RARE>
+  static __device__ void ry_bwd(C* x, C* y, uint32_t rmask, const T* ry, double* redw)
+  {
+    const bool lane63 = (thread() & 63) == 63;
+#pragma unroll
+    for (int j = LR - 1; j >= 0; --j) {
+      if (j == RARE && !((rmask >> j) & 1u)) continue;
       if ((rmask >> j) & 1u) {
-        const C cs = row[4 * g.gq(a + j)];
-        const T c = cs.x, sn = cs.y;
         T acc = 0;
 #pragma unroll
         for (int k = 0; k < R; ++k) {
           if ((k >> j) & 1) continue;
           const int k1 = k | (1 << j);
-          const C p0 = x[k], p1 = x[k1], l0 = y[k], l1 = y[k1];
           // Im(conj(l0) (-i p1) + conj(l1) (i p0)) = Re(conj(l1) p0) - Re(conj(l0) p1)
-          acc += (l1.x * p0.x + l1.y * p0.y) - (l0.x * p1.x + l0.y * p1.y);
-          x[k].x = c * p0.x + sn * p1.x;
-          x[k].y = c * p0.y + sn * p1.y;
-          x[k1].x = c * p1.x - sn * p0.x;
-          x[k1].y = c * p1.y - sn * p0.y;
-          y[k].x = c * l0.x + sn * l1.x;
-          y[k].y = c * l0.y + sn * l1.y;
-          y[k1].x = c * l1.x - sn * l0.x;
-          y[k1].y = c * l1.y - sn * l0.y;
+          acc += (y[k1].x * x[k].x + y[k1].y * x[k].y) - (y[k].x * x[k1].x + y[k].y * x[k1].y);
         }
         const double sum = wave_sum63((double)acc);
-        if (lane63) redw[slot0 + a + j - g.la] = sum;
+        if (lane63) redw[j] = sum;
       }
+      const T t = -tan_of(ry, j, rmask);
+      rotate(x, j, t);
+      rotate(y, j, t);
     }
   }
 
@@ -313,104 +408,173 @@ struct Tile {
     return m & ((1u << LR) - 1u);
   }
 
-  // Diagonal tables of one sweep: zt[k][r] = product of the RZ factors of phase k's
-  // register bits for register index r (bit 0 -> e^{-i phi/2}, bit 1 -> e^{+i phi/2}).
-  // Barriers on both sides: no thread still reads the previous sweep's table.
-  static __device__ void build_tables(C* zt, const G& g, const C* row, bool defer_b)
+  // Parity of the CZ pairs in czm that are set in x, and the qubits with an odd number of set
+  // neighbours in x: the sign of x | r is that of x, that of r, and r & neighbours.
+  static __device__ uint32_t cz_parity(uint32_t x, uint32_t czm) { return (uint32_t)__popc(x & (x >> 1) & czm) & 1u; }
+  static __device__ uint32_t cz_neighbours(uint32_t x, uint32_t czm)
   {
+    return ((x >> 1) & czm) ^ ((x & czm) << 1);
+  }
+
+  // The qubits on the registers' bits.
+  static __device__ uint32_t reg_qubits(const G& g, int a) { return g.gidx(((1u << LR) - 1u) << a) ^ g.gidx(0); }
+
+  // Which of the 8 signed copies of phase k's diagonal this thread takes: the CZ sign of its
+  // lane and tile bits, and whether they flip the sign of the lowest and of the highest register
+  // bit (the register bits between have no lane bit next to them).
+  static __device__ uint32_t diag_variant(const G& g, int a, uint32_t czm, uint32_t flip)
+  {
+    const uint32_t x = g.gidx(lidx<LR>(thread(), 0, a)) ^ (flip & ~reg_qubits(g, a));
+    const uint32_t nb = cz_neighbours(x, czm);
+    return cz_parity(x, czm) | ((nb >> g.gq(a)) & 1u) << 1 | ((nb >> g.gq(a + LR - 1)) & 1u) << 2;
+  }
+
+  // Inverted bits in the values of row_pre's layer, and those that its rotations inverted.
+  struct Flip {
+    uint32_t all, now;
+  };
+  static __device__ Flip flip_of(const HeaArgs<T>& A, const HeaInst& I, int layer)
+  {
+    if (layer < 0) return Flip{0, 0};
+    const uint32_t f = uniform(A.flips[I.lay + layer]);
+    return Flip{f, layer ? f ^ uniform(A.flips[I.lay + layer - 1]) : f};
+  }
+
+  // The gates of one sweep into LDS, then per phase the diagonal of its register bits in the
+  // 8 variants of diag_variant: RZ factors (with the rotations' scales) and CZ signs.  Barriers
+  // on both sides: no thread still reads the previous sweep's tables.
+  static __device__ void build_tables(Tab& tb, const G& g, const HeaGate<T>* gates, int64_t row_pre, int64_t row_post,
+                                      bool defer_b, Flip f2)
+  {
+    const int i = (int)threadIdx.x;
+    static_assert(NT >= 3 * M, "one gate per thread");
+    HeaGate<T> h;
+    const bool pre = row_pre >= 0 && i < g.n;
+    const bool post = row_post >= 0 && i >= 2 * M && i < 2 * M + g.lb - g.la;
+    if (pre) h = gates[row_pre + i];
+    if (post) h = gates[row_post + g.gq(g.la + i - 2 * M)];
     __syncthreads();
-    const uint32_t i = threadIdx.x;
-    if (i < (uint32_t)(g.K * R)) {
-      const int k = i / R, r = i % R, a = g.a(k);
-      const uint32_t m = zreg(g, k, defer_b);
-      C f{1, 0};
-      for (int j = 0; j < LR; ++j)
-        if ((m >> j) & 1u) {
-          const C h = row[4 * g.gq(a + j) + 1];
-          f = cx_mul(f, C{h.x, ((r >> j) & 1) ? h.y : -h.y});
+    if (pre) {
+      tb.rz[i] = h.rz;
+      tb.ik2[i] = h.ik2;
+      // local bit of qubit i, where the pass rotates it
+      const int lb = g.kind == 2 ? (i >= M ? i - M + g.c : -1) : i;
+      if (lb >= g.la && lb < g.lb) tb.ry[0][lb] = h.tan;
+    }
+    if (post) {
+      tb.ry[1][g.la + i - 2 * M] = h.tan;
+      tb.ik2[i] = h.ik2;
+    }
+    __syncthreads();
+    if (row_pre >= 0) {
+      const uint32_t tile = g.gidx(0);
+      // tile bits as values
+      const uint32_t tilev = (tile ^ f2.all) & ~(g.gidx((1u << M) - 1u) ^ tile);
+      for (int e = i; e < g.K * 4 * R; e += NT) {
+        const uint32_t r = e % R, lh = e / R % 4;
+        const int k = e / (4 * R), a = g.a(k);
+        const uint32_t m = zreg(g, k, defer_b), czm = g.czmask(k);
+        const uint32_t xr = g.gidx(r << a) ^ tile ^ (f2.all & reg_qubits(g, a)), nb = cz_neighbours(tilev, czm);
+        uint32_t sg = cz_parity(xr, czm);
+        C f{1, 0};
+#pragma unroll
+        for (int j = 0; j < LR; ++j) {
+          const int q = g.gq(a + j);
+          const uint32_t one = (xr >> q) & 1u;
+          sg ^= one & (j == 0 ? lh : j == LR - 1 ? lh >> 1 : nb >> q);
+          if ((m >> j) & 1u) {
+            const C z = tb.rz[q];
+            f = cx_mul(f, C{z.x, one ? z.y : -z.y});
+            sg ^= (f2.now >> q) & ~one;
+          }
         }
-      zt[i] = f;
+        sg &= 1u;
+        if (sg) f = C{-f.x, -f.y};
+        C* to = tb.zt + k * 8 * R + (r & ~(uint32_t)(CH - 1)) * 8 + (r & (CH - 1)) + 2 * lh * CH;
+        to[0] = f;
+        to[CH] = C{-f.x, -f.y};
+      }
     }
     __syncthreads();
   }
 
-  // This thread's factor of the deferred RZs on bits that are not register bits in phase 0
-  // (lane bits and tile bits).  defer: global qubits [q0, q1) of the previous pass.
-  static __device__ C deferred_factor(const G& g, const C* row, int q0, int q1)
+  // This thread's factor of the deferred RZs on bits that are not register bits in phase 0 (lane
+  // bits and tile bits; the lane bits are the same in the load/store layout).  Global qubits
+  // [q0, q1) of the previous pass.  The pass does not rotate them before their RZ: the factor is
+  // applied to the loaded amplitudes, and backward to the ones to be stored.
+  static __device__ C deferred_factor(const G& g, const C* rz, int q0, int q1, Flip f2)
   {
     const int a = g.a(0);
-    const uint32_t x0 = g.gidx(lidx<LR>(threadIdx.x, 0, a));  // register bits 0
+    const uint32_t x0 = g.gidx(lidx<LR>(thread(), 0, a)) ^ f2.all;  // register bits 0
     C f{1, 0};
+    uint32_t sg = 0;
     for (int q = q0; q < q1; ++q) {
       // register bit in phase 0: the table has it (only local bits [a, a + LR) of a B tile)
       if (g.kind == 2 && q < g.c && q >= a && q < a + LR) continue;
-      const C h = row[4 * q + 1];
+      const C h = rz[q];
       f = cx_mul(f, C{h.x, ((x0 >> q) & 1u) ? h.y : -h.y});
+      sg ^= (f2.now & ~x0) >> q;
     }
-    return f;
+    return sg & 1u ? C{-f.x, -f.y} : f;
   }
 
-  // x *= diag (conj: x *= conj(diag), and y likewise when given); diag = CZ signs (czm) x
-  // zt[k][r] (x f0 in phase 0).
-  template <bool BOTH>
-  static __device__ void diag_apply(C* x, C* y, const C* ztk, const C& f0, bool use_f0, uint32_t czm, int a,
-                                    const G& g, bool conj)
+  // x *= diagonal of phase k, or its conjugate on x and y.
+  template <bool BWD>
+  static __device__ void diag_apply(C* x, C* y, const Tab& tb, int k, const G& g, uint32_t flip)
   {
-    const uint32_t tid = threadIdx.x;
-#pragma unroll
-    for (int k = 0; k < R; ++k) {
-      C f = ztk[k];
-      if (use_f0) f = cx_mul(f, f0);
-      if (czm) {
-        const uint32_t xg = g.gidx(lidx<LR>(tid, k, a));
-        if (__popc(xg & (xg >> 1) & czm) & 1) f = C{-f.x, -f.y};
-      }
-      x[k] = conj ? cx_mulc(x[k], f) : cx_mul(x[k], f);
-      if (BOTH) y[k] = conj ? cx_mulc(y[k], f) : cx_mul(y[k], f);
-    }
-  }
-
-  // Im<lam|Z_q|psi> for the RZ qubits of phase k into redw[slot0 + q] (register bits of
-  // zreg, and in phase 0 the deferred qubits [q0, q1) on lane or tile bits).
-  static __device__ void dphi(const C* x, const C* y, int k, const G& g, bool defer_b, int q0, int q1, double* redw,
-                              int slot0)
-  {
-    const bool lane63 = (threadIdx.x & 63) == 63;
-    const int a = g.a(k);
-    T tot = 0, hi[LR];  // hi[j]: registers with bit j set (Z = -1 there)
-#pragma unroll
-    for (int j = 0; j < LR; ++j) hi[j] = 0;
+    const C* zt = tb.zt + k * 8 * R + diag_variant(g, g.a(k), g.czmask(k), flip) * CH;
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-      const T t = y[r].x * x[r].y - y[r].y * x[r].x;  // Im(conj(lam) psi)
-      tot += t;
-#pragma unroll
-      for (int j = 0; j < LR; ++j)
-        if ((r >> j) & 1) hi[j] += t;
+      const C f = zt[(r & ~(CH - 1)) * 8 + (r & (CH - 1))];
+      x[r] = BWD ? cx_mulc(x[r], f) : cx_mul(x[r], f);
+      if (BWD) y[r] = cx_mulc(y[r], f);
     }
+  }
+
+  // Im<lam|Z_q|psi> (Z of the bits) for the RZ qubits of phase k into redw[q] (register bits of zreg, and in
+  // phase 0 the deferred qubits [q0, q1) on lane or tile bits).
+  static __device__ void dphi(const C* x, const C* y, int k, const G& g, bool defer_b, int q0, int q1, double* redw)
+  {
+    const bool lane63 = (thread() & 63) == 63;
+    const int a = g.a(k);
+    T s[R], hi[LR];  // hi[j]: registers with bit j set (Z = -1 there)
+#pragma unroll
+    for (int r = 0; r < R; ++r) s[r] = y[r].x * x[r].y - y[r].y * x[r].x;  // Im(conj(lam) psi)
+#pragma unroll
+    for (int j = 0; j < LR; ++j) {
+      hi[j] = s[1];
+#pragma unroll
+      for (int r = 3; r < (R >> j); r += 2) hi[j] += s[r];
+#pragma unroll
+      for (int r = 0; r < (R >> (j + 1)); ++r) s[r] = s[2 * r] + s[2 * r + 1];
+    }
+    const T tot = s[0];
     const uint32_t m = zreg(g, k, defer_b);
 #pragma unroll
     for (int j = 0; j < LR; ++j) {
       if ((m >> j) & 1u) {
         const double sum = wave_sum63((double)(tot - 2 * hi[j]));
-        if (lane63) redw[slot0 + g.gq(a + j)] = sum;
+        if (lane63) redw[g.gq(a + j)] = sum;
       }
     }
     if (k == 0 && q1 > q0) {
-      const uint32_t x0 = g.gidx(lidx<LR>(threadIdx.x, 0, a));
+      const uint32_t x0 = g.gidx(lidx<LR>(thread(), 0, a));
+      const double all = wave_sum63((double)tot);
       for (int q = q0; q < q1; ++q) {
-        if (g.kind == 2 && q < g.c && q >= a && q < a + LR) continue;  // register bit: done above
-        const double sum = wave_sum63((double)(((x0 >> q) & 1u) ? -tot : tot));
-        if (lane63) redw[slot0 + q] = sum;
+        double sum = ((x0 >> q) & 1u) ? -all : all;  // a qubit on a wave or tile bit: the same in every lane
+        if (g.kind == 2 && q < g.c) {
+          if (q >= a && q < a + LR) continue;  // register bit: done above
+          if ((q < a ? q : q - LR) < 6) sum = wave_sum63((double)(((x0 >> q) & 1u) ? -tot : tot));
+        }
+        if (lane63) redw[q] = sum;
       }
     }
   }
 
-  // Forward sweep: per phase, RY of layer row_pre on the pre bits, the diagonal (RZ of
-  // row_pre on those bits and the deferred qubits [q0, q1), CZ pairs), RY of row_post.
-  // A negative row skips that layer.  zt: tables built for row_pre.
-  static __device__ void sweep_fwd(C* x, C* lds, int& cur, const G& g, const C* mats, int64_t row_pre,
-                                   int64_t row_post, const C* zt, const C& f0, bool has_f0)
+  // Forward sweep: per phase, RY of layer j-1 on the pre bits, the diagonal (RZ of that layer
+  // on those bits and the deferred qubits [q0, q1), CZ pairs), RY of layer j.
+  static __device__ void sweep_fwd(C* x, C* lds, int& cur, const G& g, const Tab& tb, bool pre, bool post,
+                                   uint32_t flip)
   {
     for (int k = 0; k < g.K; ++k) {
       const int nb = g.nb(k), ne = g.ne(k), a = g.a(k);
@@ -418,22 +582,21 @@ struct Tile {
         relayout(x, lds, cur, a);
         cur = a;
       }
-      if (row_pre >= 0) {
-        ry_fwd(x, bit_range(nb - a, ne - a), mats + 4 * row_pre, a, g);
-        diag_apply<false>(x, x, zt + k * R, f0, k == 0 && has_f0, g.czmask(k), a, g, false);
+      if (pre) {
+        ry_fwd<0>(x, bit_range(nb - a, ne - a), tb.ry[0] + a);
+        diag_apply<false>(x, x, tb, k, g, flip);
       }
-      if (row_post >= 0) {
+      if (post) {
         const int lo = max(nb - 1, g.la), hi = (k == g.K - 1) ? g.lb : ne - 1;
-        ry_fwd(x, bit_range(lo - a, hi - a), mats + 4 * row_post, a, g);
+        ry_fwd<LR - 1>(x, bit_range(lo - a, hi - a), tb.ry[1] + a);
       }
     }
   }
 
-  // Exact reverse of sweep_fwd on psi and lam with the gradient sums: dtheta of row_post at
-  // slots [0, M), of row_pre at [M, 2M) (by local bit - la), dphi of row_pre at 2M + qubit.
-  static __device__ void sweep_bwd(C* x, C* y, C* lds, int& cur, const G& g, const C* mats, int64_t row_pre,
-                                   int64_t row_post, const C* zt, const C& f0, bool has_f0, bool defer_b, int q0,
-                                   int q1, double* redw)
+  // Exact reverse of sweep_fwd on psi and lam with the gradient sums: dtheta of the post row at
+  // slots [0, M), of the pre row at [M, 2M) (by local bit), dphi of the pre row at 2M + qubit.
+  static __device__ void sweep_bwd(C* x, C* y, C* lds, int& cur, const G& g, const Tab& tb, bool pre, bool post,
+                                   uint32_t flip, bool defer_b, int q0, int q1, double* redw)
   {
     for (int k = g.K - 1; k >= 0; --k) {
       const int nb = g.nb(k), ne = g.ne(k), a = g.a(k);
@@ -442,27 +605,53 @@ struct Tile {
         relayout(y, lds, cur, a);
         cur = a;
       }
-      if (row_post >= 0) {
+      if (post) {
         const int lo = max(nb - 1, g.la), hi = (k == g.K - 1) ? g.lb : ne - 1;
-        ry_bwd(x, y, bit_range(lo - a, hi - a), mats + 4 * row_post, a, g, redw, 0);
+        ry_bwd<LR - 1>(x, y, bit_range(lo - a, hi - a), tb.ry[1] + a, redw + a);
       }
-      if (row_pre >= 0) {
-        dphi(x, y, k, g, defer_b, q0, q1, redw, 2 * M);
-        diag_apply<true>(x, y, zt + k * R, f0, k == 0 && has_f0, g.czmask(k), a, g, true);
-        ry_bwd(x, y, bit_range(nb - a, ne - a), mats + 4 * row_pre, a, g, redw, M);
+      if (pre) {
+        dphi(x, y, k, g, defer_b, q0, q1, redw + 2 * M);
+        diag_apply<true>(x, y, tb, k, g, flip);
+        ry_bwd<0>(x, y, bit_range(nb - a, ne - a), tb.ry[0] + a, redw + M + a);
       }
     }
   }
 
+  // What the sums of sweep_bwd are multiplied with: 1 / kap^2 of every rotation that the sweep
+  // had not yet undone while its scale was already applied.  Those are the post rotations of lower
+  // bits and the bit itself; for a pre bit of phase k the post rotations of lower phases and the
+  // pre ones of the phase up to the bit itself.
+  static __device__ double post_scale(const G& g, const Tab& tb, int end)
+  {
+    double f = 1;
+    for (int b = 0; b < end - g.la; ++b) f *= tb.ik2[2 * M + b];
+    return f;
+  }
+  static __device__ int phase_of(const G& g, int lbit)
+  {
+    int k = 0;
+    while (g.ne(k) <= lbit) ++k;
+    return k;
+  }
+  static __device__ double pre_scale(const G& g, const Tab& tb, bool post, int lbit)
+  {
+    const int k = phase_of(g, lbit);
+    double f = post ? post_scale(g, tb, max(g.nb(k) - 1, g.la)) : 1.0;
+    for (int b = g.nb(k); b <= lbit; ++b) f *= tb.ik2[g.gq(b)];
+    for (int q = 0; k == 0 && g.kind == 2 && q < g.c; ++q)  // deferred, on register bits
+      if (q >= g.a(0)) f *= tb.ik2[q];
+    return f;
+  }
+
   // Cost sum o(x)|psi_x|^2 of this workgroup's amplitudes (FP64, fixed order) and, if
   // lam_out, lam = o psi.  Returns the total on thread 0.
-  static __device__ double cost_and_lam(C* x, C* y, bool lam_out, int cur, const G& g, double* redc)
+  static __device__ double cost_and_lam(C* x, C* y, bool lam_out, int cur, const G& g, uint32_t flip, double* redc)
   {
     const uint32_t tid = threadIdx.x;
     double cs = 0;
 #pragma unroll
     for (int k = 0; k < R; ++k) {
-      const uint32_t xg = g.gidx(lidx<LR>(tid, k, cur));
+      const uint32_t xg = g.gidx(lidx<LR>(tid, k, cur)) ^ flip;
       const int o = g.n - 2 * __popc(xg);
       const double re = x[k].x, im = x[k].y;
       cs += (double)o * (re * re + im * im);
@@ -477,7 +666,7 @@ struct Tile {
     return tot;
   }
 
-  static __device__ void run_whole(const HeaArgs<T>& A, const HeaInst& I, uint32_t b, C* lds, C* zt, double* red,
+  static __device__ void run_whole(const HeaArgs<T>& A, const HeaInst& I, uint32_t b, C* lds, Tab& tb, double* red,
                                    double* redc)
   {
     const uint32_t tid = threadIdx.x;
@@ -486,7 +675,6 @@ struct Tile {
     G g;
     g.init(n, 0, 0, n, 0, 0);
     C x[R], y[R];
-    const C one{1, 0};
     int cur = g.a(0);
 #pragma unroll
     for (int k = 0; k < R; ++k) {
@@ -495,17 +683,20 @@ struct Tile {
     }
     for (int l = 0; l < D; ++l) {
       const uint64_t row = I.par + (uint64_t)l * n;
-      build_tables(zt, g, A.mats + 4 * row, false);
-      sweep_fwd(x, lds, cur, g, A.mats, (int64_t)row, -1, zt, one, false);
+      const Flip f2 = flip_of(A, I, l);
+      build_tables(tb, g, A.gates, (int64_t)row, -1, false, f2);
+      sweep_fwd(x, lds, cur, g, tb, true, false, f2.all);
     }
-    const double cost = cost_and_lam(x, y, grad, cur, g, redc);
+    const uint32_t flip = flip_of(A, I, D - 1).all;
+    const double cost = cost_and_lam(x, y, grad, cur, g, flip, redc);
     if (tid == 0) A.cost[b] = cost;
     if (grad) {
       double* redw = red + (tid >> 6) * SLOTS;
       for (int l = D - 1; l >= 0; --l) {
         const uint64_t row = I.par + (uint64_t)l * n;
-        build_tables(zt, g, A.mats + 4 * row, false);
-        sweep_bwd(x, y, lds, cur, g, A.mats, (int64_t)row, -1, zt, one, false, false, 0, 0, redw);
+        const Flip f2 = flip_of(A, I, l);
+        build_tables(tb, g, A.gates, (int64_t)row, -1, false, f2);
+        sweep_bwd(x, y, lds, cur, g, tb, true, false, f2.all, false, 0, 0, redw);
         __syncthreads();
         for (int q = tid; q < n; q += NT) {
           double st = 0, sp = 0;
@@ -513,8 +704,9 @@ struct Tile {
             st += red[w * SLOTS + M + q];
             sp += red[w * SLOTS + 2 * M + q];
           }
-          A.grad[2 * (row + q)] = st;
-          A.grad[2 * (row + q) + 1] = sp;
+          st *= pre_scale(g, tb, false, q);
+          A.grad[2 * (row + q)] = ((f2.all ^ f2.now) >> q) & 1u ? -st : st;
+          A.grad[2 * (row + q) + 1] = (f2.all >> q) & 1u ? -sp : sp;
         }
       }
     }
@@ -528,10 +720,10 @@ struct Tile {
     }
   }
 
-  static __device__ void run_pass(const HeaArgs<T>& A, const HeaInst& I, int s, uint32_t t, C* lds, C* zt,
+  static __device__ void run_pass(const HeaArgs<T>& A, const HeaInst& I, int s, uint32_t t, C* lds, Tab& tb,
                                   double* red, double* redc)
   {
-    const uint32_t tid = threadIdx.x;
+    const uint32_t tid = thread();
     const int n = I.n, D = I.depth;
     const bool grad = A.flags & kGrad;
     const int j = s <= D ? s : 2 * D - s;
@@ -546,36 +738,46 @@ struct Tile {
     constexpr int L = M - LR;  // load/store layout: consecutive threads, consecutive amplitudes
     C* psi = A.arena + I.psi;
     C* lam = A.arena + I.lam;
+    // amplitude of (thread, register k): a thread's offset and a scalar one
+    const uint32_t at = g.gidx(lidx<LR>(tid, 0, L));
+    const uint32_t tile = g.gidx(0);
+    auto amp = [&](C* v, int k) -> C& { return (v + (g.gidx((uint32_t)k << L) ^ tile))[at]; };
     C x[R], y[R];
     if (s == 0) {
 #pragma unroll
-      for (int k = 0; k < R; ++k) {
-        x[k] = C{0, 0};
-        if (g.gidx(lidx<LR>(tid, k, L)) == 0) x[k].x = 1;
-      }
+      for (int k = 0; k < R; ++k) x[k] = C{0, 0};
+      if (at == 0) x[0].x = 1;
     } else {
 #pragma unroll
-      for (int k = 0; k < R; ++k) x[k] = psi[g.gidx(lidx<LR>(tid, k, L))];
+      for (int k = 0; k < R; ++k) x[k] = amp(psi, k);
     }
     if (s > D) {
 #pragma unroll
-      for (int k = 0; k < R; ++k) y[k] = lam[g.gidx(lidx<LR>(tid, k, L))];
+      for (int k = 0; k < R; ++k) y[k] = amp(lam, k);
     }
-    C f0{1, 0};
-    if (row_pre >= 0) {
-      build_tables(zt, g, A.mats + 4 * row_pre, isB);
-      f0 = deferred_factor(g, A.mats + 4 * row_pre, q0, q1);
-    }
-    const bool has_f0 = q1 > q0;
+    const bool pre = row_pre >= 0, post = row_post >= 0;
+    const Flip f2 = flip_of(A, I, j - 1);
+    build_tables(tb, g, A.gates, row_pre, row_post, isB, f2);
+    const C f0 = deferred_factor(g, tb.rz, q0, q1, f2);
     int cur = L;
     double* redw = red + (tid >> 6) * SLOTS;
-    if (s <= D) sweep_fwd(x, lds, cur, g, A.mats, row_pre, row_post, zt, f0, has_f0);
+    if (s <= D) {
+#pragma unroll
+      for (int k = 0; k < R; ++k) x[k] = cx_mul(x[k], f0);
+      sweep_fwd(x, lds, cur, g, tb, pre, post, f2.all);
+    }
     if (s == D) {
-      const double cs = cost_and_lam(x, y, grad, cur, g, redc);
+      const double cs = cost_and_lam(x, y, grad, cur, g, f2.all, redc);
       if (tid == 0) A.cpart[I.cpart + t] = cs;
     }
-    if (grad && s >= D)
-      sweep_bwd(x, y, lds, cur, g, A.mats, row_pre, row_post, zt, f0, has_f0, isB, q0, q1, redw);
+    if (grad && s >= D) {
+      sweep_bwd(x, y, lds, cur, g, tb, pre, post, f2.all, isB, q0, q1, redw);
+#pragma unroll
+      for (int k = 0; k < R; ++k) {
+        x[k] = cx_mulc(x[k], f0);
+        y[k] = cx_mulc(y[k], f0);
+      }
+    }
     const bool store_x = s < D || (s == D && (grad || (A.flags & kKeep))) || (s > D && s < 2 * D);
     const bool store_y = grad && s >= D && s < 2 * D;
     if ((store_x || store_y) && cur != L) {
@@ -585,47 +787,73 @@ struct Tile {
     }
     if (store_x) {
 #pragma unroll
-      for (int k = 0; k < R; ++k) psi[g.gidx(lidx<LR>(tid, k, L))] = x[k];
+      for (int k = 0; k < R; ++k) amp(psi, k) = x[k];
     }
     if (store_y) {
 #pragma unroll
-      for (int k = 0; k < R; ++k) lam[g.gidx(lidx<LR>(tid, k, L))] = y[k];
+      for (int k = 0; k < R; ++k) amp(lam, k) = y[k];
     }
     if (grad && s >= D) {
       __syncthreads();
-      // slots: [0, gg) dtheta of layer j (post), [M, M + gg) dtheta of layer j-1 (pre),
+      // slots by local bit: [0, M) dtheta of layer j (post), [M, 2M) of layer j-1 (pre);
       // [2M, 2M + n) dphi of layer j-1 (every qubit: pre bits and deferred)
       const int gg = g.lb - g.la;
-      const int nsl = 2 * gg + (row_pre >= 0 ? n : 0);
+      const int nsl = 2 * gg + (pre ? n : 0);
       for (int sl = tid; sl < nsl; sl += NT) {
         int layer, q, kind, slot;
-        if (sl < 2 * gg) {
-          const int which = sl / gg;  // 0: layer j (post), 1: layer j-1 (pre)
-          layer = which ? j - 1 : j;
-          q = g.gq(g.la + sl % gg);
+        uint32_t flip;  // qubits with the opposite sign
+        double f;
+        if (sl < gg) {
+          if (!post) continue;
+          layer = j;
+          q = g.gq(g.la + sl);
           kind = 0;
-          slot = which * M + sl % gg;
+          slot = g.la + sl;
+          f = post_scale(g, tb, slot + 1);
+          flip = f2.all;
+        } else if (sl < 2 * gg) {
+          if (!pre) continue;
+          const int lbit = g.la + sl - gg;
+          layer = j - 1;
+          q = g.gq(lbit);
+          kind = 0;
+          slot = M + lbit;
+          f = pre_scale(g, tb, post, lbit);
+          flip = f2.all ^ f2.now;
         } else {
           layer = j - 1;
           q = sl - 2 * gg;
           kind = 1;
           slot = 2 * M + q;
+          // rotated by this pass (in phase k), or deferred (phase 0)
+          const int lbit = isB ? (q >= M ? q - M + c : -1) : (q < M ? q : -1);
+          const int k = lbit >= 0 ? phase_of(g, lbit) : 0;
+          f = post ? post_scale(g, tb, max(g.nb(k) - 1, g.la)) : 1.0;
+          flip = f2.all;
         }
-        if (layer < 0 || layer >= D) continue;
         double v = 0;
         for (int w = 0; w < NW; ++w) v += red[w * SLOTS + slot];
+        v *= (flip >> q) & 1u ? -f : f;
         A.part[I.part + ((((uint64_t)layer * n + q) * 2 + kind) << I.ntl) + t] = v;
       }
     }
   }
 };
 
+// Wavefronts per SIMD: two workgroups per compute unit, so that one computes while the other
+// loads, stores or waits for a barrier.  Workgroups of 8 wavefronts then have 128 registers per
+// thread, of which the two vectors take 64 (about 40 values that do not change in a pass are kept
+// in scratch memory): 64 registers of 10-22 qubits in complex64 43.4 ms, with one workgroup and 190
+// registers 52.1 ms; in complex128 81.6 against 101.6.  Workgroups of 4 are as fast or faster with
+// the registers that the compiler takes by itself (44.5 against 47.8 ms).
+constexpr int simd_waves(int threads) { return threads >= 512 ? 4 : 2; }
+
 template <typename T, int M, int R>
-__global__ __launch_bounds__((Tile<T, M, R>::NT), 2) void k_hea(HeaArgs<T> A)
+__global__ __launch_bounds__((Tile<T, M, R>::NT), (simd_waves(Tile<T, M, R>::NT))) void k_hea(HeaArgs<T> A)
 {
   using Tl = Tile<T, M, R>;
   __shared__ V<T> lds[1 << M];
-  __shared__ V<T> zt[Tl::KMAX * R];
+  __shared__ typename Tl::Tab tb;
   __shared__ double red[Tl::NW * Tl::SLOTS];
   __shared__ double redc[Tl::NW];
   __shared__ uint32_t sh[2];
@@ -655,13 +883,13 @@ __global__ __launch_bounds__((Tile<T, M, R>::NT), 2) void k_hea(HeaArgs<T> A)
   }
   for (;;) {
     __syncthreads();
-    const uint32_t i = sh[0];
+    const uint32_t i = uniform(sh[0]);
     if (i >= ntask) return;
-    const HeaTask tk = sh_tk;
-    const HeaInst I = sh_in;
+    const HeaTask tk = uniform(sh_tk);
+    const HeaInst I = uniform(sh_in);
     __syncthreads();  // every thread holds its copy before thread 0 stages the next task
     if (I.whole) {
-      Tl::run_whole(A, I, tk.inst, lds, zt, red, redc);
+      Tl::run_whole(A, I, tk.inst, lds, tb, red, redc);
       if (tid == 0) {
         stage(next);
         next = atomicAdd(head, 1u);
@@ -686,10 +914,10 @@ __global__ __launch_bounds__((Tile<T, M, R>::NT), 2) void k_hea(HeaArgs<T> A)
         sh[1] = ok;
       }
       __syncthreads();
-      const bool ok = sh[1];
+      const bool ok = uniform(sh[1]);
       if (ok) {
         if (tk.step > 0) acquire_tiles();
-        Tl::run_pass(A, I, tk.step, tk.tile, lds, zt, red, redc);
+        Tl::run_pass(A, I, tk.step, tk.tile, lds, tb, red, redc);
       }
       __syncthreads();  // sh[1] read by all before it is reused
       if (tid == 0) {
@@ -729,20 +957,58 @@ __global__ void k_hea_zero(uint32_t* p, uint32_t n)
   if (i < n) p[i] = 0;
 }
 
-// Per (layer, qubit) pair: (cos theta/2, sin theta/2) and (cos phi/2, sin phi/2), computed in
-// FP64 and rounded once to T (RY = [[c, -s], [s, c]], RZ = diag(e^{-i phi/2}, e^{i phi/2})).
+// The gate factors of every (layer, qubit) pair, computed in FP64 and rounded once to T
+// (RY = [[c, -s], [s, c]], RZ = diag(e^{-i phi/2}, e^{i phi/2})); tan is that of the values.
 template <typename T>
-__global__ void k_hea_mats(const double* __restrict__ ang, V<T>* __restrict__ mats, uint64_t npairs)
+__global__ void k_hea_gates(const double* __restrict__ ang, HeaGate<T>* __restrict__ gates, uint64_t npairs)
 {
   const uint64_t p = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x;
   if (p >= npairs) return;
   double s, c, sp, cp;
   sincos(0.5 * ang[2 * p], &s, &c);
   sincos(0.5 * ang[2 * p + 1], &sp, &cp);
-  mats[4 * p + 0] = V<T>{(T)c, (T)s};
-  mats[4 * p + 1] = V<T>{(T)cp, (T)sp};
-  mats[4 * p + 2] = V<T>{0, 0};
-  mats[4 * p + 3] = V<T>{0, 0};
+  const bool far = fabs(s) > fabs(c);
+  const double kap = far ? s : c;
+  gates[p] = HeaGate<T>{(T)((far ? -c : s) / kap), (T)(far ? 1 : 0), {(T)(kap * cp), (T)(kap * sp)}, 1 / (kap * kap), 0};
+}
+
+// One wavefront per instance, one lane per qubit: flips after every layer, and tan for the bits.
+template <typename T>
+__global__ void k_hea_flips(const HeaInst* __restrict__ inst, HeaGate<T>* gates, uint32_t* flips)
+{
+  const HeaInst& I = inst[blockIdx.x];
+  const uint32_t q = threadIdx.x;
+  const bool on = q < I.n;
+  HeaGate<T>* g = gates + I.par + (on ? q : 0);
+  bool flip = false;
+  constexpr uint32_t B = 8;  // layers whose gates are in flight together
+  for (uint32_t l0 = 0; l0 < I.depth; l0 += B) {
+    T t[B], far[B];
+#pragma unroll
+    for (uint32_t i = 0; i < B; ++i) {
+      const HeaGate<T>& h = g[(uint64_t)min(l0 + i, I.depth - 1) * I.n];
+      t[i] = h.tan;
+      far[i] = h.far;
+    }
+#pragma unroll
+    for (uint32_t i = 0; i < B; ++i) {
+      if (l0 + i >= I.depth) break;
+      if (on && flip) g[(uint64_t)(l0 + i) * I.n].tan = -t[i];
+      flip ^= on && far[i] != 0;
+      const uint64_t m = __ballot(flip);
+      if (q == 0) flips[I.lay + l0 + i] = (uint32_t)m;
+    }
+  }
+}
+
+// The kept state of an instance with every amplitude at its values, into lam.
+template <typename T>
+__global__ void k_hea_place(const HeaInst* __restrict__ inst, V<T>* arena, const uint32_t* __restrict__ flips)
+{
+  const uint32_t flip = inst->depth ? flips[inst->lay + inst->depth - 1] : 0;
+  const uint64_t N = uint64_t(1) << inst->n;
+  for (uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; i < N; i += (uint64_t)gridDim.x * blockDim.x)
+    arena[inst->lam + i] = arena[inst->psi + (i ^ flip)];
 }
 
 // One block per (tiled instance, layer): thread q sums the tile partials of qubit q in
@@ -777,8 +1043,7 @@ __global__ void k_hea_epi(const HeaInst* __restrict__ inst, const uint2* __restr
 struct Variant {
   int M, R, test;
 };
-// Every variant keeps its registers within 256 VGPRs (two waves per SIMD); tiles that
-// needed the accumulation registers as spill space ran at one wave per SIMD and are left out.
+// Tiles whose two vectors leave room for two workgroups per compute unit, in registers and LDS.
 constexpr Variant kVar64[] = {{13, 16, 0}, {12, 16, 0}, {12, 8, 0}, {8, 4, 1}};
 constexpr Variant kVar128[] = {{12, 8, 0}, {11, 8, 0}, {10, 8, 0}, {8, 4, 1}};
 constexpr int kNumVar = 4;
@@ -789,10 +1054,15 @@ template <typename T, int M, int R>
 hipError_t launch_t(const HeaArgs<T>& a, int workers_per_cu, int cus, hipStream_t st)
 {
   constexpr int NT = Tile<T, M, R>::NT;
-  int fit = 0;
-  hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&fit, k_hea<T, M, R>, NT, 0);
+  // Workgroups that fit a compute unit: 160 KB of LDS, and per SIMD 512 registers (in steps of 8)
+  // and 8 wavefronts.  (hipOccupancyMaxActiveBlocksPerMultiprocessor reckons with 64 KB of LDS,
+  // and workgroups that it leaves out do not leave compute units evenly filled: the dispatcher
+  // packs a smaller grid on some of them.)
+  hipFuncAttributes fa;
+  hipError_t e = hipFuncGetAttributes(&fa, reinterpret_cast<const void*>(k_hea<T, M, R>));
   if (e != hipSuccess) return e;
-  fit = std::max(fit, 1);
+  const int waves = 4 * std::min(8, 512 / std::max(8, (fa.numRegs + 7) / 8 * 8));
+  const int fit = std::max(1, std::min((int)(160 * 1024 / fa.sharedSizeBytes), waves * 64 / NT));
   const int w = workers_per_cu > 0 ? std::min(workers_per_cu, fit) : fit;
   hipLaunchKernelGGL((k_hea<T, M, R>), dim3(std::max(1, w * cus)), dim3(NT), 0, st, a);
   return hipGetLastError();
@@ -840,7 +1110,8 @@ struct iqsh_hea {
   hipStream_t cap = nullptr;  // private stream for graph capture
 
   void* arena = nullptr;
-  void* mats = nullptr;
+  void* gates = nullptr;
+  uint32_t* flips = nullptr;
   double* ang = nullptr;
   double* grad = nullptr;
   double* cost = nullptr;
@@ -860,6 +1131,7 @@ struct iqsh_hea {
   size_t epi_cap = 0;
 
   int built_mode = -1;  // flags (GRAD | KEEP) the schedule was built for
+  int work_per_cu = 64;  // workgroups per compute unit that find work (see build)
   uint32_t ntask = 0, nepi = 0, nctl = 0;
   hipGraph_t graph = nullptr;
   hipGraphExec_t gexec = nullptr;
@@ -904,7 +1176,7 @@ int build(iqsh_hea* h, int mode)
   const bool grad = mode & kGrad;
   std::vector<HeaInst> I(h->count);
   uint64_t part = 0, cpart = 0;
-  uint32_t arrive = 0;
+  uint32_t arrive = 0, lay = 0;
   std::vector<int> tiled, whole;
   int smax = 0;
   for (int b = 0; b < h->count; ++b) {
@@ -916,6 +1188,8 @@ int build(iqsh_hea* h, int mode)
     x.psi = h->soff[b];
     x.lam = h->soff[b] + (uint64_t(1) << h->n[b]);
     x.par = h->par[b];
+    x.lay = lay;
+    lay += (uint32_t)h->d[b];
     if (x.whole) {
       whole.push_back(b);
       continue;
@@ -966,6 +1240,7 @@ int build(iqsh_hea* h, int mode)
   std::vector<HeaTask> tasks;
   std::vector<uint32_t> qoff(kQueues + 1, 0);
   const int order = h->tune.order;
+  uint64_t round = 0;  // most tile tasks of one round in a queue
   for (int qi = 0; qi < kQueues; ++qi) {
     qoff[qi] = (uint32_t)tasks.size();
     std::vector<int> tq, wq;
@@ -973,6 +1248,9 @@ int build(iqsh_hea* h, int mode)
       if (qof[b] == qi) tq.push_back(b);
     for (int b : whole)
       if (qof[b] == qi) wq.push_back(b);
+    uint64_t tiles = 0;
+    for (int b : tq) tiles += uint64_t(1) << I[b].ntl;
+    round = std::max(round, tiles);
     auto push_whole = [&](size_t lo, size_t hi) {
       for (size_t i = lo; i < hi; ++i) tasks.push_back(HeaTask{(uint32_t)wq[i], 0, 0});
     };
@@ -1046,6 +1324,13 @@ int build(iqsh_hea* h, int mode)
   IQSI_TRY(hipStreamSynchronize(st));
   h->qlen.assign(kQueues, 0);
   for (int qi = 0; qi < kQueues; ++qi) h->qlen[qi] = qoff[qi + 1] - qoff[qi];
+  // A task waits for the tiles of the round before it: with as many workgroups as half a round has
+  // tasks these have finished by the time it is taken, further ones would only poll (one, two and
+  // three workgroups per compute unit, complex64: 64 registers of 16 qubits as 128 tasks of 2^12
+  // amplitudes per XCD and round 4.4, 2.7 and 6.0 ms, as 64 of 2^13 3.4 and 5.0; complex128: as 256
+  // of 2^11 8.2, 5.0 and 4.5).
+  const uint64_t half = 2 * (uint64_t)h->cus / kQueues;
+  h->work_per_cu = round ? (int)std::min<uint64_t>(64, (round + half - 1) / half) : 64;
   h->ntask = (uint32_t)tasks.size();
   h->nepi = (uint32_t)epi.size();
   h->nctl = kCtlArrive + arrive;
@@ -1064,7 +1349,8 @@ int enqueue_t(iqsh_hea* h, int mode, hipStream_t st)
   a.flags = (uint32_t)mode;
   a.ctl = h->ctl;
   a.arena = (V<T>*)h->arena;
-  a.mats = (const V<T>*)h->mats;
+  a.gates = (const HeaGate<T>*)h->gates;
+  a.flips = h->flips;
   a.grad = h->grad;
   a.cost = h->cost;
   a.part = h->part;
@@ -1073,10 +1359,13 @@ int enqueue_t(iqsh_hea* h, int mode, hipStream_t st)
   a.wait_extra = h->wait_extra;
   hipLaunchKernelGGL(k_hea_zero, dim3((h->nctl + 255) / 256), dim3(256), 0, st, h->ctl, h->nctl);
   IQSI_TRY(hipGetLastError());
-  hipLaunchKernelGGL(k_hea_mats<T>, dim3((unsigned)((h->npairs + 255) / 256)), dim3(256), 0, st, (const double*)h->ang,
-                     (V<T>*)h->mats, h->npairs);
+  hipLaunchKernelGGL(k_hea_gates<T>, dim3((unsigned)((h->npairs + 255) / 256)), dim3(256), 0, st, (const double*)h->ang,
+                     (HeaGate<T>*)h->gates, h->npairs);
   IQSI_TRY(hipGetLastError());
-  IQSI_TRY(launch_var<T>(h->tune.variant, a, h->tune.workers_per_cu, h->cus, st));
+  hipLaunchKernelGGL(k_hea_flips<T>, dim3((unsigned)h->count), dim3(64), 0, st, (const HeaInst*)h->inst,
+                     (HeaGate<T>*)h->gates, h->flips);
+  IQSI_TRY(hipGetLastError());
+  IQSI_TRY(launch_var<T>(h->tune.variant, a, h->tune.workers_per_cu > 0 ? h->tune.workers_per_cu : h->work_per_cu, h->cus, st));
   if (h->nepi) {
     hipLaunchKernelGGL(k_hea_epi, dim3(h->nepi), dim3(64), 0, st, (const HeaInst*)h->inst, (const uint2*)h->epi,
                        (const double*)h->part, (const double*)h->cpart, h->grad, h->cost,
@@ -1163,7 +1452,11 @@ int iqsh_hea_create(int dtype, int count, const int* nq, const int* depth, const
   };
   int rc;
   if ((rc = alloc(&h->arena, h->arena_amps * h->esz(), "batch states"))) return bail(rc);
-  if ((rc = alloc(&h->mats, h->npairs * 4 * h->esz(), "gate matrices"))) return bail(rc);
+  const size_t gate = dtype == IQSH_C128 ? sizeof(HeaGate<double>) : sizeof(HeaGate<float>);
+  if ((rc = alloc(&h->gates, h->npairs * gate, "gate factors"))) return bail(rc);
+  size_t layers = 0;
+  for (int d : h->d) layers += (size_t)d;
+  if ((rc = alloc((void**)&h->flips, layers * sizeof(uint32_t), "inverted qubits"))) return bail(rc);
   if ((rc = alloc((void**)&h->ang, h->npairs * 2 * sizeof(double), "angles"))) return bail(rc);
   if ((rc = alloc((void**)&h->grad, h->npairs * 2 * sizeof(double), "gradients"))) return bail(rc);
   if ((rc = alloc((void**)&h->cost, (size_t)count * sizeof(double), "costs"))) return bail(rc);
@@ -1199,7 +1492,7 @@ int iqsh_hea_destroy(iqsh_hea_handle h)
   if (!h) return IQSH_OK;
   (void)hipStreamSynchronize(iqsi::stream());
   drop_graph(h);
-  void* bufs[] = {h->arena, h->mats, h->ang, h->grad, h->cost, h->part, h->cpart, h->inst, h->task, h->ctl, h->epi,
+  void* bufs[] = {h->arena, h->gates, h->flips, h->ang, h->grad, h->cost, h->part, h->cpart, h->inst, h->task, h->ctl, h->epi,
                   h->qoff};
   for (void* p : bufs)
     if (p) (void)hipFree(p);
@@ -1347,7 +1640,17 @@ int iqsh_hea_state(iqsh_hea_handle h, int b, void* host)
   if (b < 0 || b >= h->count || !host) return fail(IQSH_ERR_ARG, "bad instance %d or null buffer", b);
   if (!h->kept) return fail(IQSH_ERR_ARG, "no state kept: run with IQSH_HEA_KEEP_STATE first");
   hipStream_t st = iqsi::stream();
-  IQSI_TRY(hipMemcpyAsync(host, (const char*)h->arena + h->soff[b] * h->esz(), (size_t(1) << h->n[b]) * h->esz(),
+  // the bits that the last layer left inverted: amplitudes in order into the second vector
+  const dim3 grid((unsigned)std::min<uint64_t>((uint64_t(1) << h->n[b]) / 256 + 1, 8u * (unsigned)h->cus));
+  if (h->dtype == IQSH_C128)
+    hipLaunchKernelGGL(k_hea_place<double>, grid, dim3(256), 0, st, (const HeaInst*)h->inst + b, (V<double>*)h->arena,
+                       (const uint32_t*)h->flips);
+  else
+    hipLaunchKernelGGL(k_hea_place<float>, grid, dim3(256), 0, st, (const HeaInst*)h->inst + b, (V<float>*)h->arena,
+                       (const uint32_t*)h->flips);
+  IQSI_TRY(hipGetLastError());
+  const uint64_t amps = uint64_t(1) << h->n[b];
+  IQSI_TRY(hipMemcpyAsync(host, (const char*)h->arena + (h->soff[b] + amps) * h->esz(), amps * h->esz(),
                           hipMemcpyDeviceToHost, st));
   IQSI_TRY(hipStreamSynchronize(st));
   return IQSH_OK;

@@ -217,3 +217,37 @@ def test_dependency_wait_gives_up_cleanly():
     c, g = b.evaluate(ang)
     assert np.array_equal(c, c0) and np.array_equal(g, g0)
     b.close()
+
+
+@pytest.mark.parametrize("dtype,tol", [("c128", 1e-12), ("c64", 1e-5)])
+@pytest.mark.parametrize("theta", [0.5 * math.pi, math.pi, -0.75 * math.pi, 2.0 * math.pi, 3.5 * math.pi])
+def test_rotations_past_a_quarter_turn(dtype, tol, theta):
+    """Angles at which the rotation's tangent is 1, undefined or of either sign, the same on every
+    qubit and layer (so bits stay inverted through several layers) and with two neighbours of
+    another kind: states, costs and gradients, whole registers and tiles of 2^8."""
+    nq, dp = [3, 9, 10, 12], [3, 2, 5, 1]
+    off = param_offsets(nq, dp)
+    ang = np.full(int(off[-1]), theta)
+    ang[1::2] = np.linspace(-3.0, 3.0, len(ang) // 2)  # phi
+    ang[0::10] = 0.3
+    ang[4::14] = 2.0
+    for variant in (TEST_VARIANT, 0):
+        b = HeaBatch(nq, dp, dtype, tune=(variant, 0, 0))
+        b.set_angles(ang)
+        b.run(grad=False, keep_state=True)
+        cost = b.results(grad=False)
+        for i, (n, d) in enumerate(zip(nq, dp)):
+            st_ref, c_ref = oracle_run(n, d, ang[off[i]:off[i + 1]], "dp")
+            err = np.max(np.abs(b.state(i).astype(np.complex128) - st_ref))
+            assert err < tol and abs(cost[i] - c_ref) < 10 * n * tol, (i, n, d, err, cost[i] - c_ref)
+        b.run(grad=True)
+        _, grad = b.results()
+        shifts = [np.where(np.arange(len(ang)) == k, 0.5 * math.pi, 0.0) for k in (0, 4, 7, len(ang) - 2, len(ang) - 1)]
+        for s in shifts:  # dC/da = (C(a + pi/2) - C(a - pi/2)) / 2
+            k = int(np.argmax(s))
+            i = int(np.searchsorted(off, k, side="right")) - 1
+            n, d, (lo, hi) = nq[i], dp[i], (off[i], off[i + 1])
+            up = oracle_run(n, d, (ang + s)[lo:hi], "dp")[1]
+            dn = oracle_run(n, d, (ang - s)[lo:hi], "dp")[1]
+            assert abs(grad[k] - 0.5 * (up - dn)) < 10 * n * tol, (k, grad[k], 0.5 * (up - dn))
+        b.close()
