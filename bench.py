@@ -575,7 +575,7 @@ def qaoa_measure(n: int, p: int, full: bool, torch):
 
 def brick_fused_measure(sv, layers, torch):
     """The timed brick circuit again through the drop-in with fusion on (TurnOnFusion,
-    <= 5-position blocks on the matrix cores): gates/s of the whole queued-and-flushed run
+    passes of <= 4-position blocks on the matrix cores): gates/s of the whole queued-and-flushed run
     and its distance from the unfused state `sv` (complex128, same gates)."""
     import ctypes as C
 
@@ -602,7 +602,7 @@ def brick_fused_measure(sv, layers, torch):
     call("iqsh_maxabsdiff", C.c_void_p(reg.DeviceHandle()), sv.handle, 1.0, 0.0, C.byref(mx))
     del reg
     return {"workload": f"the timed {n}-qubit brick layers ({len(c.ops)} gates) through the drop-in with "
-                        f"TurnOnFusion, <= 5-position blocks; not the headline value (that is one pass per gate)",
+                        f"TurnOnFusion (blocks: passes over the state); not the headline value (that is one pass per gate)",
             "gates": gates, "blocks": blocks, "s": t, "gates_per_s": gates / t,
             "max_abs_diff_vs_unfused": mx.value}
 

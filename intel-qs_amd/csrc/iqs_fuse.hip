@@ -12,13 +12,14 @@
 // What bounds it (complex64, 30 qubits, 120 random gates, 7 passes of 4 blocks): a pass takes 4.5
 // ms, of which its loads and stores alone are 3.5 ms (4.9 TB/s of 2S in 128-byte rows) and its
 // matrix products alone 2.5 ms (48 products per block and amplitude; the matrix cores are
-// busy 0.56 of the time); the phases of the 5 workgroups on a CU overlap in part.  67.1 ms as
-// 20 passes of 5-position blocks -> 31.4 ms.  complex128, 29 qubits, 100 gates: 27.7 ms in 6
+// busy 0.56 of the time); the phases of the 5 workgroups on a CU overlap in part.  61.3 ms
+// as 20 passes of 5-position blocks -> 33.1 ms.  complex128, 29 qubits, 100 gates: 27.7 ms in 6
 // passes.  On registers of 20 qubits and below a workgroup per CU runs alone, and a block
 // costs about 4 us (exchange and its barriers 2, products 1.3): 10 brick layers of 20 qubits
-// 794 -> 158 us with the host's planning (65 us).  The error against 64 bits is below that of
-// the 5-position blocks (complex64, 200 random gates on 24 qubits 7.5e-7 against 8.2e-7): sums of
-// 16 terms instead of 32.
+// 790 -> 145 us with the host's planning (65 us).  Error against 64 bits: complex64, 200 random
+// gates on 24 qubits, 7.5e-7 (5-position blocks 8.2e-7: sums of 32 terms instead of 16);
+// complex128, the 20-qubit brick, 4.6e-15 (2.5e-15: fewer blocks); with four real products
+// instead of three the same to 3%.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

@@ -22,7 +22,7 @@
 // are each under a third of that time.  A layer takes 4.73 ms forward and 9.57 ms adjoint
 // (7.45 and 18.2 with one lane pass over 8 positions and register passes over 5 and 4 above,
 // which moved the state 5 and 6 times); 25 qubits complex64, weighted: 8.45 -> 4.6 ms for
-// cost and gradient at p = 4; 14 qubits complex128: 700 -> 380 us at p = 6.
+// cost and gradient at p = 4; 14 qubits complex128: 700 -> 375 us at p = 6 (201 in one call).
 //
 // Adjoint: the gates of a layer act on different qubits, so each generator G_q commutes
 // with every gate of the layer except its own, and inserting G_q after U_q equals inserting

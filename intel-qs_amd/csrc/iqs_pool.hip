@@ -91,8 +91,8 @@ int mats_slot(size_t bytes, int* slot)
 }
 
 // Where a kernel finds the matrix of a state: in device memory, or in its own arguments for
-// pools whose matrices fit them (no copy at all: a noise gate on 32 states of 16 qubits 24 ->
-// 8 us, against 24 -> 14 with an asynchronous copy).
+// pools whose matrices fit them (no copy at all: a noise gate on 32 states of 16 qubits 32.7 ->
+// 8.9 us).
 constexpr size_t kArgBytes = 2048;
 template <typename MT>
 struct MatsAt {
