@@ -16,15 +16,18 @@
 // as 20 passes of 5-position blocks -> 33.1 ms.  complex128, 29 qubits, 100 gates: 27.7 ms in 6
 // passes.  On registers of 20 qubits and below a workgroup per CU runs alone, and a block
 // costs about 4 us (exchange and its barriers 2, products 1.3): 10 brick layers of 20 qubits
-// 790 -> 145 us with the host's planning (65 us).  Error against 64 bits: complex64, 200 random
-// gates on 24 qubits, 7.5e-7 (5-position blocks 8.2e-7: sums of 32 terms instead of 16);
-// complex128, the 20-qubit brick, 4.6e-15 (2.5e-15: fewer blocks); with four real products
-// instead of three the same to 3%.
+// 790 -> 141 us with the host's planning (65 us).  Error against 64 bits: complex64, 200 random
+// gates on 24 qubits, 7.5e-7 (5-position blocks 8.2e-7: sums of 32 terms instead of 16), with four
+// real products instead of three 0.9 of that at 1.1 times the time; complex128, the 20-qubit
+// brick, 1.9e-15 (5-position blocks 2.5e-15).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
 #include <cstring>
+#include <exception>
+#include <memory>
 #include <mutex>
+#include <utility>
 #include <vector>
 
 #include "../../include/iqs_hip.h"
@@ -38,95 +41,182 @@ namespace {
 // ---------------------------------------------------------------------------------------
 // Planning
 
-// a := b a as d x d complex matrices (interleaved parts), b acting after a.
-void mul_after(double* a, const double* b, unsigned d)
-{
-  double r[32];
-  for (unsigned i = 0; i < d; ++i)
-    for (unsigned j = 0; j < d; ++j) {
-      double re = 0, im = 0;
-      for (unsigned k = 0; k < d; ++k) {
-        const double *x = b + 2 * (i * d + k), *y = a + 2 * (k * d + j);
-        re += x[0] * y[0] - x[1] * y[1];
-        im += x[0] * y[1] + x[1] * y[0];
+// A D x D gate while others are multiplied into it.  A block's matrix acts alike on every amplitude,
+// so the roundings of these products do not average out as those of the amplitudes do, but add up
+// to a drift of the norm; they are rounded once, at the end.  Until then an entry is h + l with h a
+// multiple of 2^-24: for entries up to 1 products of two h and their sums are exact, and what
+// involves an l is small enough that its rounding does not count.  (Entries of any size are as
+// good as plain products at least.  The same in long double takes twice as long.)  10 brick layers
+// of 20 qubits, error against 64 bits: 1.9e-15, with plain products 4.1e-15, in the same 141 us.
+template <int D>
+struct Wide {
+  double h[2][D][D], l[2][D][D];  // real and imaginary parts
+
+  Wide() = default;
+  explicit Wide(const double* m)
+  {
+    for (int r = 0; r < D; ++r)
+      for (int c = 0; c < D; ++c)
+        for (int p = 0; p < 2; ++p) put(p, r, c, *m++, 0);
+  }
+  void put(int p, int r, int c, double hi, double lo)
+  {
+    constexpr double k = 1.5 * (1 << 28);  // sums with k are multiples of 2^-24
+    const double v = hi + lo;
+    h[p][r][c] = (v + k) - k;
+    l[p][r][c] = (hi - h[p][r][c]) + lo;
+  }
+  Wide operator*(const Wide& y) const
+  {
+    Wide z;
+    for (int r = 0; r < D; ++r) {
+      double h0[D] = {}, h1[D] = {}, l0[D] = {}, l1[D] = {};
+      for (int k = 0; k < D; ++k) {
+        const double a = h[0][r][k], b = h[1][r][k], al = l[0][r][k], bl = l[1][r][k];
+        if (a == 0 && b == 0 && al == 0 && bl == 0) continue;
+        for (int c = 0; c < D; ++c) {
+          const double u = y.h[0][k][c], v = y.h[1][k][c], ul = y.l[0][k][c], vl = y.l[1][k][c];
+          h0[c] += a * u - b * v;
+          h1[c] += a * v + b * u;
+          l0[c] += (a * ul - b * vl) + (al * (u + ul) - bl * (v + vl));
+          l1[c] += (a * vl + b * ul) + (al * (v + vl) + bl * (u + ul));
+        }
       }
-      r[2 * (i * d + j)] = re;
-      r[2 * (i * d + j) + 1] = im;
+      for (int c = 0; c < D; ++c) {
+        z.put(0, r, c, h0[c], l0[c]);
+        z.put(1, r, c, h1[c], l1[c]);
+      }
     }
-  std::memcpy(a, r, 2 * d * d * sizeof(double));
-}
+    return z;
+  }
+  void write(double* m) const
+  {
+    for (int r = 0; r < D; ++r)
+      for (int c = 0; c < D; ++c)
+        for (int p = 0; p < 2; ++p) *m++ = h[p][r][c] + l[p][r][c];
+  }
+};
 
-// m4 := the 2x2 m2 on index bit `bit` of a 4x4.
-void widen(const double* m2, unsigned bit, double* m4)
+// hi (x) lo: index bit 1 under hi, bit 0 under lo; one of them may be null, for the identity.
+Wide<4> kron(const Wide<2>* hi, const Wide<2>* lo)
 {
-  std::memset(m4, 0, 32 * sizeof(double));
-  for (unsigned i = 0; i < 4; ++i)
-    for (unsigned j = 0; j < 4; ++j)
-      if (((i ^ j) & ~(1u << bit)) == 0)
-        std::memcpy(m4 + 2 * (i * 4 + j), m2 + 2 * (((i >> bit) & 1) * 2 + ((j >> bit) & 1)), 2 * sizeof(double));
+  Wide<4> z;
+  if (!hi || !lo) {
+    std::memset(&z, 0, sizeof z);
+    const Wide<2>& x = hi ? *hi : *lo;
+    const int s = hi ? 2 : 1, o = 3 - s;  // strides of x's index and of the other
+    for (int p = 0; p < 2; ++p)
+      for (int i = 0; i < 2; ++i)
+        for (int j = 0; j < 2; ++j)
+          for (int k = 0; k < 2; ++k) {
+            z.h[p][i * s + k * o][j * s + k * o] = x.h[p][i][j];
+            z.l[p][i * s + k * o][j * s + k * o] = x.l[p][i][j];
+          }
+    return z;
+  }
+  for (int i = 0; i < 2; ++i)
+    for (int j = 0; j < 2; ++j) {
+      const double a = hi->h[0][i][j], b = hi->h[1][i][j], al = hi->l[0][i][j], bl = hi->l[1][i][j];
+      for (int r = 0; r < 2; ++r)
+        for (int c = 0; c < 2; ++c) {
+          const double u = lo->h[0][r][c], v = lo->h[1][r][c], ul = lo->l[0][r][c], vl = lo->l[1][r][c];
+          z.put(0, 2 * i + r, 2 * j + c, a * u - b * v, (a * ul - b * vl) + (al * (u + ul) - bl * (v + vl)));
+          z.put(1, 2 * i + r, 2 * j + c, a * v + b * u, (a * vl + b * ul) + (al * (v + vl) + bl * (u + ul)));
+        }
+    }
+  return z;
 }
 
-// The list with every one-qubit gate multiplied into the gate before it on its position (or,
-// as the first gate there, into the two-qubit gate after it), and consecutive two-qubit gates
-// on the same pair multiplied together: a small product each, instead of one with a block's
+// The list with the one-qubit gates on a position multiplied together and into the two-qubit
+// gate that follows there (after the last one, into that), and consecutive two-qubit gates on the
+// same pair multiplied together: a small product each, instead of one with a block's
 // matrix.  A brick layer of 20 qubits (H, rotation on every qubit, 9 or 10 CNOTs) becomes its 9
 // or 10 two-qubit gates.
 std::vector<iqsh_gate> merge_gates(const iqsh_gate* g, int ngates)
 {
   std::vector<iqsh_gate> out;
-  int last[64];  // last gate on each position
+  // Per position: the last two-qubit gate of the list there, and the one-qubit gates since, with
+  // their own place in the list where none is before them (-1: none).  The matrix of a two-qubit
+  // gate that is still last on a position is in `pair` at one of its positions, home[gate].
+  int last[64], place[64];
+  bool some[64] = {};
+  const std::unique_ptr<Wide<2>[]> lone(new Wide<2>[64]);
+  const std::unique_ptr<Wide<4>[]> pair(new Wide<4>[64]);
+  std::vector<uint8_t> home;
   std::fill(last, last + 64, -1);
-  std::vector<char> gone;
+  std::fill(place, place + 64, -1);
+  auto add = [&](const iqsh_gate& x) {
+    out.emplace_back();
+    out.back().np = x.np;
+    out.back().p[0] = x.p[0];
+    out.back().p[1] = x.p[1];
+    home.push_back((uint8_t)x.p[0]);
+    return (int)out.size() - 1;
+  };
+  // The one-qubit gates on q, which go into a two-qubit gate; null if there are none.
+  auto take = [&](unsigned q) -> const Wide<2>* {
+    if (!some[q]) return nullptr;
+    if (place[q] >= 0) out[place[q]].np = 0;
+    place[q] = -1;
+    some[q] = false;
+    return &lone[q];
+  };
+  // Another gate becomes the last one on q.
+  auto leave = [&](unsigned q) {
+    const int i = last[q];
+    if (i < 0) return;
+    const unsigned other = out[i].p[out[i].p[0] == q];
+    if (last[other] != i) pair[q].write(out[i].m);
+    else if (home[i] == q) {
+      pair[other] = pair[q];
+      home[i] = (uint8_t)other;
+    }
+  };
   for (int i = 0; i < ngates; ++i) {
     const iqsh_gate& x = g[i];
-    double w[32];
+    const unsigned a = x.p[0], b = x.p[1];
     if (x.np == 1) {
-      const int l = last[x.p[0]];
-      if (l >= 0) {
-        iqsh_gate& y = out[l];
-        if (y.np == 1) mul_after(y.m, x.m, 2);
-        else {
-          widen(x.m, y.p[0] == x.p[0] ? 1 : 0, w);
-          mul_after(y.m, w, 4);
-        }
-        continue;
+      if (some[a]) lone[a] = Wide<2>(x.m) * lone[a];
+      else {
+        lone[a] = Wide<2>(x.m);
+        some[a] = true;
+        if (last[a] < 0) place[a] = add(x);
       }
-    } else {
-      const int l0 = last[x.p[0]], l1 = last[x.p[1]];
-      if (l0 >= 0 && l0 == l1) {
-        iqsh_gate& y = out[l0];
-        if (y.p[0] == x.p[0]) std::memcpy(w, x.m, sizeof w);
-        else  // the same pair the other way round: exchange the index bits
-          for (unsigned r = 0; r < 4; ++r)
-            for (unsigned c = 0; c < 4; ++c) {
-              const unsigned rr = (r >> 1) | ((r & 1) << 1), cc = (c >> 1) | ((c & 1) << 1);
-              std::memcpy(w + 2 * (r * 4 + c), x.m + 2 * (rr * 4 + cc), 2 * sizeof(double));
-            }
-        mul_after(y.m, w, 4);
-        continue;
-      }
+      continue;
     }
-    out.push_back(x);
-    gone.push_back(0);
-    iqsh_gate& y = out.back();
-    for (unsigned j = 0; j < x.np; ++j) {
-      const int l = last[x.p[j]];
-      if (x.np == 2 && l >= 0 && out[l].np == 1) {  // y := y (before it, the lone gate)
-        widen(out[l].m, j == 0 ? 1 : 0, w);
-        mul_after(w, y.m, 4);
-        std::memcpy(y.m, w, sizeof w);
-        gone[l] = 1;
-      }
-      last[x.p[j]] = (int)out.size() - 1;
+    Wide<4> m(x.m);
+    const Wide<2>*ma = take(a), *mb = take(b);
+    if (ma || mb) m = m * kron(ma, mb);
+    if (last[a] >= 0 && last[a] == last[b]) {
+      if (out[last[a]].p[0] != a)  // the same pair the other way round: exchange the index bits
+        for (auto* e : {m.h, m.l})
+          for (int p = 0; p < 2; ++p) {
+            for (int v = 0; v < 4; ++v) std::swap(e[p][1][v], e[p][2][v]);
+            for (int v = 0; v < 4; ++v) std::swap(e[p][v][1], e[p][v][2]);
+          }
+      Wide<4>& z = pair[home[last[a]]];
+      z = m * z;
+      continue;
     }
+    leave(a);
+    leave(b);
+    last[a] = last[b] = add(x);
+    pair[a] = m;
   }
-  size_t n = 0;
-  for (size_t i = 0; i < out.size(); ++i)
-    if (!gone[i]) {
-      if (n != i) out[n] = out[i];
-      ++n;
+  for (unsigned q = 0; q < 64; ++q) {
+    if (last[q] < 0) {
+      if (some[q]) lone[q].write(out[place[q]].m);
+      continue;
     }
-  out.resize(n);
+    iqsh_gate& x = out[last[q]];
+    if (home[last[q]] != q) continue;
+    const bool first = x.p[0] == q;
+    const unsigned other = x.p[first];
+    const Wide<2>*mq = take(q), *mo = last[other] == last[q] ? take(other) : nullptr;
+    if (mq || mo) pair[q] = kron(first ? mq : mo, first ? mo : mq) * pair[q];
+    pair[q].write(x.m);
+  }
+  out.erase(std::remove_if(out.begin(), out.end(), [](const iqsh_gate& x) { return x.np == 0; }), out.end());
   return out;
 }
 

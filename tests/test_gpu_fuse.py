@@ -85,3 +85,34 @@ def test_bad_gate_lists_are_refused():
         with pytest.raises(IqsError):
             call("iqsh_apply_gates", sv.handle, 1, C.byref(g), block, None)
     assert sv.prob1(0) == 1.0 and sv.norm2() == 1.0
+
+
+@pytest.mark.parametrize("seed", [1, 2])
+def test_double_precision_error_of_merged_gates(seed):
+    """Forty brick layers of 14 qubits (H, rotation, CNOT ladder; 74 blocks of 4 positions,
+    96 allowed for) against the same gates in 80-bit arithmetic.  Tolerance (2-norm of a state of norm 1): a block
+    rounds its matrix and, per amplitude, sums of 16 terms in three real products, 6 units of 2^-53 at
+    most, independent from block to block: sqrt(96) * 6 * 2^-53.  (Roundings that all amplitudes
+    share add up with the number of gates instead.)"""
+    from iqs_amd import gates as G
+    n, r = 14, SplitMix64(seed)
+    c = Circuit(n, precision="dp", init="plus")
+    want = np.full(1 << n, 2.0 ** (-n / 2), dtype=np.clongdouble)
+    for layer in range(40):
+        mats = [(q, m) for rnd in (lambda: G.H, lambda: (G.rx, G.ry, G.rz)[r.randint(3)](r.uniform(0.0, 6.28)))
+                for q in range(n) for m in (rnd(),)]
+        for q, m in mats:
+            c.add("Apply1QubitGate", q, m)
+            v = want.reshape(-1, 2, 1 << q)
+            m = m.astype(np.clongdouble)
+            v[:, 0], v[:, 1] = m[0, 0] * v[:, 0] + m[0, 1] * v[:, 1], m[1, 0] * v[:, 0] + m[1, 1] * v[:, 1]
+        for q in range(layer % 2, n - 1, 2):
+            c.add("ApplyCPauliX", q, q + 1)
+            v = want.reshape(-1, 2, 2, 1 << q)
+            v[:, :, 1] = v[:, ::-1, 1].copy()
+    reg = runner.new_register(c)
+    reg.TurnOnFusion()
+    reg, _ = runner.run(c, reg)
+    err = float(np.sqrt(np.sum(np.abs(runner.state_of(reg) - want) ** 2)))
+    print(f"brick 14 x 40, seed {seed}: error {err:.2e}", flush=True)
+    assert err < 96 ** 0.5 * 6 * 2.0 ** -53
