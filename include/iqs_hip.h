@@ -135,8 +135,8 @@ int iqsh_apply_kq(iqsh_handle h, unsigned k, const unsigned *pos, const double *
  * p[1]), row index 2*b(p[0]) + b(p[1])), applied together: gates on disjoint positions are
  * reordered, and every pass over the state applies all gates that become ready on the
  * positions of one tile, multiplied into dense blocks of at most `block` (1..5) positions.
- * Registers below 10 qubits take one pass per block.  *launched (may be null) receives the
- * number of passes.  Replaces the reference's fused-gate replay (src/qureg_fusion.cpp:56-94). */
+ * Registers below 10 qubits, and block kernels other than the default (iqsh_set_block_mfma), take
+ * one pass per block.  *launched (may be null) receives the number of passes.  Replaces the reference's fused-gate replay (src/qureg_fusion.cpp:56-94). */
 typedef struct {
   unsigned np;
   unsigned p[2];

@@ -1034,6 +1034,7 @@ int fail(int code, const char* fmt, ...)
   return code;
 }
 hipStream_t stream() { return g_stream; }
+int block_kernel() { return g_block_mfma; }
 int device_cus()
 {
   int dev = 0, cus = 0;

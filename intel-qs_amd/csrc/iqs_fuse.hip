@@ -847,7 +847,8 @@ int apply_tiled(iqsh_handle h, const iqsh_gate* g, int ngates, unsigned block, u
   return flush();
 }
 
-// Registers smaller than a tile: one dense block of up to `block` positions per pass.
+// One dense block of up to `block` positions per pass: registers smaller than a tile, and block
+// kernels that the caller has chosen instead of the tiles' three real products.
 int apply_blocks(iqsh_handle h, const iqsh_gate* g, int ngates, unsigned block, uint64_t* launched)
 {
   Dag all;
@@ -897,7 +898,7 @@ extern "C" int iqsh_apply_gates(iqsh_handle h, uint64_t ngates, const iqsh_gate*
     const std::vector<iqsh_gate> merged = merge_gates(gates, (int)ngates);
     gates = merged.data();
     const int ng = (int)merged.size();
-    if (h->n < 10) rc = apply_blocks(h, gates, ng, block, &count);
+    if (h->n < 10 || iqsi::block_kernel() != 1) rc = apply_blocks(h, gates, ng, block, &count);
     else if (h->dtype == IQSH_C128)
       rc = h->n < 12 ? apply_tiled<double, 10>(h, gates, ng, tb, &count) : apply_tiled<double, 12>(h, gates, ng, tb, &count);
     else

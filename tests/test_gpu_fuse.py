@@ -116,3 +116,36 @@ def test_double_precision_error_of_merged_gates(seed):
     err = float(np.sqrt(np.sum(np.abs(runner.state_of(reg) - want) ** 2)))
     print(f"brick 14 x 40, seed {seed}: error {err:.2e}", flush=True)
     assert err < 96 ** 0.5 * 6 * 2.0 ** -53
+
+
+@pytest.mark.parametrize("dt", ["c128", "c64"])
+@pytest.mark.parametrize("mode", [0, 2])
+def test_chosen_block_kernel_applies_gate_lists(dt, mode):
+    """With a block kernel chosen (iqsh_set_block_mfma), a list on five positions is one pass of that
+    kernel: the same bits as iqsh_apply_kq with the product, which is exact for these entries."""
+    class Gate(C.Structure):
+        _fields_ = [("np", C.c_uint), ("p", C.c_uint * 2), ("m", C.c_double * 32)]
+
+    n, pos = 13, [1, 4, 6, 9, 12]
+    r = np.random.default_rng(mode)
+    v = r.normal(size=1 << n) + 1j * r.normal(size=1 << n)
+    v = (v / np.linalg.norm(v)).astype(np.complex128 if dt == "c128" else np.complex64)
+    ms = [r.choice([0.5, -0.5, 0.5j, -0.25j, 0.75], (2, 2)) for _ in pos]
+    u = np.ones((1, 1), dtype=np.complex128)
+    gates = (Gate * 5)()
+    for i, (p, m) in enumerate(zip(pos, ms)):
+        u = np.kron(m, u)  # index bit i <-> pos[i]
+        gates[i].np, gates[i].p[0] = 1, p
+        gates[i].m[:8] = np.ascontiguousarray(m).view(np.float64).reshape(-1).tolist()
+    a, b, passes = StateVector(n, dt), StateVector(n, dt), C.c_uint64()
+    a.upload(v)
+    b.upload(v)
+    u = np.ascontiguousarray(u)
+    call("iqsh_set_block_mfma", mode)
+    try:
+        call("iqsh_apply_gates", a.handle, 5, gates, 5, C.byref(passes))
+        call("iqsh_apply_kq", b.handle, 5, (C.c_uint * 5)(*pos), C.c_void_p(u.ctypes.data))
+    finally:
+        call("iqsh_set_block_mfma", 1)
+    assert passes.value == 1
+    assert np.array_equal(a.download(), b.download())
