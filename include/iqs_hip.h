@@ -136,7 +136,8 @@ int iqsh_apply_kq(iqsh_handle h, unsigned k, const unsigned *pos, const double *
  * reordered, and every pass over the state applies all gates that become ready on the
  * positions of one tile, multiplied into dense blocks of at most `block` (1..5) positions.
  * Registers below 10 qubits, and block kernels other than the default (iqsh_set_block_mfma), take
- * one pass per block.  *launched (may be null) receives the number of passes.  Replaces the reference's fused-gate replay (src/qureg_fusion.cpp:56-94). */
+ * one pass per block; while the stream is captured into a graph the blocks are of at most two
+ * positions.  *launched (may be null) receives the number of passes.  Replaces the reference's fused-gate replay (src/qureg_fusion.cpp:56-94). */
 typedef struct {
   unsigned np;
   unsigned p[2];

@@ -1034,6 +1034,13 @@ int fail(int code, const char* fmt, ...)
   return code;
 }
 hipStream_t stream() { return g_stream; }
+bool capturing()
+{
+  hipStreamCaptureStatus s = hipStreamCaptureStatusNone;
+  if (!g_stream) return false;
+  if (hipStreamIsCapturing(g_stream, &s) != hipSuccess) (void)hipGetLastError();
+  return s != hipStreamCaptureStatusNone;
+}
 int block_kernel() { return g_block_mfma; }
 int device_cus()
 {

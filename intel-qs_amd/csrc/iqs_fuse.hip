@@ -847,8 +847,8 @@ int apply_tiled(iqsh_handle h, const iqsh_gate* g, int ngates, unsigned block, u
   return flush();
 }
 
-// One dense block of up to `block` positions per pass: registers smaller than a tile, and block
-// kernels that the caller has chosen instead of the tiles' three real products.
+// One dense block of up to `block` positions per pass: registers smaller than a tile, block kernels
+// that the caller has chosen instead of the tiles' three real products, and captures.
 int apply_blocks(iqsh_handle h, const iqsh_gate* g, int ngates, unsigned block, uint64_t* launched)
 {
   Dag all;
@@ -894,11 +894,15 @@ extern "C" int iqsh_apply_gates(iqsh_handle h, uint64_t ngates, const iqsh_gate*
   uint64_t count = 0;
   int rc;
   const unsigned tb = std::min(block, 4u);
+  // A graph is replayed after the ring's slots have been used again: in a capture every gate is in
+  // its kernel's arguments.
+  const bool capture = iqsi::capturing();
+  if (capture) block = std::min(block, 2u);
   try {
     const std::vector<iqsh_gate> merged = merge_gates(gates, (int)ngates);
     gates = merged.data();
     const int ng = (int)merged.size();
-    if (h->n < 10 || iqsi::block_kernel() != 1) rc = apply_blocks(h, gates, ng, block, &count);
+    if (h->n < 10 || capture || iqsi::block_kernel() != 1) rc = apply_blocks(h, gates, ng, block, &count);
     else if (h->dtype == IQSH_C128)
       rc = h->n < 12 ? apply_tiled<double, 10>(h, gates, ng, tb, &count) : apply_tiled<double, 12>(h, gates, ng, tb, &count);
     else

@@ -28,6 +28,8 @@ namespace iqsi {
 int fail(int code, const char* fmt, ...) __attribute__((format(printf, 2, 3)));
 // The library stream (iqsh_set_stream).
 hipStream_t stream();
+// Whether the library stream is being captured into a graph.
+bool capturing();
 // The kernel of dense blocks of three and more positions (iqsh_set_block_mfma).
 int block_kernel();
 // Compute units of the current device.

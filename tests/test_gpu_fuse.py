@@ -149,3 +149,50 @@ def test_chosen_block_kernel_applies_gate_lists(dt, mode):
         call("iqsh_set_block_mfma", 1)
     assert passes.value == 1
     assert np.array_equal(a.download(), b.download())
+
+
+@pytest.mark.parametrize("block", [2, 5])
+@pytest.mark.parametrize("dt", ["c128", "c64"])
+def test_captured_gate_lists_replay_their_own_gates(dt, block):
+    """A list captured into a graph, replayed between and after other lists (which use every slot of
+    the ring again), against the same list applied without a graph: three times the roundings of
+    the fused-against-unfused tests."""
+    torch = pytest.importorskip("torch")
+
+    class Gate(C.Structure):
+        _fields_ = [("np", C.c_uint), ("p", C.c_uint * 2), ("m", C.c_double * 32)]
+
+    def gates(seed, count):
+        r = SplitMix64(seed)
+        out = (Gate * count)()
+        for g in out:
+            a = r.randint(n)
+            g.np, g.p[0], g.p[1] = 2, a, (a + 1 + r.randint(n - 1)) % n
+            g.m[:] = haar_unitary(4, r).astype(np.complex128).view(np.float64).reshape(-1).tolist()
+        return out
+
+    n, count = 13, 12
+    one = gates(1, count)
+    a, b, other = (StateVector(n, dt) for _ in range(3))
+    for sv in (a, b, other):
+        sv.init_uniform(2.0 ** (-n / 2))
+    call("iqsh_apply_gates", other.handle, count, one, block, None)  # buffers exist
+    call("iqsh_sync")
+    stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    stream.wait_stream(torch.cuda.current_stream())
+    try:
+        call("iqsh_set_stream", C.c_void_p(stream.cuda_stream))
+        with torch.cuda.graph(graph, stream=stream):
+            call("iqsh_apply_gates", a.handle, count, one, block, None)
+        for k in range(3):
+            for i in range(5):
+                call("iqsh_apply_gates", other.handle, count, gates(10 * k + i + 2, count), block, None)
+            call("iqsh_sync")
+            with torch.cuda.stream(stream):
+                graph.replay()
+            call("iqsh_apply_gates", b.handle, count, one, block, None)
+            call("iqsh_sync")
+            assert np.abs(a.download() - b.download()).max() < 3 * TOL["dp" if dt == "c128" else "sp"]
+    finally:
+        call("iqsh_sync")
+        call("iqsh_set_stream", None)
