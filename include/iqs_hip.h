@@ -134,7 +134,8 @@ int iqsh_apply_kq(iqsh_handle h, unsigned k, const unsigned *pos, const double *
 /* A list of one- and two-qubit gates (np = 1: a row-major 2x2 on p[0]; np = 2: a 4x4 on (p[0],
  * p[1]), row index 2*b(p[0]) + b(p[1])), applied together: gates on disjoint positions are
  * reordered, and every pass over the state applies all gates that become ready on the
- * positions of one tile, multiplied into dense blocks of at most `block` (1..5) positions.
+ * positions of one tile, multiplied into dense blocks of at most `block` (1..5) positions
+ * (several blocks of up to four to a pass, or one of five).
  * Registers below 10 qubits, and block kernels other than the default (iqsh_set_block_mfma), take
  * one pass per block; while the stream is captured into a graph the blocks are of at most two
  * positions.  *launched (may be null) receives the number of passes.  Replaces the reference's fused-gate replay (src/qureg_fusion.cpp:56-94). */

@@ -773,24 +773,41 @@ int submit(iqsh_handle h, int slot, const std::vector<Staged>& staged, unsigned 
   return IQSH_OK;
 }
 
-// A block of one or two positions by itself: the 2x2 and 4x4 kernels.
-int launch_small(iqsh_handle h, const iqsh_gate* g, const Planned& b)
+// A block by itself, one pass: the 2x2 and 4x4 kernels, or that of up to five positions.
+int launch_dense(iqsh_handle h, const iqsh_gate* g, const Planned& b)
 {
   Product u;
   u.build(g, b.gates, 0, nullptr);
-  double m[32];
-  for (unsigned r = 0; r < (1u << u.k); ++r)
-    for (unsigned c = 0; c < (1u << u.k); ++c) {
-      m[2 * ((r << u.k) + c)] = u.re[r][c];
-      m[2 * ((r << u.k) + c) + 1] = u.im[r][c];
+  const unsigned D = 1u << u.k;
+  double m[2 * 32 * 32];
+  for (unsigned r = 0; r < D; ++r)
+    for (unsigned c = 0; c < D; ++c) {
+      m[2 * (r * D + c)] = u.re[r][c];
+      m[2 * (r * D + c) + 1] = u.im[r][c];
     }
-  return u.k == 1 ? iqsh_apply_1q(h, u.pos[0], m) : iqsh_apply_2q(h, u.pos[1], u.pos[0], m);
+  if (u.k == 1) return iqsh_apply_1q(h, u.pos[0], m);
+  if (u.k == 2) return iqsh_apply_2q(h, u.pos[1], u.pos[0], m);
+  return iqsh_apply_kq(h, u.k, u.pos, m);
 }
 
 // Passes of tile blocks.  Passes are staged until a launch's share of a slot is full, then
 // copied and launched together (one copy for a short list; a long one is planned while the
 // GPU works on what came before).
 constexpr unsigned kSubmitBlocks = 32;
+
+// Whether the gates of a pass are faster as `dense` passes of one 5-position block each than as one
+// pass of `tiled` blocks: few positions under many gates (a circuit on five qubits is one such
+// block).  From 64 MiB of amplitudes on, where the kernels' time counts, not the host's, a tile's
+// block takes about a quarter of a pass of the 5-position kernel in complex128, a fifth in complex64.
+// One dense block against 2, 3, 4, 5 and 10 of a tile: complex128, 27 qubits, 885 us against
+// 853, 1023, 1244, 1469 and 2646, 22 qubits 37 against 41, 57, 66, 72 and 115; complex64, 27
+// qubits, 450 (positions above 5; 635 on the lowest) against 430, 525, 676, 805 and 1387.  Below,
+// 21 qubits complex128, 34-79 (planning) against 26-74.
+template <typename T>
+bool dense_is_faster(iqsh_handle h, size_t tiled, size_t dense)
+{
+  return h->size() * h->esz() >= (uint64_t(64) << 20) && tiled + 1 >= (sizeof(T) == 8 ? 4 : 5) * dense;
+}
 
 template <typename T, int M>
 int apply_tiled(iqsh_handle h, const iqsh_gate* g, int ngates, unsigned block, uint64_t* launched)
@@ -801,7 +818,7 @@ int apply_tiled(iqsh_handle h, const iqsh_gate* g, int ngates, unsigned block, u
   const uint64_t every = (uint64_t(1) << h->n) - 1;
   const uint64_t low = (uint64_t(1) << FTile<T, M>::kLowBits) - 1;
   std::vector<int> gates;
-  std::vector<Planned> blocks;
+  std::vector<Planned> blocks, dense;
   std::vector<Staged> staged;
   unsigned used = 0;
   int slot = -1;
@@ -818,17 +835,33 @@ int apply_tiled(iqsh_handle h, const iqsh_gate* g, int ngates, unsigned block, u
     all.absorb(g, nullptr, set, M, gates);
     // Fill the tile up with the lowest other positions (longer rows).
     for (uint64_t rest = every & ~set; __builtin_popcountll(set) < M; rest &= rest - 1) set |= rest & -rest;
-    blocks.clear();
-    in.build(g, gates.data(), (int)gates.size());
-    while (!in.ready.empty()) {
-      Planned b{{}, 0};
-      in.absorb(g, gates.data(), b.set, block, b.gates);
-      blocks.push_back(std::move(b));
+    auto plan = [&](unsigned limit, std::vector<Planned>& list) {
+      list.clear();
+      in.build(g, gates.data(), (int)gates.size());
+      while (!in.ready.empty()) {
+        list.push_back(Planned{{}, 0});
+        in.absorb(g, gates.data(), list.back().set, limit, list.back().gates);
+      }
+    };
+    plan(std::min(block, 4u), blocks);
+    bool alone = blocks.size() == 1 && __builtin_popcountll(blocks[0].set) <= 2;
+    if (block == 5) {  // 5-position blocks need at least one pass per five positions
+      uint64_t touched = 0;
+      for (const Planned& b : blocks) touched |= b.set;
+      if (dense_is_faster<T>(h, blocks.size(), (__builtin_popcountll(touched) + 4) / 5)) {
+        plan(5, dense);
+        if (dense_is_faster<T>(h, blocks.size(), dense.size())) {
+          blocks.swap(dense);
+          alone = true;
+        }
+      }
     }
-    if (blocks.size() == 1 && __builtin_popcountll(blocks[0].set) <= 2) {
+    if (alone) {
       if (int rc = flush()) return rc;
-      if (int rc = launch_small(h, g, blocks[0])) return rc;
-      ++*launched;
+      for (const Planned& b : blocks) {
+        if (int rc = launch_dense(h, g, b)) return rc;
+        ++*launched;
+      }
       continue;
     }
     for (size_t i = 0; i < blocks.size();) {
@@ -853,25 +886,11 @@ int apply_blocks(iqsh_handle h, const iqsh_gate* g, int ngates, unsigned block, 
 {
   Dag all;
   all.build(g, nullptr, ngates);
-  std::vector<double> m;
   while (!all.ready.empty()) {
     Planned b{{}, 0};
     all.absorb(g, nullptr, b.set, block, b.gates);
+    if (int rc = launch_dense(h, g, b)) return rc;
     ++*launched;
-    if (__builtin_popcountll(b.set) <= 2) {
-      if (int rc = launch_small(h, g, b)) return rc;
-      continue;
-    }
-    Product u;
-    u.build(g, b.gates, 0, nullptr);
-    const unsigned D = 1u << u.k;
-    m.resize(2 * D * D);
-    for (unsigned r = 0; r < D; ++r)
-      for (unsigned c = 0; c < D; ++c) {
-        m[2 * (r * D + c)] = u.re[r][c];
-        m[2 * (r * D + c) + 1] = u.im[r][c];
-      }
-    if (int rc = iqsh_apply_kq(h, u.k, u.pos, m.data())) return rc;
   }
   return IQSH_OK;
 }
@@ -893,7 +912,6 @@ extern "C" int iqsh_apply_gates(iqsh_handle h, uint64_t ngates, const iqsh_gate*
   }
   uint64_t count = 0;
   int rc;
-  const unsigned tb = std::min(block, 4u);
   // A graph is replayed after the ring's slots have been used again: in a capture every gate is in
   // its kernel's arguments.
   const bool capture = iqsi::capturing();
@@ -904,9 +922,9 @@ extern "C" int iqsh_apply_gates(iqsh_handle h, uint64_t ngates, const iqsh_gate*
     const int ng = (int)merged.size();
     if (h->n < 10 || capture || iqsi::block_kernel() != 1) rc = apply_blocks(h, gates, ng, block, &count);
     else if (h->dtype == IQSH_C128)
-      rc = h->n < 12 ? apply_tiled<double, 10>(h, gates, ng, tb, &count) : apply_tiled<double, 12>(h, gates, ng, tb, &count);
+      rc = h->n < 12 ? apply_tiled<double, 10>(h, gates, ng, block, &count) : apply_tiled<double, 12>(h, gates, ng, block, &count);
     else
-      rc = h->n < 12 ? apply_tiled<float, 10>(h, gates, ng, tb, &count) : apply_tiled<float, 12>(h, gates, ng, tb, &count);
+      rc = h->n < 12 ? apply_tiled<float, 10>(h, gates, ng, block, &count) : apply_tiled<float, 12>(h, gates, ng, block, &count);
   } catch (const std::exception& e) {
     return iqsi::fail(IQSH_ERR_ALLOC, "planning %llu gates: %s", (unsigned long long)ngates, e.what());
   }

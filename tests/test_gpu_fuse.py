@@ -196,3 +196,35 @@ def test_captured_gate_lists_replay_their_own_gates(dt, block):
     finally:
         call("iqsh_sync")
         call("iqsh_set_stream", None)
+
+
+@pytest.mark.parametrize("dt,n", [("c128", 22), ("c64", 23)])
+def test_many_gates_on_five_qubits_are_one_block(dt, n):
+    """Many gates on five positions of a large register are one dense block (not a pass of many
+    smaller ones): the same bits as iqsh_apply_kq with the product, which is exact for these
+    gates (permutations with phases of +-1 and +-i, one term per row and so the same sums in any
+    order).  A block of four positions at most rounds again in between."""
+    class Gate(C.Structure):
+        _fields_ = [("np", C.c_uint), ("p", C.c_uint * 2), ("m", C.c_double * 32)]
+
+    count, pos = 60, [2, 7, 11, 16, n - 1]
+    r = np.random.default_rng(n)
+    u = np.eye(32, dtype=np.complex128)
+    gates = (Gate * count)()
+    for g in gates:
+        a, b = (int(x) for x in r.choice(5, 2, replace=False))
+        m = np.eye(4)[r.permutation(4)] * r.choice([1, -1, 1j, -1j], 4)[:, None]
+        g.np, g.p[0], g.p[1] = 2, pos[a], pos[b]
+        g.m[:] = m.astype(np.complex128).view(np.float64).reshape(-1).tolist()
+        i = np.arange(32)
+        sub = 2 * ((i >> a) & 1) + ((i >> b) & 1)
+        rest = i & ~((1 << a) | (1 << b))
+        u = (m[np.ix_(sub, sub)] * (rest[:, None] == rest[None, :])) @ u
+    v = (r.standard_normal(1 << n) + 1j * r.standard_normal(1 << n)) * 2.0 ** (-n / 2)
+    a, b, passes = StateVector(n, dt), StateVector(n, dt), C.c_uint64()
+    a.upload(v.astype(np.complex128 if dt == "c128" else np.complex64))
+    b.copy_from(a)
+    u = np.ascontiguousarray(u)
+    call("iqsh_apply_kq", b.handle, 5, (C.c_uint * 5)(*pos), C.c_void_p(u.ctypes.data))
+    call("iqsh_apply_gates", a.handle, count, gates, 5, C.byref(passes))
+    assert passes.value == 1 and a.maxabsdiff(b) == 0.0
