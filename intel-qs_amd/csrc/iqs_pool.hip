@@ -14,7 +14,6 @@
 #include <cmath>
 #include <mutex>
 #include <type_traits>
-#include <vector>
 
 #include "../../include/iqs_hip.h"
 #include "iqs_internal.hpp"
@@ -40,26 +39,35 @@ struct PoolWork {
   hipEvent_t done[kSlots];
   bool events = false, used[kSlots] = {};
   int next = 0;
-  double* pinned = nullptr;  // kHostParts partial sums written by the kernels
-  double* part = nullptr;    // more than that: on the device
+  double* pinned = nullptr;  // partial sums of up to kHostChunks workgroups, written by the kernels
+  double* part = nullptr;    // of more than that: on the device, and pinned where they are copied to
+  double* copy = nullptr;
   size_t part_bytes = 0;
-  std::vector<double> host;
 };
-// Chunk sums up to this many go straight to pinned host memory (512 KiB).
-constexpr uint64_t kHostParts = 65536;
+// The sums of up to this many workgroups go straight to pinned host memory, which spares the copy
+// and its wait; each workgroup's write crosses the bus by itself, so more of them are faster on
+// the device and copied (norms of 3-qubit states: 512 workgroups 8.6 against 16.5 us, 8192 28.6
+// against 31.5, 16384 52.5 against 41-46, 65536 182 against 96-114; overlaps, two sums each: 8192
+// 36.5 against 39.8, 16384 71 against 58).
+constexpr uint64_t kHostChunks = 8192;
 PoolWork g_pw;
 std::mutex g_pm;
 
-int grow(void** p, size_t* have, size_t need)
+// Space for `need` bytes of partial sums on the device and their copy.
+int grow_parts(size_t need)
 {
-  if (*have >= need) return IQSH_OK;
-  // The buffer may still be read by earlier work on the stream.
-  IQSI_TRY(hipStreamSynchronize(iqsi::stream()));
-  if (*p) IQSI_TRY(hipFree(*p));
-  *p = nullptr;
-  *have = 0;
-  if (hipMalloc(p, need) != hipSuccess) return iqsi::fail(IQSH_ERR_ALLOC, "pool work buffer of %zu bytes", need);
-  *have = need;
+  if (g_pw.part_bytes >= need) return IQSH_OK;
+  need = std::max(need, size_t(2) << 20);
+  g_pw.part_bytes = 0;
+  if (g_pw.part) IQSI_TRY(hipFree(g_pw.part));
+  g_pw.part = nullptr;
+  if (g_pw.copy) IQSI_TRY(hipHostFree(g_pw.copy));
+  g_pw.copy = nullptr;
+  if (hipMalloc((void**)&g_pw.part, need) != hipSuccess || hipHostMalloc((void**)&g_pw.copy, need, hipHostMallocDefault) != hipSuccess) {
+    (void)hipGetLastError();
+    return iqsi::fail(IQSH_ERR_ALLOC, "pool work buffer of %zu bytes", need);
+  }
+  g_pw.part_bytes = need;
   return IQSH_OK;
 }
 
@@ -555,7 +563,7 @@ int do_2q_each(iqsh_handle h, unsigned sbits, unsigned ph, unsigned pl, const do
   });
 }
 
-// Launch `nchunks` chunk reductions with NV values each, then sum them per state on the host.
+// Launch `nchunks` chunk reductions with nv (1 or 2) values each, then sum them per state on the host.
 template <typename Launch>
 int reduce_per_state(unsigned sbits, uint64_t nstates, int nv, double* out, Launch launch)
 {
@@ -566,21 +574,20 @@ int reduce_per_state(unsigned sbits, uint64_t nstates, int nv, double* out, Laun
   const uint64_t nchunks = nstates * per_state;
   if (nchunks > 0x7fffffffull) return iqsi::fail(IQSH_ERR_NOTSUP, "pool reduction needs %llu workgroups", (unsigned long long)nchunks);
   const double* sums;
-  if (nchunks * nv <= kHostParts) {
-    if (!g_pw.pinned) IQSI_TRY(hipHostMalloc((void**)&g_pw.pinned, kHostParts * sizeof(double), hipHostMallocDefault));
+  if (nchunks <= kHostChunks) {
+    if (!g_pw.pinned) IQSI_TRY(hipHostMalloc((void**)&g_pw.pinned, 2 * kHostChunks * sizeof(double), hipHostMallocDefault));
     iqsi::mark_pending(g_pw.pinned, nchunks * nv);
     launch((unsigned)nchunks, clog, g_pw.pinned);
     IQSI_TRY(hipGetLastError());
     if (int rc = iqsi::await_results(g_pw.pinned, nchunks * nv)) return rc;
     sums = g_pw.pinned;
   } else {
-    if (int rc = grow((void**)&g_pw.part, &g_pw.part_bytes, nchunks * nv * sizeof(double))) return rc;
+    if (int rc = grow_parts(nchunks * nv * sizeof(double))) return rc;
     launch((unsigned)nchunks, clog, g_pw.part);
     IQSI_TRY(hipGetLastError());
-    g_pw.host.resize(nchunks * nv);
-    IQSI_TRY(hipMemcpyAsync(g_pw.host.data(), g_pw.part, nchunks * nv * sizeof(double), hipMemcpyDeviceToHost, iqsi::stream()));
+    IQSI_TRY(hipMemcpyAsync(g_pw.copy, g_pw.part, nchunks * nv * sizeof(double), hipMemcpyDeviceToHost, iqsi::stream()));
     IQSI_TRY(hipStreamSynchronize(iqsi::stream()));
-    sums = g_pw.host.data();
+    sums = g_pw.copy;
   }
   for (uint64_t s = 0; s < nstates; ++s)
     for (int r = 0; r < nv; ++r) {

@@ -305,3 +305,34 @@ def test_per_state_matrices_and_probabilities_over_sizes(dt, sbits, nstates):
     call("iqsh_pool_reduce", sv.handle, C.c_uint(sbits), C.c_int(0), C.c_uint64(0), C.c_void_p(out.ctypes.data),
          C.c_uint64(nstates))
     assert np.abs(out - p[:nstates].sum(axis=1)).max() < 1e-13
+
+
+@pytest.mark.parametrize("dt", ["c128", "c64"])
+@pytest.mark.parametrize("sbits,nstates", [(3, 8192), (3, 8193), (3, 70000), (12, 4097), (9, 9000)])
+def test_reductions_over_many_states(dt, sbits, nstates):
+    """Sums written to the host by the kernels (up to 8192 workgroups) and copied from the device
+    (more), around the limit and far beyond it, one and two values per workgroup, against numpy.
+    Tolerance: sums of at most 2^12 products in FP64, of states of norm 1."""
+    import ctypes as C
+
+    from iqs_amd._lib import call
+    from iqs_amd.engine import StateVector
+    n = sbits + (nstates - 1).bit_length()
+    r = np.random.default_rng(nstates)
+    v = r.standard_normal((1 << (n - sbits), 1 << sbits)) + 1j * r.standard_normal((1 << (n - sbits), 1 << sbits))
+    v = (v / np.linalg.norm(v, axis=1, keepdims=True)).astype(np.complex128 if dt == "c128" else np.complex64)
+    sv, ref = StateVector(n, dt), StateVector(sbits, dt)
+    sv.upload(v.reshape(-1))
+    ref.upload(v[1])
+    w = v.astype(np.complex128)[:nstates]
+    p = np.abs(w) ** 2
+    sign = np.array([1 - 2 * (bin(i & 5).count("1") & 1) for i in range(1 << sbits)])
+    top = sbits - 1
+    out = np.zeros(2 * nstates)
+    for kind, arg, want in ((0, 0, p.sum(1)), (1, 0, p.reshape(nstates, -1, 2)[:, :, 1].sum(1)),
+                            (1, top, p[:, 1 << top:].sum(1)), (2, 5, (p * sign).sum(1))):
+        call("iqsh_pool_reduce", sv.handle, C.c_uint(sbits), C.c_int(kind), C.c_uint64(arg), C.c_void_p(out.ctypes.data),
+             C.c_uint64(nstates))
+        assert np.abs(out[:nstates] - want).max() < 1e-13
+    call("iqsh_pool_overlap", sv.handle, C.c_uint(sbits), ref.handle, C.c_void_p(out.ctypes.data), C.c_uint64(nstates))
+    assert np.abs(out.view(np.complex128) - w @ w[1].conj()).max() < 1e-13
