@@ -489,27 +489,28 @@ int layer_m(const LayerArgs& a, LayerShape* shape)
 // Tile size: large tiles (long rows, fewest passes) for registers that fill the chip with
 // them; below that the smallest tile that takes no more passes, for more workgroups (18
 // qubits complex128 takes 14.1 us with 64 tiles of 2^12, 12.6 with 128 of 2^11, but at 20 qubits
-// 2^11 needs one pass more: 21.1 against 25.5 us).  complex64 forward: 2^13 with 32
-// amplitudes per thread (256-byte rows as in complex128); its adjoint 2^12 with 16, since
-// psi and lambda of 32 amplitudes left two waves per SIMD and spilled (25 qubits weighted
-// low pass 535 against 287 us).
+// 2^11 needs one pass more: 21.1 against 25.5 us).  complex64 forward: the same, and from 26 qubits
+// on 2^13 with 32 amplitudes per thread (256-byte rows as in complex128) where that is one pass
+// less (29 qubits 6.22 -> 5.15 ms) or the products are the short ones (28 qubits RX 2.37 -> 2.32 ms;
+// with the weighted phase 2.58 against 2.69), and for the one tile of 13 qubits with those (9.1 ->
+// 7.9 us; general 2x2 9.2 against 12.1).  Elsewhere 32 amplitudes leave too few waves: general
+// 2x2, 12 qubits 12.8 -> 7.0 us with 16, 15 qubits 15.3 -> 10.4, 19 qubits 24.9 -> 16.7, 25 qubits
+// with the weighted phase 343 -> 329, RX 303 -> 278.  The adjoint has psi and lambda in registers: 32
+// amplitudes of each left two waves per SIMD and spilled (25 qubits weighted low pass 535 against 287
+// us).
 template <typename T, bool ADJ, int F>
 int layer_n(const LayerArgs& a, LayerShape* shape)
 {
   const unsigned n = a.psi->n;
   const bool cached = iqsi::cache_set(a.psi->size() * sizeof(typename Vec<T>::t) * (ADJ ? 2 : 1));
-  if constexpr (sizeof(T) == 8) {
-    if (n <= 10 || (n > 12 && n <= 16)) return layer_m<T, 10, 4, ADJ, F>(a, shape);
-    if (n == 11 || n == 17 || n == 18) return layer_m<T, 11, 4, ADJ, F>(a, shape);
-    return cached ? layer_m<T, 12, 4, ADJ, F, false>(a, shape) : layer_m<T, 12, 4, ADJ, F>(a, shape);
-  } else if constexpr (ADJ) {
-    if (n <= 11 || (n > 12 && n <= 16)) return layer_m<T, 10, 4, ADJ, F>(a, shape);
-    return cached ? layer_m<T, 12, 4, ADJ, F, false>(a, shape) : layer_m<T, 12, 4, ADJ, F>(a, shape);
-  } else {
-    if (n <= 10) return layer_m<T, 10, 4, ADJ, F>(a, shape);
-    if (n <= 12 || (n > 13 && n <= 17)) return layer_m<T, 11, 5, ADJ, F>(a, shape);
-    return cached ? layer_m<T, 13, 5, ADJ, F, false>(a, shape) : layer_m<T, 13, 5, ADJ, F>(a, shape);
+  if constexpr (sizeof(T) == 4 && !ADJ) {
+    const bool short_products = (F & kFormRX) != 0 && !(a.cs && a.cs->weighted);
+    if ((n >= 26 && (short_products || (n - 13) % 8 == 0)) || (n == 13 && short_products)) return layer_m<T, 13, 5, ADJ, F>(a, shape);
   }
+  if (n <= 10 || (n > 12 && n <= 16) || (sizeof(T) == 4 && ADJ && n == 11)) return layer_m<T, 10, 4, ADJ, F>(a, shape);
+  if constexpr (sizeof(T) == 8 || !ADJ)
+    if (n == 11 || n == 17 || n == 18) return layer_m<T, 11, 4, ADJ, F>(a, shape);
+  return cached ? layer_m<T, 12, 4, ADJ, F, false>(a, shape) : layer_m<T, 12, 4, ADJ, F>(a, shape);
 }
 
 // With `shape` only that is filled in.  The RX-form kernels when the 2x2 has a real diagonal and an imaginary off-diagonal (the

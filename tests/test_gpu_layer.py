@@ -162,3 +162,58 @@ def test_layer_tiles(dt, weighted, n):
     tol = 1e-11 if dt == "c128" else 2e-5
     assert abs(db - db1) < tol * max(1, abs(db1)) and abs(dg - dg1) < tol * max(1, abs(dg1))
     assert a.maxabsdiff(b) < TOL[dt] and la.maxabsdiff(lb) < TOL[dt]
+
+
+@pytest.mark.parametrize("dt,n", [(dt, n) for dt in ("c128", "c64") for n in (10, 11, 12, 13, 16, 17, 18, 19, 21, 22, 24, 25)]
+                         + [("c64", 26), ("c64", 29)])
+def test_general_layer_tiles(dt, n):
+    """A general 2x2 and a general generator in every tile size, cache policy and number of passes, with
+    and without a weighted phase, and the generator X with a general inverse: against the phase and the
+    gates one by one.  Tolerances: 4 n + 2 roundings per amplitude of size <= 1, and for the sums the
+    relative ones above."""
+    r = np.random.default_rng(n)
+    pairs = [tuple(int(v) for v in r.choice(n, 2, replace=False)) for _ in range(min(64, 2 * n))]
+    edges = [(u, v, float(r.uniform(0.1, 2.0))) for u, v in pairs]
+    gamma, u = 0.37, _unitary(3 * n)
+    uinv = u.conj().T
+    a, b = StateVector(n, dt), StateVector(n, dt)
+
+    def start(sv, angle):  # a generic state made on the GPU (29 qubits are 4 GiB)
+        sv.init_uniform(2.0 ** (-n / 2))
+        sv.qaoa_phase(edges, angle)
+        for q in range(n):
+            sv.apply_1q(q, _unitary(7 * n + q))
+
+    def gates(sv, m):
+        for q in range(n):
+            sv.apply_1q(q, m)
+
+    start(a, 0.9)
+    b.copy_from(a)
+    a.apply_1q_all(u)
+    gates(b, u)
+    assert a.maxabsdiff(b) < TOL[dt]
+    a.qaoa_layer(edges, gamma, u)
+    b.qaoa_phase(edges, gamma)
+    gates(b, u)
+    assert a.maxabsdiff(b) < TOL[dt]
+    if n > 25:
+        return  # the adjoint's tiles are those of 25 qubits
+    X = np.array([[0, 1], [1, 0]], dtype=complex)
+    G = np.array([[0.3, 1.2 - 0.4j], [1.2 + 0.4j, -0.7]])
+    tol = 1e-11 if dt == "c128" else 2e-5
+    la, lb = StateVector(n, dt), StateVector(n, dt)
+    start(la, 0.2)
+    lb.copy_from(la)
+    for gen in (G, X):
+        b.copy_from(a)
+        lb.copy_from(la)
+        got = a.adjoint_1q_all(la, uinv, gen)
+        want = sum(b.adjoint_1q(lb, q, uinv, gen) for q in range(n))
+        assert abs(got - want) < tol * max(1, abs(want))
+        assert a.maxabsdiff(b) < TOL[dt] and la.maxabsdiff(lb) < TOL[dt]
+    dg, dm = a.qaoa_layer_adjoint(la, edges, gamma, uinv, G)
+    dm1 = sum(b.adjoint_1q(lb, q, uinv, G) for q in range(n))
+    dg1 = b.qaoa_phase_adjoint(lb, edges, gamma)
+    assert abs(dg - dg1) < tol * max(1, abs(dg1)) and abs(dm - dm1) < tol * max(1, abs(dm1))
+    assert a.maxabsdiff(b) < TOL[dt] and la.maxabsdiff(lb) < TOL[dt]
