@@ -391,7 +391,8 @@ int iqsh_pool_init(iqsh_handle h, unsigned state_qubits, int style, uint64_t ind
 /* A different 2x2 matrix per state on position pos < state_qubits: mats holds nstates
  * row-major complex 2x2 matrices (8 doubles each).  One launch for the whole pool; what the
  * reference does with one Apply1QubitGate per rank group (noise gates and channel branches
- * differ from state to state). */
+ * differ from state to state).  While the stream is captured into a graph, only matrices that fit
+ * the kernel's arguments (2 KiB in the register's precision) are accepted, here and below. */
 int iqsh_pool_apply_1q_each(iqsh_handle h, unsigned state_qubits, unsigned pos, const double *mats,
                             uint64_t nstates);
 /* A different dense 4x4 matrix per state on positions (ph, pl) < state_qubits, row index

@@ -125,6 +125,9 @@ int with_mats(uint64_t nstates, Fill fill, Launch launch)
     IQSI_TRY(hipGetLastError());
     return IQSH_OK;
   }
+  // A graph would be replayed after the slot has been refilled.
+  if (iqsi::capturing())
+    return iqsi::fail(IQSH_ERR_NOTSUP, "per-state matrices of more than %zu bytes cannot be captured into a graph", kArgBytes);
   int slot;
   if (int rc = mats_slot(bytes, &slot)) return rc;
   MT* host = (MT*)(g_pw.mats_host + slot * g_pw.slot_bytes);

@@ -336,3 +336,49 @@ def test_reductions_over_many_states(dt, sbits, nstates):
         assert np.abs(out[:nstates] - want).max() < 1e-13
     call("iqsh_pool_overlap", sv.handle, C.c_uint(sbits), ref.handle, C.c_void_p(out.ctypes.data), C.c_uint64(nstates))
     assert np.abs(out.view(np.complex128) - w @ w[1].conj()).max() < 1e-13
+
+
+def test_per_state_matrices_in_a_capture():
+    """Matrices that fit a kernel's arguments can be captured into a graph and are replayed as they
+    were; more of them (a slot that later calls refill) are refused, and the capture goes on."""
+    import ctypes as C
+
+    torch = pytest.importorskip("torch")
+    from iqs_amd._lib import IqsError, call
+    from iqs_amd.engine import StateVector
+    sbits, n = 5, 12
+    sv, want = StateVector(n, "c128"), StateVector(n, "c128")
+
+    def rotations(ns, seed):
+        th = np.random.default_rng(seed).uniform(0, 6, ns)
+        m = np.zeros((ns, 2, 2), dtype=np.complex128)
+        m[:, 0, 0] = m[:, 1, 1] = np.cos(th)
+        m[:, 0, 1], m[:, 1, 0] = -np.sin(th), np.sin(th)
+        return m
+
+    def each(target, m):
+        call("iqsh_pool_apply_1q_each", target.handle, C.c_uint(sbits), C.c_uint(3), C.c_void_p(m.ctypes.data), C.c_uint64(len(m)))
+
+    few, many = rotations(30, 1), rotations(100, 2)
+    for v in (sv, want):
+        v.init_uniform(2.0 ** (-n / 2))
+        each(v, many)
+    call("iqsh_sync")
+    stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    try:
+        call("iqsh_set_stream", C.c_void_p(stream.cuda_stream))
+        with torch.cuda.graph(graph, stream=stream):
+            with pytest.raises(IqsError):
+                each(sv, many)
+            each(sv, few)
+        for k in range(3):
+            with torch.cuda.stream(stream):
+                graph.replay()
+            each(want, few)
+            assert sv.maxabsdiff(want) < 1e-14
+            each(sv, many)
+            each(want, many)
+            assert sv.maxabsdiff(want) < 1e-14
+    finally:
+        call("iqsh_sync")
+        call("iqsh_set_stream", None)
