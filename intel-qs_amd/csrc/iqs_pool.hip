@@ -80,15 +80,19 @@ int mats_slot(size_t bytes, int* slot)
   }
   if (g_pw.slot_bytes < bytes) {
     const size_t want = std::max<size_t>(4096, (bytes + 255) & ~size_t(255));
-    IQSI_TRY(hipStreamSynchronize(iqsi::stream()));
+    // Copies and launches that still read the old slots may be on other streams than this call's.
+    for (int i = 0; i < kSlots; ++i)
+      if (g_pw.used[i]) IQSI_TRY(hipEventSynchronize(g_pw.done[i]));
     g_pw.slot_bytes = 0;
     if (g_pw.mats_host) IQSI_TRY(hipHostFree(g_pw.mats_host));
     g_pw.mats_host = nullptr;
     if (g_pw.mats) IQSI_TRY(hipFree(g_pw.mats));
     g_pw.mats = nullptr;
     if (hipHostMalloc((void**)&g_pw.mats_host, want * kSlots, hipHostMallocDefault) != hipSuccess ||
-        hipMalloc((void**)&g_pw.mats, want * kSlots) != hipSuccess)
+        hipMalloc((void**)&g_pw.mats, want * kSlots) != hipSuccess) {
+      (void)hipGetLastError();
       return iqsi::fail(IQSH_ERR_ALLOC, "pool matrices of %zu bytes", bytes);
+    }
     g_pw.slot_bytes = want;
     std::fill(g_pw.used, g_pw.used + kSlots, false);
   }

@@ -382,3 +382,49 @@ def test_per_state_matrices_in_a_capture():
     finally:
         call("iqsh_sync")
         call("iqsh_set_stream", None)
+
+
+@pytest.mark.parametrize("dt", ["c128", "c64"])
+def test_matrix_slots_grow_between_streams(dt):
+    """Per-state 2x2 and 4x4 matrices of pools that take turns, each larger one growing the slots while
+    the launches of the one before are still on another stream: 2x2 in arguments and slots for both
+    precisions, 4x4 likewise, against numpy.  Tolerance: one product of two or four terms per call and
+    amplitude (8 roundings of amplitudes below 8), three calls."""
+    import ctypes as C
+
+    torch = pytest.importorskip("torch")
+    from iqs_amd._lib import call
+    from iqs_amd.circuits import SplitMix64, haar_unitary
+    from iqs_amd.engine import StateVector
+    npdt = np.complex128 if dt == "c128" else np.complex64
+    tol = 3 * 8 * 8 * (2.0 ** -53 if dt == "c128" else 2.0 ** -24)
+    rng, r = SplitMix64(3), np.random.default_rng(4)
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    pools = []
+    try:
+        for k, (sbits, ns) in enumerate([(12, 9), (6, 66), (11, 17), (5, 300), (10, 40), (4, 2000), (9, 100), (4, 9000)]):
+            n = sbits + (ns - 1).bit_length()
+            host = (r.uniform(-1, 1, 1 << n) + 1j * r.uniform(-1, 1, 1 << n)).astype(npdt)
+            want = host.astype(np.complex128).reshape(-1, 1 << sbits)
+            call("iqsh_set_stream", C.c_void_p(streams[k % 2].cuda_stream))
+            sv = StateVector(n, dt)
+            sv.upload(host)
+            for pos in ((sbits - 1,), (2, 0), (1, sbits - 1)):
+                d = 1 << len(pos)
+                few = [haar_unitary(d, rng) for _ in range(min(ns, 50))]
+                us = np.stack([few[s % len(few)] * np.exp(1j * s) for s in range(ns)]).astype(npdt).astype(np.complex128)
+                name = "iqsh_pool_apply_1q_each" if d == 2 else "iqsh_pool_apply_2q_each"
+                call(name, sv.handle, C.c_uint(sbits), *(C.c_uint(p) for p in pos), C.c_void_p(us.ctypes.data), C.c_uint64(ns))
+                i = np.arange(1 << sbits)
+                base = i[sum((i >> p) & 1 for p in pos) == 0]
+                rows = [base + sum(((t >> (len(pos) - 1 - j)) & 1) << p for j, p in enumerate(pos)) for t in range(d)]
+                x = np.stack([want[:ns][:, rw] for rw in rows], 1)
+                y = us @ x
+                for t, rw in enumerate(rows):
+                    want[:ns, rw] = y[:, t]
+            pools.append((sv, want))
+    finally:
+        torch.cuda.synchronize()
+        call("iqsh_set_stream", None)
+    for sv, want in pools:
+        assert np.abs(sv.download().reshape(want.shape) - want).max() < tol
