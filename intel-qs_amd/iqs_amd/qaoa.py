@@ -33,6 +33,11 @@ X = np.array([[0, 1], [1, 0]], dtype=np.complex128)
 LAYER_MIN_QUBITS = 10
 
 
+def _number(x) -> float:
+    """An angle of any numeric type (Python, numpy, a tensor of one element on any device)."""
+    return float(1.0 * x)
+
+
 @dataclass
 class MaxCutQaoa:
     num_qubits: int
@@ -73,8 +78,11 @@ class MaxCutQaoa:
         psi = self._state("_psi")
         fused = self.num_qubits >= LAYER_MIN_QUBITS
         if fused and not shift and not self.renorm_every:
-            layers = min(len(gammas), len(betas))
-            psi.qaoa_run(self.edges, gammas[:layers], betas[:layers])
+            angles = [(_number(g), _number(b)) for g, b in zip(gammas, betas)]
+            if angles:
+                psi.qaoa_run(self.edges, *zip(*angles))
+            else:
+                self._prepare(psi)
             return psi
         self._prepare(psi)
         for l, (g, b) in enumerate(zip(gammas, betas)):
@@ -106,7 +114,7 @@ class MaxCutQaoa:
         psi = self._state("_psi")
         lam = self._state("_lam")
         if self.num_qubits >= LAYER_MIN_QUBITS:
-            return psi.qaoa_gradient(lam, self.edges, gammas, betas[:p])
+            return psi.qaoa_gradient(lam, self.edges, [_number(g) for g in gammas], [_number(betas[l]) for l in range(p)])
         cost = psi.qaoa_cost_apply(lam, self.edges)
         dg, db = np.zeros(p), np.zeros(p)
         for l in reversed(range(p)):
