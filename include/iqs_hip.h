@@ -291,7 +291,7 @@ enum iqsh_hea_flags {
 
 /* Tuning of a batch: `variant` picks the kernel's tile (tile qubits, amplitudes per thread,
  * see iqsh_hea_variant_info); `workers_per_cu` persistent workgroups per compute unit
- * (0 = as many as fit); `order` the task order: 0 = tiled instances first, single-tile
+ * (0 = as many as fit and the tiled instances keep busy); `order` the task order: 0 = tiled instances first, single-tile
  * instances last; 1 = single-tile first; 2 = single-tile instances interleaved among the
  * steps of the tiled ones; 3 = as 0 with every tiled instance's steps aligned to end on
  * the last round.  `group_mib` > 0 processes the tiled instances in consecutive groups
@@ -318,7 +318,7 @@ int iqsh_hea_variants(int dtype, int *count);
 int iqsh_hea_variant_info(int dtype, int variant, int *tile_qubits, int *amps_per_thread,
                           int *threads, int *for_tests);
 /* Create a batch (allocates every state and work buffer); tune NULL = default variant 0,
- * as many workers as fit and find work, order 0. */
+ * as many workers as fit and the tiled instances keep busy, order 0. */
 int iqsh_hea_create(int dtype, int count, const int *nqubits, const int *depth,
                     const iqsh_hea_tune *tune, iqsh_hea_handle *out);
 int iqsh_hea_destroy(iqsh_hea_handle h);
