@@ -217,3 +217,33 @@ def test_general_layer_tiles(dt, n):
     dg1 = b.qaoa_phase_adjoint(lb, edges, gamma)
     assert abs(dg - dg1) < tol * max(1, abs(dg1)) and abs(dm - dm1) < tol * max(1, abs(dm1))
     assert a.maxabsdiff(b) < TOL[dt] and la.maxabsdiff(lb) < TOL[dt]
+
+
+@pytest.mark.parametrize("dt", ["c128", "c64"])
+@pytest.mark.parametrize("weighted", [False, True])
+@pytest.mark.parametrize("n,p", [(10, 20), (13, 20), (18, 20), (10, 300)])
+def test_qaoa_circuit_in_one_call(dt, weighted, n, p):
+    """qaoa_run and qaoa_gradient against a loop of the layer calls: more sums than one list of runs
+    holds (20 layers), and more results than the first buffer has room for (300 layers of 10 qubits).
+    The layers are the same kernels, so the states are the same bits; sums that were taken together
+    differ by the order of at most 2^8 partials (2^8 roundings of 2^-53 of sums of magnitude up to
+    the cost, 2 n)."""
+    from iqs_amd import gates as Gt
+    edges = _graph(n, 5, weighted)
+    r = np.random.default_rng(p)
+    gammas, betas = r.uniform(0, np.pi, p), r.uniform(0, np.pi, p)
+    X = np.array([[0, 1], [1, 0]])
+    a, la, b, lb = (StateVector(n, dt) for _ in range(4))
+    a.qaoa_run(edges, gammas, betas)
+    b.init_uniform(1.0 / np.sqrt(float(1 << n)))
+    for g, t in zip(gammas, betas):
+        b.qaoa_layer(edges, g, Gt.rx(2 * t))
+    assert a.maxabsdiff(b) == 0.0
+    cost, dg, db = a.qaoa_gradient(la, edges, gammas, betas)
+    want = b.qaoa_cost_apply(lb, edges)
+    tol = 2.0 ** 8 * 2.0 ** -53 * 2 * n
+    assert abs(cost - want) < tol
+    for l in reversed(range(p)):
+        wg, wb = b.qaoa_layer_adjoint(lb, edges, gammas[l], Gt.rx(-2 * betas[l]), X)
+        assert abs(dg[l] - wg) < 2 * tol and abs(db[l] - wb) < 2 * tol * n
+    assert a.maxabsdiff(b) == 0.0 and la.maxabsdiff(lb) == 0.0
