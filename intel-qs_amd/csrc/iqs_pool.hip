@@ -48,8 +48,9 @@ struct PoolWork {
 // and its wait; each workgroup's write crosses the bus by itself, so more of them are faster on
 // the device and copied (norms of 3-qubit states: 512 workgroups 8.6 against 16.5 us, 8192 28.6
 // against 31.5, 16384 52.5 against 41-46, 65536 182 against 96-114; overlaps, two sums each: 8192
-// 36.5 against 39.8, 16384 71 against 58).
-constexpr uint64_t kHostChunks = 8192;
+// 36.5 against 39.8, 16384 71 against 58).  The buffer is larger than they need: with 128 KiB of
+// pinned memory each reduction took 0.3 us more than with 512.
+constexpr uint64_t kHostChunks = 8192, kHostDoubles = 65536;
 PoolWork g_pw;
 std::mutex g_pm;
 
@@ -582,7 +583,7 @@ int reduce_per_state(unsigned sbits, uint64_t nstates, int nv, double* out, Laun
   if (nchunks > 0x7fffffffull) return iqsi::fail(IQSH_ERR_NOTSUP, "pool reduction needs %llu workgroups", (unsigned long long)nchunks);
   const double* sums;
   if (nchunks <= kHostChunks) {
-    if (!g_pw.pinned) IQSI_TRY(hipHostMalloc((void**)&g_pw.pinned, 2 * kHostChunks * sizeof(double), hipHostMallocDefault));
+    if (!g_pw.pinned) IQSI_TRY(hipHostMalloc((void**)&g_pw.pinned, kHostDoubles * sizeof(double), hipHostMallocDefault));
     iqsi::mark_pending(g_pw.pinned, nchunks * nv);
     launch((unsigned)nchunks, clog, g_pw.pinned);
     IQSI_TRY(hipGetLastError());

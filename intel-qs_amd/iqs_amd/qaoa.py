@@ -35,7 +35,7 @@ LAYER_MIN_QUBITS = 10
 
 def _number(x) -> float:
     """An angle of any numeric type (Python, numpy, a tensor of one element on any device)."""
-    return float(1.0 * x)
+    return x if type(x) is float else float(1.0 * x)
 
 
 @dataclass
