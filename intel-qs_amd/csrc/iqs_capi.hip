@@ -3,6 +3,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <chrono>
 #include <cmath>
 #include <complex>
@@ -202,11 +203,11 @@ constexpr unsigned line_bits() { return sizeof(T) == 8 ? 3u : 4u; }
 constexpr int kSB = 256, kSP = 4;   // plain kernels for small states
 
 // Calls f with std::true_type (non-temporal accesses) or std::false_type (ordinary ones), by
-// the register's size (iqsi::cache_set).
+// the register's size and last use (iqsi::cached_pass).
 template <typename F>
 void by_cache_policy(iqsh_handle h, F f)
 {
-  if (iqsi::cache_set(h->size() * h->esz())) f(std::false_type{});
+  if (iqsi::cached_pass(h, h->size() * h->esz())) f(std::false_type{});
   else f(std::true_type{});
 }
 
@@ -1042,6 +1043,13 @@ bool capturing()
   return s != hipStreamCaptureStatusNone;
 }
 int block_kernel() { return g_block_mfma; }
+bool cached_pass(iqsh_handle h, uint64_t bytes)
+{
+  static std::atomic<uint64_t> total{1};  // bytes of all passes so far; 0 in a register: none yet
+  const uint64_t now = total.fetch_add(bytes, std::memory_order_relaxed);
+  const uint64_t last = h->touched.exchange(now + bytes, std::memory_order_relaxed);
+  return cache_set(bytes) && (last == 0 || now - last + bytes <= kCacheBytes);
+}
 int device_cus()
 {
   int dev = 0, cus = 0;

@@ -762,7 +762,7 @@ int submit(iqsh_handle h, int slot, const std::vector<Staged>& staged, unsigned 
   for (const Staged& p : staged) {
     const FBlock* desc = (const FBlock*)dev + p.first;
     const T* frag = (const T*)(dev + kSlotBlocks * sizeof(FBlock)) + (size_t)p.first * kMats * 4 * 64;
-    if (iqsi::cache_set(h->size() * h->esz()))
+    if (iqsi::cached_pass(h, h->size() * h->esz()))
       k_tile_blocks<T, M, false><<<grid, F::NT, 0, iqsi::stream()>>>((V*)h->d, p.pass, desc, frag);
     else
       k_tile_blocks<T, M, true><<<grid, F::NT, 0, iqsi::stream()>>>((V*)h->d, p.pass, desc, frag);

@@ -5,6 +5,8 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#include <atomic>
+
 #include "../../include/iqs_hip.h"
 
 // A register: 2^n interleaved complex amplitudes in device memory.
@@ -14,6 +16,7 @@ struct iqsh_state {
   void* d = nullptr;        // amplitudes
   bool owned = true;
   void* spare = nullptr;    // second buffer for out-of-place permutation
+  std::atomic<uint64_t> touched{0};  // iqsi::cached_pass
   uint64_t size() const { return uint64_t(1) << n; }
   size_t esz() const { return dtype == IQSH_C128 ? 16 : 8; }
 };
@@ -55,7 +58,12 @@ int await_results(const double* p, uint64_t count);
 // against 177 us, layer at 26 qubits 1188 against 1236); below 32 MiB stores that stay in the
 // L2s cost more when the kernel ends and writes them back (20 qubits 4.6 against 5.3 us, layer 21
 // against 30).
-inline bool cache_set(uint64_t bytes) { return bytes >= (uint64_t(32) << 20) && bytes <= (uint64_t(256) << 20); }
+constexpr uint64_t kCacheBytes = uint64_t(256) << 20;
+inline bool cache_set(uint64_t bytes) { return bytes >= (uint64_t(32) << 20) && bytes <= kCacheBytes; }
+// The same for a pass over `bytes` of h that starts now: not if passes over other registers since
+// the last one over h have put more through the cache than it holds beside h (gates on 4 registers
+// of 23 complex128 qubits in turn: 52 us with ordinary accesses, 47 with non-temporal ones).
+bool cached_pass(iqsh_handle h, uint64_t bytes);
 // Edge-parity tables and phase table of a MaxCut cost for register h (at most 64 edges):
 // the phase exp(-i gamma cut) per amplitude.
 int build_cut_spec(iqsh_handle h, unsigned ne, const unsigned* u, const unsigned* v, const double* w, double gamma,

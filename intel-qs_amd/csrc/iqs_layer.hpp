@@ -502,7 +502,7 @@ template <typename T, bool ADJ, int F>
 int layer_n(const LayerArgs& a, LayerShape* shape)
 {
   const unsigned n = a.psi->n;
-  const bool cached = iqsi::cache_set(a.psi->size() * sizeof(typename Vec<T>::t) * (ADJ ? 2 : 1));
+  const bool cached = !shape && iqsi::cached_pass(a.psi, a.psi->size() * sizeof(typename Vec<T>::t) * (ADJ ? 2 : 1));
   if constexpr (sizeof(T) == 4 && !ADJ) {
     const bool short_products = (F & kFormRX) != 0 && !(a.cs && a.cs->weighted);
     if ((n >= 26 && (short_products || (n - 13) % 8 == 0)) || (n == 13 && short_products)) return layer_m<T, 13, 5, ADJ, F>(a, shape);

@@ -493,11 +493,11 @@ int do_init(iqsh_handle h, unsigned sbits, int style, uint64_t index, uint64_t n
   return IQSH_OK;
 }
 
-// Cache policy by the pool's size (iqsi::cache_set): f(std::true_type) for non-temporal accesses.
+// Cache policy by the pool's size and last use (iqsi::cached_pass): f(std::true_type) for non-temporal accesses.
 template <typename F>
 void by_cache_policy(iqsh_handle h, F f)
 {
-  if (iqsi::cache_set(h->size() * h->esz())) f(std::false_type{});
+  if (iqsi::cached_pass(h, h->size() * h->esz())) f(std::false_type{});
   else f(std::true_type{});
 }
 

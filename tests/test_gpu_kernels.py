@@ -647,3 +647,28 @@ def test_reductions_between_unfinished_work(dt, n):
         o = np.vdot(b.download().astype(np.complex128), v.astype(np.complex128))
         assert abs(a.overlap(b) - o) < tol
     assert a.maxabsdiff(a) == 0.0
+
+
+@pytest.mark.parametrize("dt,n", [("c128", 23), ("c64", 24)])
+def test_registers_in_turn_have_the_same_bits(dt, n):
+    """Gates on three registers of 128 MiB in turn (more than the last-level cache holds: other
+    accesses than on one register at a time) give the bits of the same gates register by register."""
+    from iqs_amd import gates as G
+
+    def gates(sv, k):
+        sv.apply_1q(7, G.ry(0.3 + k))
+        sv.apply_c1q(1, n - 1, G.rx(0.7))
+        sv.apply_1q(n - 2, G.rz(0.2))
+        sv.apply_2q(n - 3, 2, np.kron(G.rx(0.4), G.ry(1.1 + k)))
+        sv.apply_c1q(n - 1, 4, G.X)
+
+    turns, alone = ([StateVector(n, dt) for _ in range(3)] for _ in range(2))
+    for sv in turns + alone:
+        sv.init_uniform(2.0 ** (-n / 2))
+    for step in range(2):
+        for k in range(3):
+            gates(turns[k], k + step)
+    for k in range(3):
+        for step in range(2):
+            gates(alone[k], k + step)
+        assert alone[k].maxabsdiff(turns[k]) == 0.0
