@@ -230,8 +230,9 @@ int iqsh_adjoint_1q(iqsh_handle psi, iqsh_handle lam, unsigned pos, const double
 /* ---- layers of one gate on every qubit -------------------------------------------------
  * psi := m (x) m (x) ... (x) m psi (the same 2x2 matrix on every position) in
  * 1 + ceil((n - 12) / 8) passes instead of n (registers below 19 qubits in smaller tiles; a
- * matrix with a real diagonal and an imaginary off-diagonal, such as RX, takes shorter kernels).  Replaces the per-qubit loop that applies a
- * QAOA mixer, RX(2 beta) on every qubit, after ImplementQaoaLayerBasedOnCostFunction
+ * matrix with a real diagonal and an imaginary off-diagonal, such as RX, takes shorter kernels).
+ * Replaces the per-qubit loop that applies a QAOA mixer, RX(2 beta) on every qubit, after
+ * ImplementQaoaLayerBasedOnCostFunction
  * (src/qaoa_features.cpp:73-110 users; src/qureg_apply1qubitgate.cpp:277-285).  n >= 10. */
 int iqsh_apply_1q_all(iqsh_handle h, const double m[8]);
 /* Backward step through such a layer for both states: *grad := sum_q 2 Im <lam| G_q |psi>

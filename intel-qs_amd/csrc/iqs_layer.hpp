@@ -21,8 +21,8 @@
 // 6.5; the exchanges (one write and one read of LDS per amplitude each) and the products
 // are each under a third of that time.  A layer takes 4.73 ms forward and 9.57 ms adjoint
 // (7.45 and 18.2 with one lane pass over 8 positions and register passes over 5 and 4 above,
-// which moved the state 5 and 6 times); 25 qubits complex64, weighted: 8.45 -> 4.6 ms for
-// cost and gradient at p = 4; 14 qubits complex128: 700 -> 375 us at p = 6 (201 in one call).
+// which moved the state 5 and 6 times); 25 qubits complex64, weighted: 8.45 -> 4.1 ms for
+// cost and gradient at p = 4; 14 qubits complex128: 700 -> 200 us at p = 6.
 //
 // Adjoint: the gates of a layer act on different qubits, so each generator G_q commutes
 // with every gate of the layer except its own, and inserting G_q after U_q equals inserting

@@ -163,9 +163,9 @@ class QubitRegister
 
   // ---- fusion ----
   /// Gates are queued, multiplied into dense blocks of up to FusionBlockQubits() qubits and
-  /// applied several blocks to a pass over the state (iqsh_apply_gates; the reference's fusion
-  /// replays queued gates cache block by cache block, src/qureg_fusion.cpp).  log2llc is kept
-  /// for API compatibility.
+  /// applied, several blocks of up to four to a pass over the state or one of five
+  /// (iqsh_apply_gates; the reference's fusion replays queued gates cache block by cache block,
+  /// src/qureg_fusion.cpp).  log2llc is kept for API compatibility.
   void TurnOnFusion(unsigned log2llc = 20);
   void TurnOffFusion();
   bool IsFusionEnabled();

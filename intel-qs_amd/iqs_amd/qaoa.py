@@ -12,7 +12,7 @@ lambda = C psi.  Walking the gates backwards, each parameterized gate U = exp(-i
 contributes dC/dtheta = 2 Im <lambda| G |psi> (psi is the state just after U), then U is
 undone on both vectors.  The mixer's qubit rotations commute with one another and with
 every X_q, so each <lambda|X_q|psi> can be taken in the fused pass that undoes its qubit's
-rotation (12, then 8 qubits per pass: iqsh_adjoint_1q_all).  Memory: the state,
+rotation (up to 12, then 8 qubits per pass: iqsh_adjoint_1q_all).  Memory: the state,
 lambda, and nothing else (no checkpoints).
 """
 from __future__ import annotations

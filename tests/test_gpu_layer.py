@@ -1,6 +1,6 @@
 """Layers of one gate on every qubit (iqsh_apply_1q_all / iqsh_adjoint_1q_all): the forward
-layer against the oracle applying the gate qubit by qubit (20 qubits and up: register
-passes of one tile per workgroup; below: the grid-stride form); the adjoint layer against the
+layer against the oracle applying the gate qubit by qubit (tiles of 2^10 to 2^13 amplitudes, by
+size and precision; one to three passes); the adjoint layer against the
 per-qubit adjoint step on the GPU and against sum_q 2 Im <lam| G_q |psi> computed with the
 oracle's 1q kernel on the host (G_q psi for each q), then the oracle's per-qubit undo."""
 import numpy as np
