@@ -282,11 +282,22 @@ __device__ __forceinline__ void window_phase(typename LT::V (&x)[LT::R], typenam
   }
 }
 
+// Waves per SIMD that a pass's registers are held to.  complex128 forward, the upper passes of a
+// general 2x2: with four of them 56 of 128 registers were spilled (24 qubits 316 -> 244 us with
+// three, 28 qubits 4.80 -> 4.59 ms).  Its adjoint spills 66 with two; one wave is slower (28 qubits
+// 12.2 -> 15.4 ms).
+template <typename T, int LR, bool ADJ, bool LOW, int F, int CUT>
+constexpr int layer_waves()
+{
+  if (ADJ) return sizeof(T) == 8 ? 2 : 3;
+  return CUT == kCutWeighted || LR == 5 || (sizeof(T) == 8 && !LOW && F == 0) ? 3 : 4;
+}
+
 // One pass.  LOW: the low pass (c = M), with the QAOA phase (CUT) before the gates going
 // forward and after them (undone) in the adjoint.  part (adjoint): the workgroup's sum of
 // generator terms at part[block], of phase terms at part[blocks + block].
 template <typename T, int M, int LR, bool ADJ, bool LOW, int F, int CUT, bool NT>
-__global__ __launch_bounds__((LTile<T, M, LR>::NT), (ADJ ? (sizeof(T) == 8 ? 2 : 3) : (CUT == kCutWeighted || LR == 5 ? 3 : 4))) void k_layer_tile(
+__global__ __launch_bounds__((LTile<T, M, LR>::NT), (layer_waves<T, LR, ADJ, LOW, F, CUT>())) void k_layer_tile(
     typename Vec<T>::t* __restrict__ psi, typename Vec<T>::t* __restrict__ lam, TilePass tp, Mat2<T> u, Mat2<double> g,
     CutArg<CUT> cs, WinArg<CUT> cw, double* __restrict__ part)
 {
