@@ -910,6 +910,12 @@ extern "C" int iqsh_apply_gates(iqsh_handle h, uint64_t ngates, const iqsh_gate*
       if (x.p[j] >= h->n) return iqsi::fail(IQSH_ERR_ARG, "position %u out of range for %u qubits", x.p[j], h->n);
     if (x.np == 2 && x.p[0] == x.p[1]) return iqsi::fail(IQSH_ERR_ARG, "gate positions coincide");
   }
+  if (ngates == 1) {
+    const iqsh_gate& x = gates[0];
+    const int rc = x.np == 1 ? iqsh_apply_1q(h, x.p[0], x.m) : iqsh_apply_2q(h, x.p[0], x.p[1], x.m);
+    if (launched) *launched = rc == IQSH_OK;
+    return rc;
+  }
   uint64_t count = 0;
   int rc;
   // A graph is replayed after the ring's slots have been used again: in a capture every gate is in
