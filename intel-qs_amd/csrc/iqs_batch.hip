@@ -958,46 +958,50 @@ __global__ void k_hea_zero(uint32_t* p, uint32_t n)
 }
 
 // The gate factors of every (layer, qubit) pair, computed in FP64 and rounded once to T
-// (RY = [[c, -s], [s, c]], RZ = diag(e^{-i phi/2}, e^{i phi/2})); tan is that of the values.
+// (RY = [[c, -s], [s, c]], RZ = diag(e^{-i phi/2}, e^{i phi/2})), and the qubits inverted after
+// every layer: one workgroup per instance, kGateLayers layers at a time.  tan is that of the values, then
+// of the bits (the opposite on qubits inverted before the layer).  (With the inversions in a launch of
+// their own 4 qubits and 12 layers, forward, took 99.6 us against 96.0.)
+constexpr uint32_t kGateLayers = 64;
 template <typename T>
-__global__ void k_hea_gates(const double* __restrict__ ang, HeaGate<T>* __restrict__ gates, uint64_t npairs)
+__global__ __launch_bounds__(256) void k_hea_gates(const double* __restrict__ ang, const HeaInst* __restrict__ inst,
+                                                   HeaGate<T>* gates, uint32_t* flips)
 {
-  const uint64_t p = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x;
-  if (p >= npairs) return;
-  double s, c, sp, cp;
-  sincos(0.5 * ang[2 * p], &s, &c);
-  sincos(0.5 * ang[2 * p + 1], &sp, &cp);
-  const bool far = fabs(s) > fabs(c);
-  const double kap = far ? s : c;
-  gates[p] = HeaGate<T>{(T)((far ? -c : s) / kap), (T)(far ? 1 : 0), {(T)(kap * cp), (T)(kap * sp)}, 1 / (kap * kap), 0};
-}
-
-// One wavefront per instance, one lane per qubit: flips after every layer, and tan for the bits.
-template <typename T>
-__global__ void k_hea_flips(const HeaInst* __restrict__ inst, HeaGate<T>* gates, uint32_t* flips)
-{
+  __shared__ uint32_t far[kGateLayers], before[kGateLayers];
   const HeaInst& I = inst[blockIdx.x];
-  const uint32_t q = threadIdx.x;
-  const bool on = q < I.n;
-  HeaGate<T>* g = gates + I.par + (on ? q : 0);
-  bool flip = false;
-  constexpr uint32_t B = 8;  // layers whose gates are in flight together
-  for (uint32_t l0 = 0; l0 < I.depth; l0 += B) {
-    T t[B], far[B];
-#pragma unroll
-    for (uint32_t i = 0; i < B; ++i) {
-      const HeaGate<T>& h = g[(uint64_t)min(l0 + i, I.depth - 1) * I.n];
-      t[i] = h.tan;
-      far[i] = h.far;
+  const uint32_t n = I.n, depth = I.depth, tid = threadIdx.x;
+  uint32_t inverted = 0;  // so far (first wavefront)
+  for (uint32_t l0 = 0; l0 < depth; l0 += kGateLayers) {
+    const uint32_t pairs = min(kGateLayers, depth - l0) * n;
+    const uint64_t row = I.par + (uint64_t)l0 * n;
+    if (tid < kGateLayers) far[tid] = 0;
+    __syncthreads();
+    for (uint32_t i = tid; i < pairs; i += 256) {
+      const uint64_t p = row + i;
+      double s, c, sp, cp;
+      sincos(0.5 * ang[2 * p], &s, &c);
+      sincos(0.5 * ang[2 * p + 1], &sp, &cp);
+      const bool inv = fabs(s) > fabs(c);
+      const double kap = inv ? s : c;
+      gates[p] = HeaGate<T>{(T)((inv ? -c : s) / kap), (T)(inv ? 1 : 0), {(T)(kap * cp), (T)(kap * sp)}, 1 / (kap * kap), 0};
+      if (inv) atomicOr(&far[i / n], 1u << (i % n));
     }
-#pragma unroll
-    for (uint32_t i = 0; i < B; ++i) {
-      if (l0 + i >= I.depth) break;
-      if (on && flip) g[(uint64_t)(l0 + i) * I.n].tan = -t[i];
-      flip ^= on && far[i] != 0;
-      const uint64_t m = __ballot(flip);
-      if (q == 0) flips[I.lay + l0 + i] = (uint32_t)m;
+    __syncthreads();
+    if (tid < kGateLayers) {  // one wavefront: XOR over the layers so far
+      const uint32_t f = far[tid];
+      uint32_t m = f;
+      for (uint32_t d = 1; d < kGateLayers; d *= 2) {
+        const uint32_t o = __shfl_up(m, d);
+        if (tid >= d) m ^= o;
+      }
+      m ^= inverted;
+      before[tid] = m ^ f;
+      if (l0 + tid < depth) flips[I.lay + l0 + tid] = m;
+      inverted = __shfl(m, kGateLayers - 1);
     }
+    __syncthreads();
+    for (uint32_t i = tid; i < pairs; i += 256)
+      if ((before[i / n] >> (i % n)) & 1u) gates[row + i].tan = -gates[row + i].tan;
   }
 }
 
@@ -1332,9 +1336,12 @@ int build(iqsh_hea* h, int mode)
   // (all that fit, then): they wait for nothing, but while the rounds last the second workgroup
   // polls beside them.  512 of 12 qubits with one of 14, one against two workgroups: complex64 895
   // and 790 us, complex128 994 and 938; with eight of 16, complex64 1088 and 1087, complex128 1336
-  // and 1606.
+  // and 1606.  Nor more than the fullest queue has tasks, if each XCD gets an eighth of the grid
+  // (one register of 4 qubits and 2 layers, forward: two workgroups per compute unit 35 us, one 26).
   const uint64_t half = 2 * (uint64_t)h->cus / kQueues;
-  h->work_per_cu = round ? (int)std::min<uint64_t>(64, (round + half - 1) / half) : 64;
+  const uint64_t most = *std::max_element(h->qlen.begin(), h->qlen.end());
+  const uint64_t useful = (kQueues * most + h->cus - 1) / h->cus;
+  h->work_per_cu = (int)std::max<uint64_t>(1, std::min<uint64_t>(useful, round ? (round + half - 1) / half : 64));
   h->ntask = (uint32_t)tasks.size();
   h->nepi = (uint32_t)epi.size();
   h->nctl = kCtlArrive + arrive;
@@ -1363,11 +1370,8 @@ int enqueue_t(iqsh_hea* h, int mode, hipStream_t st)
   a.wait_extra = h->wait_extra;
   hipLaunchKernelGGL(k_hea_zero, dim3((h->nctl + 255) / 256), dim3(256), 0, st, h->ctl, h->nctl);
   IQSI_TRY(hipGetLastError());
-  hipLaunchKernelGGL(k_hea_gates<T>, dim3((unsigned)((h->npairs + 255) / 256)), dim3(256), 0, st, (const double*)h->ang,
-                     (HeaGate<T>*)h->gates, h->npairs);
-  IQSI_TRY(hipGetLastError());
-  hipLaunchKernelGGL(k_hea_flips<T>, dim3((unsigned)h->count), dim3(64), 0, st, (const HeaInst*)h->inst,
-                     (HeaGate<T>*)h->gates, h->flips);
+  hipLaunchKernelGGL(k_hea_gates<T>, dim3((unsigned)h->count), dim3(256), 0, st, (const double*)h->ang,
+                     (const HeaInst*)h->inst, (HeaGate<T>*)h->gates, h->flips);
   IQSI_TRY(hipGetLastError());
   IQSI_TRY(launch_var<T>(h->tune.variant, a, h->tune.workers_per_cu > 0 ? h->tune.workers_per_cu : h->work_per_cu, h->cus, st));
   if (h->nepi) {
