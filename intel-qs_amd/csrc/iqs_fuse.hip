@@ -46,9 +46,10 @@ namespace {
 // to a drift of the norm; they are rounded once, at the end.  Until then an entry is h + l with h a
 // multiple of 2^-24: for entries up to 1 products of two h and their sums are exact, and what
 // involves an l is small enough that its rounding does not count.  (Entries of any size are as
-// good as plain products at least.  The same in long double takes twice as long.)  10 brick layers
+// good as plain products at least.  The same in long double takes twice as long.)  Registers in
+// complex64 take plain products in double, far below their own rounding (X false: l is not used).  10 brick layers
 // of 20 qubits, error against 64 bits: 1.9e-15, with plain products 4.1e-15, in the same 141 us.
-template <int D>
+template <int D, bool X>
 struct Wide {
   double h[2][D][D], l[2][D][D];  // real and imaginary parts
 
@@ -63,23 +64,27 @@ struct Wide {
   {
     constexpr double k = 1.5 * (1 << 28);  // sums with k are multiples of 2^-24
     const double v = hi + lo;
-    h[p][r][c] = (v + k) - k;
-    l[p][r][c] = (hi - h[p][r][c]) + lo;
+    h[p][r][c] = X ? (v + k) - k : hi;
+    if (X) l[p][r][c] = (hi - h[p][r][c]) + lo;
   }
+  double low(int p, int r, int c) const { return X ? l[p][r][c] : 0.0; }
   Wide operator*(const Wide& y) const
   {
     Wide z;
     for (int r = 0; r < D; ++r) {
       double h0[D] = {}, h1[D] = {}, l0[D] = {}, l1[D] = {};
       for (int k = 0; k < D; ++k) {
-        const double a = h[0][r][k], b = h[1][r][k], al = l[0][r][k], bl = l[1][r][k];
+        const double a = h[0][r][k], b = h[1][r][k], al = low(0, r, k), bl = low(1, r, k);
         if (a == 0 && b == 0 && al == 0 && bl == 0) continue;
         for (int c = 0; c < D; ++c) {
-          const double u = y.h[0][k][c], v = y.h[1][k][c], ul = y.l[0][k][c], vl = y.l[1][k][c];
+          const double u = y.h[0][k][c], v = y.h[1][k][c];
           h0[c] += a * u - b * v;
           h1[c] += a * v + b * u;
-          l0[c] += (a * ul - b * vl) + (al * (u + ul) - bl * (v + vl));
-          l1[c] += (a * vl + b * ul) + (al * (v + vl) + bl * (u + ul));
+          if constexpr (X) {
+            const double ul = y.l[0][k][c], vl = y.l[1][k][c];
+            l0[c] += (a * ul - b * vl) + (al * (u + ul) - bl * (v + vl));
+            l1[c] += (a * vl + b * ul) + (al * (v + vl) + bl * (u + ul));
+          }
         }
       }
       for (int c = 0; c < D; ++c) {
@@ -93,33 +98,34 @@ struct Wide {
   {
     for (int r = 0; r < D; ++r)
       for (int c = 0; c < D; ++c)
-        for (int p = 0; p < 2; ++p) *m++ = h[p][r][c] + l[p][r][c];
+        for (int p = 0; p < 2; ++p) *m++ = h[p][r][c] + low(p, r, c);
   }
 };
 
 // hi (x) lo: index bit 1 under hi, bit 0 under lo; one of them may be null, for the identity.
-Wide<4> kron(const Wide<2>* hi, const Wide<2>* lo)
+template <bool X>
+Wide<4, X> kron(const Wide<2, X>* hi, const Wide<2, X>* lo)
 {
-  Wide<4> z;
+  Wide<4, X> z;
   if (!hi || !lo) {
     std::memset(&z, 0, sizeof z);
-    const Wide<2>& x = hi ? *hi : *lo;
+    const Wide<2, X>& x = hi ? *hi : *lo;
     const int s = hi ? 2 : 1, o = 3 - s;  // strides of x's index and of the other
     for (int p = 0; p < 2; ++p)
       for (int i = 0; i < 2; ++i)
         for (int j = 0; j < 2; ++j)
           for (int k = 0; k < 2; ++k) {
             z.h[p][i * s + k * o][j * s + k * o] = x.h[p][i][j];
-            z.l[p][i * s + k * o][j * s + k * o] = x.l[p][i][j];
+            if (X) z.l[p][i * s + k * o][j * s + k * o] = x.l[p][i][j];
           }
     return z;
   }
   for (int i = 0; i < 2; ++i)
     for (int j = 0; j < 2; ++j) {
-      const double a = hi->h[0][i][j], b = hi->h[1][i][j], al = hi->l[0][i][j], bl = hi->l[1][i][j];
+      const double a = hi->h[0][i][j], b = hi->h[1][i][j], al = hi->low(0, i, j), bl = hi->low(1, i, j);
       for (int r = 0; r < 2; ++r)
         for (int c = 0; c < 2; ++c) {
-          const double u = lo->h[0][r][c], v = lo->h[1][r][c], ul = lo->l[0][r][c], vl = lo->l[1][r][c];
+          const double u = lo->h[0][r][c], v = lo->h[1][r][c], ul = lo->low(0, r, c), vl = lo->low(1, r, c);
           z.put(0, 2 * i + r, 2 * j + c, a * u - b * v, (a * ul - b * vl) + (al * (u + ul) - bl * (v + vl)));
           z.put(1, 2 * i + r, 2 * j + c, a * v + b * u, (a * vl + b * ul) + (al * (v + vl) + bl * (u + ul)));
         }
@@ -132,6 +138,7 @@ Wide<4> kron(const Wide<2>* hi, const Wide<2>* lo)
 // same pair multiplied together: a small product each, instead of one with a block's
 // matrix.  A brick layer of 20 qubits (H, rotation on every qubit, 9 or 10 CNOTs) becomes its 9
 // or 10 two-qubit gates.
+template <bool X>
 std::vector<iqsh_gate> merge_gates(const iqsh_gate* g, int ngates)
 {
   std::vector<iqsh_gate> out;
@@ -140,8 +147,8 @@ std::vector<iqsh_gate> merge_gates(const iqsh_gate* g, int ngates)
   // gate that is still last on a position is in `pair` at one of its positions, home[gate].
   int last[64], place[64];
   bool some[64] = {};
-  const std::unique_ptr<Wide<2>[]> lone(new Wide<2>[64]);
-  const std::unique_ptr<Wide<4>[]> pair(new Wide<4>[64]);
+  const std::unique_ptr<Wide<2, X>[]> lone(new Wide<2, X>[64]);
+  const std::unique_ptr<Wide<4, X>[]> pair(new Wide<4, X>[64]);
   std::vector<uint8_t> home;
   std::fill(last, last + 64, -1);
   std::fill(place, place + 64, -1);
@@ -154,7 +161,7 @@ std::vector<iqsh_gate> merge_gates(const iqsh_gate* g, int ngates)
     return (int)out.size() - 1;
   };
   // The one-qubit gates on q, which go into a two-qubit gate; null if there are none.
-  auto take = [&](unsigned q) -> const Wide<2>* {
+  auto take = [&](unsigned q) -> const Wide<2, X>* {
     if (!some[q]) return nullptr;
     if (place[q] >= 0) out[place[q]].np = 0;
     place[q] = -1;
@@ -176,25 +183,25 @@ std::vector<iqsh_gate> merge_gates(const iqsh_gate* g, int ngates)
     const iqsh_gate& x = g[i];
     const unsigned a = x.p[0], b = x.p[1];
     if (x.np == 1) {
-      if (some[a]) lone[a] = Wide<2>(x.m) * lone[a];
+      if (some[a]) lone[a] = Wide<2, X>(x.m) * lone[a];
       else {
-        lone[a] = Wide<2>(x.m);
+        lone[a] = Wide<2, X>(x.m);
         some[a] = true;
         if (last[a] < 0) place[a] = add(x);
       }
       continue;
     }
-    Wide<4> m(x.m);
-    const Wide<2>*ma = take(a), *mb = take(b);
+    Wide<4, X> m(x.m);
+    const Wide<2, X>*ma = take(a), *mb = take(b);
     if (ma || mb) m = m * kron(ma, mb);
     if (last[a] >= 0 && last[a] == last[b]) {
       if (out[last[a]].p[0] != a)  // the same pair the other way round: exchange the index bits
         for (auto* e : {m.h, m.l})
-          for (int p = 0; p < 2; ++p) {
+          for (int p = 0; p < 2 && (X || e == m.h); ++p) {
             for (int v = 0; v < 4; ++v) std::swap(e[p][1][v], e[p][2][v]);
             for (int v = 0; v < 4; ++v) std::swap(e[p][v][1], e[p][v][2]);
           }
-      Wide<4>& z = pair[home[last[a]]];
+      Wide<4, X>& z = pair[home[last[a]]];
       z = m * z;
       continue;
     }
@@ -212,7 +219,7 @@ std::vector<iqsh_gate> merge_gates(const iqsh_gate* g, int ngates)
     if (home[last[q]] != q) continue;
     const bool first = x.p[0] == q;
     const unsigned other = x.p[first];
-    const Wide<2>*mq = take(q), *mo = last[other] == last[q] ? take(other) : nullptr;
+    const Wide<2, X>*mq = take(q), *mo = last[other] == last[q] ? take(other) : nullptr;
     if (mq || mo) pair[q] = kron(first ? mq : mo, first ? mo : mq) * pair[q];
     pair[q].write(x.m);
   }
@@ -923,7 +930,8 @@ extern "C" int iqsh_apply_gates(iqsh_handle h, uint64_t ngates, const iqsh_gate*
   const bool capture = iqsi::capturing();
   if (capture) block = std::min(block, 2u);
   try {
-    const std::vector<iqsh_gate> merged = merge_gates(gates, (int)ngates);
+    const std::vector<iqsh_gate> merged =
+        h->dtype == IQSH_C128 ? merge_gates<true>(gates, (int)ngates) : merge_gates<false>(gates, (int)ngates);
     gates = merged.data();
     const int ng = (int)merged.size();
     if (h->n < 10 || capture || iqsi::block_kernel() != 1) rc = apply_blocks(h, gates, ng, block, &count);
