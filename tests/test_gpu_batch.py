@@ -251,3 +251,25 @@ def test_rotations_past_a_quarter_turn(dtype, tol, theta):
             dn = oracle_run(n, d, (ang - s)[lo:hi], "dp")[1]
             assert abs(grad[k] - 0.5 * (up - dn)) < 10 * n * tol, (k, grad[k], 0.5 * (up - dn))
         b.close()
+
+
+@pytest.mark.parametrize("variant", [TEST_VARIANT, 0])
+def test_more_layers_than_the_set_up_takes_at_once(variant):
+    """The gate set-up takes 64 layers at a time and carries the inverted qubits on: depths on both
+    sides, in one batch, states and costs against the oracle, gradients of late and early angles by
+    the shift rule.  Tolerance: 130 layers of 3 gates on each of 12 qubits, one rounding each, 1e-12."""
+    nq, dp = [2, 7, 9, 12, 1, 10], [63, 64, 65, 130, 200, 128]
+    off = param_offsets(nq, dp)
+    ang = np.random.default_rng(23).uniform(-2 * math.pi, 2 * math.pi, int(off[-1]))
+    b = HeaBatch(nq, dp, "c128", tune=(variant, 0, 0))
+    b.set_angles(ang)
+    b.run(grad=False, keep_state=True)
+    cost = b.results(grad=False)
+    for i, (n, d) in enumerate(zip(nq, dp)):
+        st_ref, c_ref = oracle_run(n, d, ang[off[i]:off[i + 1]])
+        assert np.max(np.abs(b.state(i) - st_ref)) < 1e-12 and abs(cost[i] - c_ref) < 10 * n * 1e-12
+    _, grad = b.evaluate(ang)
+    for slots in ([0] * len(nq), [2 * n * d - 1 for n, d in zip(nq, dp)], [2 * n * min(d - 1, 64) for n, d in zip(nq, dp)]):
+        want = b.parameter_shift(ang, slots)
+        assert np.max(np.abs(grad[off[:-1] + slots] - want)) < 1e-10
+    b.close()
