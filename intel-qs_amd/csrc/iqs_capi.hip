@@ -1048,7 +1048,8 @@ bool cached_pass(iqsh_handle h, uint64_t bytes)
   static std::atomic<uint64_t> total{1};  // bytes of all passes so far; 0 in a register: none yet
   const uint64_t now = total.fetch_add(bytes, std::memory_order_relaxed);
   const uint64_t last = h->touched.exchange(now + bytes, std::memory_order_relaxed);
-  return cache_set(bytes) && (last == 0 || now - last + bytes <= kCacheBytes);
+  const bool cold = last != 0 && now - last + bytes > kCacheBytes;
+  return !(h->cold.exchange(cold, std::memory_order_relaxed) && cold) && cache_set(bytes);
 }
 int device_cus()
 {

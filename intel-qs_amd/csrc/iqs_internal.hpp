@@ -17,6 +17,7 @@ struct iqsh_state {
   bool owned = true;
   void* spare = nullptr;    // second buffer for out-of-place permutation
   std::atomic<uint64_t> touched{0};  // iqsi::cached_pass
+  std::atomic<bool> cold{false};
   uint64_t size() const { return uint64_t(1) << n; }
   size_t esz() const { return dtype == IQSH_C128 ? 16 : 8; }
 };
@@ -60,9 +61,11 @@ int await_results(const double* p, uint64_t count);
 // against 30).
 constexpr uint64_t kCacheBytes = uint64_t(256) << 20;
 inline bool cache_set(uint64_t bytes) { return bytes >= (uint64_t(32) << 20) && bytes <= kCacheBytes; }
-// The same for a pass over `bytes` of h that starts now: not if passes over other registers since
-// the last one over h have put more through the cache than it holds beside h (gates on 4 registers
-// of 23 complex128 qubits in turn: 52 us with ordinary accesses, 47 with non-temporal ones).
+// The same for a pass over `bytes` of h that starts now: not if h is used in turn with other
+// registers, that is if before this pass and before the last one over h, passes over others have
+// put more through the cache than it holds beside h (gates on 4 registers of 23 complex128 qubits in
+// turn: 52 us with ordinary accesses, 47 with non-temporal ones).  A first pass after others
+// brings h back into the cache for those that follow it.
 bool cached_pass(iqsh_handle h, uint64_t bytes);
 // Edge-parity tables and phase table of a MaxCut cost for register h (at most 64 edges):
 // the phase exp(-i gamma cut) per amplitude.

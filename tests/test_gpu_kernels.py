@@ -654,21 +654,19 @@ def test_registers_in_turn_have_the_same_bits(dt, n):
     """Gates on three registers of 128 MiB in turn (more than the last-level cache holds: other
     accesses than on one register at a time) give the bits of the same gates register by register."""
     from iqs_amd import gates as G
-
-    def gates(sv, k):
-        sv.apply_1q(7, G.ry(0.3 + k))
-        sv.apply_c1q(1, n - 1, G.rx(0.7))
-        sv.apply_1q(n - 2, G.rz(0.2))
-        sv.apply_2q(n - 3, 2, np.kron(G.rx(0.4), G.ry(1.1 + k)))
-        sv.apply_c1q(n - 1, 4, G.X)
-
+    gates = [lambda sv, k: sv.apply_1q(7, G.ry(0.3 + k)), lambda sv, k: sv.apply_c1q(1, n - 1, G.rx(0.7)),
+             lambda sv, k: sv.apply_1q(n - 2, G.rz(0.2)), lambda sv, k: sv.apply_1q(1, G.ry(1.0)),
+             lambda sv, k: sv.apply_2q(n - 3, 2, np.kron(G.rx(0.4), G.ry(1.1 + k))),
+             lambda sv, k: sv.apply_c1q(n - 1, 4, G.X), lambda sv, k: sv.apply_2q(n - 1, 9, np.kron(G.ry(0.8), G.H))]
     turns, alone = ([StateVector(n, dt) for _ in range(3)] for _ in range(2))
     for sv in turns + alone:
         sv.init_uniform(2.0 ** (-n / 2))
     for step in range(2):
-        for k in range(3):
-            gates(turns[k], k + step)
+        for gate in gates:
+            for k in range(3):
+                gate(turns[k], k + step)
     for k in range(3):
         for step in range(2):
-            gates(alone[k], k + step)
+            for gate in gates:
+                gate(alone[k], k + step)
         assert alone[k].maxabsdiff(turns[k]) == 0.0
