@@ -46,9 +46,11 @@ namespace {
 // to a drift of the norm; they are rounded once, at the end.  Until then an entry is h + l with h a
 // multiple of 2^-24: for entries up to 1 products of two h and their sums are exact, and what
 // involves an l is small enough that its rounding does not count.  (Entries of any size are as
-// good as plain products at least.  The same in long double takes twice as long.)  Registers in
-// complex64 take plain products in double, far below their own rounding (X false: l is not used).  10 brick layers
-// of 20 qubits, error against 64 bits: 1.9e-15, with plain products 4.1e-15, in the same 141 us.
+// good as plain products at least.  The same in long double takes twice as long.)  Error of 60
+// brick layers of 12 qubits: 2.1e-15, with plain products 3.0e-15, with every gate multiplied into
+// the two-qubit gate by itself 1.7e-14; 10 layers of 20 qubits 1.9e-15 in 141 us, 4.1e-15 by
+// itself in as many.  Registers in complex64 take plain products in double, far below their own
+// rounding (X false: l is not used).
 template <int D, bool X>
 struct Wide {
   double h[2][D][D], l[2][D][D];  // real and imaginary parts
